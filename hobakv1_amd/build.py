@@ -15,7 +15,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libhobak_hip.so")
 
-HIP_SOURCES = ["element.hip", "solver_kernels.hip", "api.hip"]
+HIP_SOURCES = ["element.hip", "solver_kernels.hip", "resident.hip", "api.hip"]
 
 # -packed-fp32-ops: keep the compiler from emitting packed FP32 VALU ops.
 HIPCC_FLAGS = [

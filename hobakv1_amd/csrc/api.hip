@@ -53,6 +53,7 @@ struct Plan;
 constexpr double kEps = 2.220446049250313e-16;  // Eigen's default CG tolerance (machine epsilon)
 constexpr int kMaxPlans = 32;
 constexpr int kMaxSamples = 512;
+constexpr int kResidentIters = 512;
 }  // namespace
 
 struct hobak_ctx {
@@ -71,6 +72,9 @@ struct hobak_ctx {
   int p_form = 1;                      // FP64 p-form iterations: 0 never, 1 with streamed matrices, 2 always
   int coarse = 1;                      // reduced-precision form: rigid-translation coarse correction
   int agg = 0;                         // reduced-precision form: spatial order and local aggregates (2: also with the coarse correction)
+  int resident = kResidentIters;       // resident PCG: iterations per launch, 0 off
+  int cus = 0;                         // compute units of the device
+  int* tickets = nullptr;              // resident PCG launches of this context's stream
   hipStream_t stream = nullptr;
   size_t budget = 0;
   size_t in_use = 0;
@@ -457,6 +461,11 @@ struct hobak_inst {
   double spmv_ms_sum = 0.0, spmv_bytes_sum = 0.0;
   long long spmv_count = 0;
   unsigned work_seen = 0;           // Ctl::spmv_work at the last status poll
+  // resident PCG: most update workgroups' rows one workgroup takes (0: never resident), what
+  // Ctl::res_abort held at the last status poll, refinement sweeps of the last solve
+  int res_pack = 0;
+  int abort_seen = 0;
+  int sweeps_seen = 0;
 };
 
 struct hobak_sched {
@@ -623,6 +632,21 @@ int agg_on(const hobak_ctx* ctx, const hobak_inst* I) {
   const InstDev& h = I->h;
   if (!I->spatial || !h.refine || h.contact) return 0;
   return (ctx->agg == 2 || !coarse_on(ctx, I)) ? 1 : 0;
+}
+
+// Update workgroups' rows that one workgroup of the resident PCG takes when compute units are short: as
+// many as keep its slots in registers and LDS (84 FP64 or 147 FP32 64-slot steps, beside the
+// columns and vectors of a lattice), with an eighth past that streamed; 0 where the instance does
+// not qualify: its update workgroups loop over several runs of rows (more rows than the cap covers), or
+// it needs more workgroups than there are compute units.
+int resident_pack(const hobak_ctx* ctx, const hobak_inst* I) {
+  const int nu = I->h.nb[K_UPD], rows = 84 * I->groups;
+  if ((long)nu * rows < I->nv) return 0;
+  const double steps = (I->tsize == 8 ? 84 : 147) * 1.125;
+  const double per_row = (double)I->P.nslots / I->nv / 64.0;
+  const int fit = std::max(1, (int)((steps / per_row - 2.5 * I->P.H) / rows));
+  const int need = (nu + ctx->cus - 1) / ctx->cus;
+  return need <= 2 * fit ? std::max(fit, need) : 0;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -873,6 +897,60 @@ bool stream_matrix(const hobak_ctx* ctx, double solving_bytes) {
   return solving_bytes > (double)ctx->spmv_stream_mb * (1 << 20);
 }
 
+// The resident PCG's launch tables in the arena: the instances, largest first (their solves take the
+// most iterations, and what runs last should be short), and the workgroups of each.  An instance takes
+// as few workgroups as hold its matrix on chip (res_pack) when the batch fills the device's
+// compute units that way, and up to one per update workgroup's rows while compute units are left.
+int resident_tables(hobak_ctx* ctx, const std::vector<hobak_inst*>& m, Batch& b) {
+  const int n = (int)m.size();
+  long packed = 0;
+  for (auto* I : m) packed += (I->h.nb[K_UPD] + I->res_pack - 1) / I->res_pack;
+  auto workgroups = [&](const hobak_inst* I) {
+    const int nu = I->h.nb[K_UPD];
+    const int least = (nu + I->res_pack - 1) / I->res_pack;
+    const long w = std::min<long>(nu, std::max<long>(least, least * (long)ctx->cus / packed));
+    const int per = (int)((nu + w - 1) / w);
+    return (nu + per - 1) / per;  // no more than it takes at that many each
+  };
+  if (n == 1) {
+    b = Batch{nullptr, nullptr, m[0]->dev, 1, workgroups(m[0])};
+    return HOBAK_OK;
+  }
+  std::vector<hobak_inst*> order = m;
+  std::stable_sort(order.begin(), order.end(), [](hobak_inst* a, hobak_inst* c) { return a->nv > c->nv; });
+  const size_t tab = al(sizeof(void*) * n), need = tab + al(sizeof(int) * (n + 1));
+  if (ctx->arena_off + need > ctx->arena_cap) return fail(ctx, HOBAK_E_INVALID, "batch table arena exhausted");
+  char* host = ctx->arena_host + ctx->arena_off;
+  char* dev = ctx->arena_dev + ctx->arena_off;
+  ctx->arena_off += need;
+  const InstDev** hp = (const InstDev**)host;
+  int* bo = (int*)(host + tab);
+  bo[0] = 0;
+  for (int i = 0; i < n; i++) {
+    hp[i] = order[i]->dev;
+    bo[i + 1] = bo[i] + workgroups(order[i]);
+  }
+  b = Batch{(const InstDev* const*)dev, (const int*)(dev + tab), nullptr, n, bo[n]};
+  HIPCHK(ctx, hipMemcpyAsync(dev, host, need, hipMemcpyHostToDevice, ctx->stream));
+  return HOBAK_OK;
+}
+
+// The gated kernels that follow a group of PCG iterations (see launch_chunk).
+template <typename T>
+int launch_solve_ends(hobak_ctx* ctx, const Plan& P) {
+  hipStream_t s = ctx->stream;
+  const int cap = ctx->grid_cap;
+  if (P.refine) {
+    HIPCHK(ctx, launch_refine_residual<T>(P.b[K_SPMV], P.b[K_DOF], P.shift, cap, s));
+    HIPCHK(ctx, launch_finish_check(P.b[K_ONE], 1, s));
+    HIPCHK(ctx, launch_refine_init<T>(P.b[K_ROW], 1, P.groups, cap, s));
+    HIPCHK(ctx, launch_cg_init(P.b[K_ONE], 1, 1, s));
+  } else {
+    HIPCHK(ctx, launch_finish_check(P.b[K_ONE], 0, s));
+  }
+  return HOBAK_OK;
+}
+
 // k PCG iterations over the batch (k even, so the current scalar set is set 0 again at the end),
 // then the gated end-of-solve kernels: the refinement residual, check and re-seed, or the plain
 // form's finish flag.  With a sampling scheduler, some SpMV launches carry timing events.
@@ -903,15 +981,7 @@ int launch_chunk(hobak_ctx* ctx, const Plan& P, int k, int stream, hobak_sched* 
     }
     HIPCHK(ctx, launch_cg_update<T>(P.b[K_UPD], P.groups, P.coarse | (P.agg << 1), j & 1, cap, s));
   }
-  if (P.refine) {
-    HIPCHK(ctx, launch_refine_residual<T>(P.b[K_SPMV], P.b[K_DOF], P.shift, cap, s));
-    HIPCHK(ctx, launch_finish_check(P.b[K_ONE], 1, s));
-    HIPCHK(ctx, launch_refine_init<T>(P.b[K_ROW], 1, P.groups, cap, s));
-    HIPCHK(ctx, launch_cg_init(P.b[K_ONE], 1, 1, s));
-  } else {
-    HIPCHK(ctx, launch_finish_check(P.b[K_ONE], 0, s));
-  }
-  return HOBAK_OK;
+  return launch_solve_ends<T>(ctx, P);
 }
 
 template <typename T>
@@ -944,7 +1014,7 @@ template <typename T>
 int tick_impl(hobak_sched* S) {
   hobak_ctx* ctx = S->ctx;
   hipStream_t s = ctx->stream;
-  TRY(arena_ensure(ctx, 5 * plan_bytes(S->members.size() + 1)));
+  TRY(arena_ensure(ctx, 7 * plan_bytes(S->members.size() + 1)));
   ctx->arena_off = 0;
   TRY(plan_get(ctx, S->members, &S->mplan));
   if (S->dirty) {
@@ -1066,10 +1136,33 @@ int tick_impl(hobak_sched* S) {
   int nsolving = 0;
   double solving_bytes = 0.0;
   long solving_wgs = 0;
-  std::vector<hobak_inst*> solving;
+  std::vector<hobak_inst*> solving, resident;
   const int k = ctx->chunk_iters;
+  int every = 0;
+  if (S->sampling && S->ephemeral) {
+    for (auto* I : S->members)
+      if (I->sample_every > 0) every = every ? std::min(every, I->sample_every) : I->sample_every;
+  } else if (S->sampling) {
+    every = S->spmv_every;
+  }
+  // a group that holds a sampled SpMV launch (index g with g % every == every - 1) runs uncaptured,
+  // with the events on that launch
+  auto sampled_group = [&]() {
+    return every > 0 && (int)S->samples.size() < kMaxSamples &&
+           (S->sample_it / every) * every + every - 1 < S->sample_it + k;
+  };
+  // instances that fit on chip run the resident PCG; a tick whose next group is sampled first runs
+  // that group over every solving instance in the two-kernel form, which the samples time
+  const bool may_reside = ctx->resident > 0 && ctx->grid_cap == 0;
+  for (auto& r : S->active)
+    if (r.stage == 1 && may_reside && r.I->res_pack > 0) resident.push_back(r.I);
+  const bool sample_first = !resident.empty() && sampled_group();
+  int sweeps = 1;
   for (auto& r : S->active) {
     if (r.stage != 1) continue;
+    const bool res = may_reside && r.I->res_pack > 0;
+    if (res && r.I->h.refine) sweeps = std::max(sweeps, r.I->sweeps_seen > 0 ? r.I->sweeps_seen : 2);
+    if (res && !sample_first) continue;
     nsolving++;
     solving_bytes += spmv_bytes_of(r.I);
     solving_wgs += r.I->h.nb[K_SPMV];
@@ -1078,16 +1171,10 @@ int tick_impl(hobak_sched* S) {
     const int q = p > 0 ? (p - r.done_iters) / k : 0;
     m = std::min(m, std::max(1, q));
   }
+  if (sample_first) m = 1;
+  if (nsolving || !resident.empty()) HIPCHK(ctx, hipEventRecord(ctx->ev[4], s));
   if (nsolving) {
     const Range r_pcg("hobak pcg groups");
-    HIPCHK(ctx, hipEventRecord(ctx->ev[4], s));
-    int every = 0;
-    if (S->sampling && S->ephemeral) {
-      for (auto* I : S->members)
-        if (I->sample_every > 0) every = every ? std::min(every, I->sample_every) : I->sample_every;
-    } else if (S->sampling) {
-      every = S->spmv_every;
-    }
     const int st = stream_matrix(ctx, solving_bytes) ? 1 : 0;
     const bool compact = nsolving < M.n && solving_wgs * 100 <= (long)ctx->compact_pct * M.b[K_SPMV].total;
     Plan PG;
@@ -1099,12 +1186,7 @@ int tick_impl(hobak_sched* S) {
       M.chunk_k[st] = k;
     }
     for (int j = 0; j < m; j++) {
-      // a group that holds a sampled SpMV launch (index g with g % every == every - 1) runs
-      // uncaptured, with the events on that launch; every other group replays the graph
-      const int g0 = S->sample_it;
-      const bool sampled = every > 0 && (int)S->samples.size() < kMaxSamples &&
-                           (g0 / every) * every + every - 1 < g0 + k;
-      if (graphs && !compact && !sampled) {
+      if (graphs && !compact && !sampled_group()) {  // every unsampled group replays the graph
         HIPCHK(ctx, hipGraphLaunch(M.chunk_exec[st], s));
         if (S->sampling) S->sample_it += k;
         S->stat[9] += 1;
@@ -1113,12 +1195,26 @@ int tick_impl(hobak_sched* S) {
         S->stat[10] += 1;
       }
     }
-    HIPCHK(ctx, hipEventRecord(ctx->ev[5], s));
     ran = true;
   }
+  if (!resident.empty()) {
+    const Range r_res("hobak resident pcg");
+    Batch rb;
+    TRY(resident_tables(ctx, resident, rb));
+    Plan PR;
+    const bool all = (int)resident.size() == M.n;
+    if (!all) TRY(plan_transient(ctx, resident, PR));
+    for (int j = 0; j < sweeps; j++) {
+      HIPCHK(ctx, launch_cg_resident<T>(rb, M.groups, ctx->tickets, ctx->resident, s));
+      TRY(launch_solve_ends<T>(ctx, all ? M : PR));
+    }
+    S->stat[1] += sweeps;
+    S->stat[10] += sweeps;
+    ran = true;
+  }
+  if (ran) HIPCHK(ctx, hipEventRecord(ctx->ev[5], s));
 
   S->stat[1] += nsolving ? m : 0;
-  if (nsolving) S->stat[7] += (double)m * k;
   // 5. statuses
   {
     const Range r_poll("hobak poll");
@@ -1128,14 +1224,24 @@ int tick_impl(hobak_sched* S) {
   }
   // algorithmic SpMV bytes of this tick: each member's matrix and vectors once per launch that
   // streamed them (counted on the device; launches after a member's solve ended read nothing)
+  // the resident PCG counts the products a solve formed; its launches are the most any instance did
   double work_bytes = 0.0;
+  unsigned res_launches = 0;
   for (int i = 0; i < M.n; i++) {
     hobak_inst* I = M.members[i];
     const unsigned w = M.status_host[i].spmv_work;
     work_bytes += (double)(unsigned)(w - I->work_seen) * spmv_bytes_of(I);
+    if (!resident.empty()) res_launches = std::max(res_launches, w - I->work_seen);
     I->work_seen = w;
+    if (M.status_host[i].res_abort != I->abort_seen) {  // did not fit, or could not run at once
+      I->abort_seen = M.status_host[i].res_abort;
+      I->res_pack /= 2;
+    }
   }
   S->stat[8] += work_bytes;
+  const long long launches = std::max<long long>(nsolving ? (long long)m * k : 0, res_launches);
+  if (ran) S->stat[7] += (double)launches;
+  if (S->sampling) S->sample_it += std::max(0, (int)res_launches - (sample_first ? k : 0));
   const double now = clock_s(S);
   if (pro) {
     if (pro_split) {
@@ -1152,7 +1258,7 @@ int tick_impl(hobak_sched* S) {
     // the window's algorithmic bytes and launches; the sampled launches (every `every`-th one)
     // give the average launch time, so bytes / (launches * average) is the window's rate
     S->spmv_bytes += work_bytes;
-    if (ran) S->spmv_launches += (long long)m * k;
+    if (ran) S->spmv_launches += launches;
   }
   if (!S->ephemeral && S->sampling && !S->samples.empty()) {
     for (auto& sm : S->samples) {
@@ -1213,6 +1319,7 @@ int tick_impl(hobak_sched* S) {
       }
       r.st.status = worse(r.st.status, code);
       r.I->pred[nk] = iters;
+      r.I->sweeps_seen = refine ? q.sweeps : 0;
       if (nk == 0) r.I->first_iters = q.first_iters;
       r.stage = 2;
       S->stat[6] += 1;
@@ -1433,6 +1540,7 @@ int hobak_ctx_create(int device, size_t hbm_budget_bytes, hobak_ctx** out) {
   hobak_ctx* ctx = new (std::nothrow) hobak_ctx;
   if (!ctx) return HOBAK_E_NOMEM;
   ctx->device = device;
+  ctx->cus = prop.multiProcessorCount;
   ctx->budget = hbm_budget_bytes;
   if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) {
     delete ctx;
@@ -1440,6 +1548,8 @@ int hobak_ctx_create(int device, size_t hbm_budget_bytes, hobak_ctx** out) {
   }
   bool ok = true;
   for (auto& e : ctx->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
+  ok = ok && hipMalloc((void**)&ctx->tickets, 2 * sizeof(int)) == hipSuccess &&
+       hipMemset(ctx->tickets, 0, 2 * sizeof(int)) == hipSuccess;
   if (!ok || arena_ensure(ctx, 1 << 20) != HOBAK_OK || scratch_of_device(device, &ctx->scratch) != HOBAK_OK) {
     hobak_ctx_destroy(ctx);
     return HOBAK_E_HIP;
@@ -1460,6 +1570,7 @@ void hobak_ctx_destroy(hobak_ctx* ctx) {
   ctx->plans.clear();
   if (ctx->arena_dev) (void)hipFree(ctx->arena_dev);
   if (ctx->arena_host) (void)hipHostFree(ctx->arena_host);
+  if (ctx->tickets) (void)hipFree(ctx->tickets);
   for (auto& e : ctx->ev)
     if (e) (void)hipEventDestroy(e);
   for (auto& e : ctx->sample_ev)
@@ -1620,6 +1731,7 @@ int hobak_inst_create(hobak_ctx* ctx, const double* rest_xyz, int32_t nv, const 
   for (int k = 0; k < K_COUNT; k++) h.nb[k] = blocks_of(k, nv, nt, P.nslots, P.shift, ctx->update_cap, I->groups);
   h.nb[K_ASM] = blocks_of(K_ASM, nv, nt, (int)P.aslot.size(), P.shift, ctx->update_cap, I->groups);
   h.nasm = (int)P.aslot.size();
+  I->res_pack = resident_pack(ctx, I);
   h.material = material->kind;
   h.precond = params->precond;
   h.bdf = I->prm.newton_iters > 1;
@@ -1707,6 +1819,7 @@ int hobak_inst_create(hobak_ctx* ctx, const double* rest_xyz, int32_t nv, const 
     ALLOC(h.part_row_c, 6 * (size_t)h.nb[K_ROW]);
     ALLOC(h.part_upd_g, 3 * (size_t)h.nb[K_UPD]);
   }
+  if (I->res_pack > 0) ALLOC(h.xwords, resident_words(h.nb[K_SPMV], h.nb[K_UPD]));
   if (I->spatial) ALLOCT(h.agg_inv, 9 * (size_t)((nv + 21 * I->groups - 1) / (21 * I->groups)));
   {
     char* rec = nullptr;  // the record and, kCtlOffset bytes after it, the control block
@@ -2208,6 +2321,10 @@ int hobak_ctx_set_tuning(hobak_ctx* ctx, int32_t key, int32_t value) {
       if (!ctx->insts.empty() && value != ctx->agg)
         return fail(ctx, HOBAK_E_INVALID, "the local aggregates are fixed once instances exist");
       ctx->agg = value;
+      return HOBAK_OK;
+    case HOBAK_TUNE_RESIDENT:
+      if (value < 0 || value > 65536) return fail(ctx, HOBAK_E_INVALID, "resident iterations out of range");
+      ctx->resident = (value + 1) & ~1;
       return HOBAK_OK;
     case HOBAK_TUNE_UPDATE_WGS:
       if (value < 1 || value > 65536) return fail(ctx, HOBAK_E_INVALID, "update workgroups out of range");

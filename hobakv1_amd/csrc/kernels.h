@@ -114,6 +114,10 @@ struct Ctl {
   int pad[3];
   double ac_inv[3];  // coarse correction: 1 / (P^T A P), diagonal (see InstDev::coarse)
   unsigned spmv_work;  // SpMV launches that streamed this instance's matrix (wraps; a count)
+  // the resident PCG (resident.hip): tag of the last published partial sums, the meeting point of an
+  // instance's workgroups, and the launches that left the instance untouched
+  unsigned res_epoch;
+  int res_arrive, res_exit, res_abort;
   int pad4;
 };
 
@@ -130,7 +134,7 @@ struct InstStatus {
   double err;       // sqrt(res^2 / b^2) of the finished solve
   double maxR;      // |S b|^2
   unsigned spmv_work;  // Ctl::spmv_work
-  int pad;
+  int res_abort;       // Ctl::res_abort
 };
 
 // Read-only per-instance record.  Pointers typed void* hold the solve's real type T.
@@ -163,6 +167,7 @@ struct InstDev {
   double *part_pt;                  // K_SPMV: p.t
   double *part_rr, *part_rz;        // K_UPD: r.r, r.z
   double *part_res;                 // K_SPMV: refinement residual
+  unsigned long long* xwords;       // resident PCG: published partial sums (resident_words of them)
   // Reduced-precision form of an instance with no pinned vertex: the inner PCG's preconditioner
   // adds a coarse correction over the rigid translations to block Jacobi,
   //   z = M^-1 r + P (P^T A P)^-1 P^T r,   P = [I I ... I]^T  (one 3x3 identity per vertex).
@@ -350,6 +355,14 @@ hipError_t launch_agg_build(const Batch& b, int groups, int cap, hipStream_t s);
 hipError_t launch_cg_p(const Batch& upd, int parity, int cap, hipStream_t s);
 hipError_t launch_cg_spmv_p(const Batch& b, int shift, int pad, int stream, int parity, int cap, hipStream_t s,
                             hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
+// Up to `iters` PCG iterations (from scalar set 0, which holds the current set again at the end) with
+// the matrices held on chip (resident.hip); b's prefix table counts each instance's workgroups, at
+// least 1 and at most nb[K_UPD], all of which must fit on the device at once; needs every update
+// workgroup to hold one run of rows (nb[K_UPD] below the cap).  tickets: two zero ints.
+template <typename T>
+hipError_t launch_cg_resident(const Batch& b, int groups, int* tickets, int iters, hipStream_t s);
+// 8-byte words of InstDev::xwords.
+size_t resident_words(int nb_spmv, int nb_upd);
 hipError_t launch_refine_begin(const Batch& b, int cap, hipStream_t s);
 template <typename T>
 hipError_t launch_refine_init(const Batch& b, int gate, int groups, int cap, hipStream_t s);

@@ -17,28 +17,14 @@
 // active) return at once, which is the per-instance convergence mask of a batched solve.
 #include <hip/hip_ext.h>
 
-#include <cfloat>
-
 #include "kernels.h"
+#include "pcg_device.h"
 
 namespace hobak {
 
 // ---------------------------------------------------------------------------------------------
 // reductions
 // ---------------------------------------------------------------------------------------------
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-// (butterfly: each step adds the same two values in both lanes, so every lane ends with the same
-// bits)
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
 // Sum of each value over the workgroup, returned in every lane.
 template <int NV>
 __device__ __forceinline__ void block_sum(double (&v)[NV]) {
@@ -143,35 +129,10 @@ __device__ __forceinline__ T ld_stream(const HOBAK_GLOBAL T* base, size_t unifor
   return __builtin_nontemporal_load((const HOBAK_GLOBAL T*)((const HOBAK_GLOBAL char*)base + uniform_off + off));
 }
 
-// A value that is the same in every lane, moved to a scalar register.
-__device__ __forceinline__ float uniform_f(float v) {
-  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-__device__ __forceinline__ double uniform_f(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffffll));
-  const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
-// s + (m0 p0 + m1 p1 + m2 p2) with its two fused multiply-adds spelled out.  Kernels that must
-// agree bitwise (the SpMV's variants, the FP64 two-kernel and p-form iterations) then contract
-// the products the same way, whatever the compiler would pick for each.
-template <typename T>
-__device__ __forceinline__ T row3(T s, T m0, T m1, T m2, T p0, T p1, T p2) {
-  return s + fma(m2, p2, fma(m0, p0, m1 * p1));
-}
-// a0 b0 + a1 b1 + a2 b2 in FP64 with its fused multiply-adds spelled out (for the same reason).
-__device__ __forceinline__ double dot3(double a0, double a1, double a2, double b0, double b1, double b2) {
-  return fma(a2, b2, fma(a1, b1, a0 * b0));
-}
-
 template <typename T>
 __device__ __forceinline__ T d_own(bool rec, T z_own, T p_own) {
   return rec ? z_own : p_own;
 }
-
-__device__ __forceinline__ bool nonfinite(double v) { return !(v == v) || v > DBL_MAX || v < -DBL_MAX; }
 
 // An instance whose current inner solve has ended and has not yet been handled.
 __device__ __forceinline__ bool solve_ended(const HOBAK_GLOBAL Ctl* c) {
@@ -1441,26 +1402,6 @@ __global__ __launch_bounds__(kBlock) void cg_spmv_p_kernel(Batch b, int parity) 
   }
 }
 
-// Local aggregate correction of update chunk ch (rows (ch * R + q) * 21 + lane / 3, component
-// c = lane % 3 of each, as in the update kernel): g = P_I^T r over the chunk's free rows, summed
-// in a fixed lane order to the same value in every lane, then z += (P_I^T A P_I)^-1 g at the free
-// rows.  pn[q] != 0: row q is pinned or past the end.  Every lane of the wave takes part.
-template <typename T, int R>
-__device__ __forceinline__ void agg_correct(const HOBAK_GLOBAL T* ainv, int ch, int c, const T (&rq)[R],
-                                            const unsigned char (&pn)[R], T (&zq)[R]) {
-  T s = T(0);
-#pragma unroll
-  for (int q = 0; q < R; q++) s += pn[q] ? T(0) : rq[q];
-  const T g0 = wave_sum(c == 0 ? s : T(0));
-  const T g1 = wave_sum(c == 1 ? s : T(0));
-  const T g2 = wave_sum(c == 2 ? s : T(0));
-  const HOBAK_GLOBAL T* m = ainv + 9 * (size_t)ch + 3 * c;
-  const T e = fma(m[2], g2, fma(m[1], g1, m[0] * g0));
-#pragma unroll
-  for (int q = 0; q < R; q++)
-    if (!pn[q]) zq[q] += e;
-}
-
 // One lane per DOF of each of R groups of 21 rows (63 lanes) per wavefront, so that a row's
 // three DOFs share a wave and the 3x3 preconditioner apply can read its siblings' residuals with
 // cross-lane moves.  A wave covers 21 R consecutive rows and issues the loads of all R groups
@@ -2034,6 +1975,7 @@ __global__ __launch_bounds__(kBlock) void status_kernel(Batch b, InstStatus* out
     o.ref_done = c->rs.done;
     o.first_iters = I->refine ? c->rs.first_iters : s->iters;
     o.spmv_work = c->spmv_work;
+    o.res_abort = c->res_abort;
     if (I->refine) {
       o.err = c->rs.b2 > 0 ? sqrt(c->rs.res2 / c->rs.b2) : 0.0;
       o.maxR = c->rs.b2;

@@ -146,6 +146,7 @@ TUNE_UPDATE_GROUPS = 11
 TUNE_P_FORM = 12
 TUNE_COARSE = 13
 TUNE_AGG = 14
+TUNE_RESIDENT = 15
 
 _lib = None
 
@@ -248,7 +249,7 @@ class Context:
     def set_tuning(self, slice_rows=None, poll_chunk=None, max_chunks=None, graphs=None,
                    grid_cap=None, update_wgs=None, spmv_pad=None, spmv_stream_mb=None,
                    row_sort=None, compact_pct=None, update_groups=None, p_form=None, coarse=None,
-                   agg=None):
+                   agg=None, resident=None):
         """Kernel and engine tuning (see hobak_ctx_set_tuning)."""
         for key, val in ((TUNE_SLICE_ROWS, slice_rows), (TUNE_POLL_CHUNK, poll_chunk),
                          (TUNE_MAX_CHUNKS, max_chunks), (TUNE_GRAPHS, graphs),
@@ -256,7 +257,7 @@ class Context:
                          (TUNE_SPMV_PAD, spmv_pad), (TUNE_SPMV_STREAM_MB, spmv_stream_mb),
                          (TUNE_ROW_SORT, row_sort), (TUNE_COMPACT_PCT, compact_pct),
                          (TUNE_UPDATE_GROUPS, update_groups), (TUNE_P_FORM, p_form),
-                         (TUNE_COARSE, coarse), (TUNE_AGG, agg)):
+                         (TUNE_COARSE, coarse), (TUNE_AGG, agg), (TUNE_RESIDENT, resident)):
             if val is not None:
                 self.check(self.lib.hobak_ctx_set_tuning(self.h, key, int(val)), "set_tuning")
 

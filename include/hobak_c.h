@@ -297,7 +297,12 @@ int hobak_kernel_stats(hobak_inst* inst, double* spmv_avg_ms, int64_t* spmv_coun
  *                          HOBAK_TUNE_COARSE applies also adds the aggregates to its correction
  *                          (both at once: for bodies resting on the ground, where the rigid
  *                          translation alone no longer helps).  Fixed once the context holds
- *                          instances */
+ *                          instances
+ *   HOBAK_TUNE_RESIDENT    most PCG iterations per launch (rounded up to even) of the resident
+ *                          form, which holds an instance's matrix in registers and LDS for the whole
+ *                          launch; instances that do not fit the device that way run the
+ *                          two-kernel form, as does everything while GRID_CAP is set.  Results do not
+ *                          depend on it.  Default 512; 0 never */
 #define HOBAK_TUNE_SLICE_ROWS 0
 #define HOBAK_TUNE_POLL_CHUNK 2
 #define HOBAK_TUNE_MAX_CHUNKS 3
@@ -312,6 +317,7 @@ int hobak_kernel_stats(hobak_inst* inst, double* spmv_avg_ms, int64_t* spmv_coun
 #define HOBAK_TUNE_P_FORM 12
 #define HOBAK_TUNE_COARSE 13
 #define HOBAK_TUNE_AGG 14
+#define HOBAK_TUNE_RESIDENT 15
 int hobak_ctx_set_tuning(hobak_ctx* ctx, int32_t key, int32_t value);
 
 /* Continuous-batching scheduler (no counterpart in the reference, whose callers step one scene
