@@ -637,11 +637,14 @@ int agg_on(const hobak_ctx* ctx, const hobak_inst* I) {
 // Update workgroups' rows that one workgroup of the resident PCG takes when compute units are short: as
 // many as keep its slots in registers and LDS (84 FP64 or 147 FP32 64-slot steps, beside the
 // columns and vectors of a lattice), with an eighth past that streamed; 0 where the instance does
-// not qualify: its update workgroups loop over several runs of rows (more rows than the cap covers), or
-// it needs more workgroups than there are compute units.
+// not qualify: its update workgroups loop over several runs of rows (more rows than the cap covers), the
+// kernel has no variant for its layout, a slice has no blocks (vertices no tet uses), or it needs more
+// workgroups than there are compute units.
 int resident_pack(const hobak_ctx* ctx, const hobak_inst* I) {
   const int nu = I->h.nb[K_UPD], rows = 84 * I->groups;
-  if ((long)nu * rows < I->nv) return 0;
+  if ((long)nu * rows < I->nv || !resident_layout(I->P.shift, I->groups, nu)) return 0;
+  for (int s = 0; s < I->P.nslices; s++)
+    if (I->P.slice_off[s + 1] == I->P.slice_off[s]) return 0;
   const double steps = (I->tsize == 8 ? 84 : 147) * 1.125;
   const double per_row = (double)I->P.nslots / I->nv / 64.0;
   const int fit = std::max(1, (int)((steps / per_row - 2.5 * I->P.H) / rows));
@@ -1205,7 +1208,7 @@ int tick_impl(hobak_sched* S) {
     const bool all = (int)resident.size() == M.n;
     if (!all) TRY(plan_transient(ctx, resident, PR));
     for (int j = 0; j < sweeps; j++) {
-      HIPCHK(ctx, launch_cg_resident<T>(rb, M.groups, ctx->tickets, ctx->resident, s));
+      HIPCHK(ctx, launch_cg_resident<T>(rb, M.shift, M.groups, ctx->tickets, ctx->resident, s));
       TRY(launch_solve_ends<T>(ctx, all ? M : PR));
     }
     S->stat[1] += sweeps;

@@ -7,15 +7,33 @@
 
 namespace hobak {
 
-// v of lane i ^ 32 and i ^ 16 (the swap exchanges halves, or odd and even rows, of two registers; with one
-// value in both, each lane finds its partner's in one of the two results), and of lane i ^ 8.
-__device__ __forceinline__ unsigned xor32(unsigned v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  return (threadIdx.x & 32) ? r[0] : r[1];
+// (a, b) with a's upper 32 lanes and b's lower 32 exchanged (SWAP32), or a's odd rows of 16 lanes and b's even
+// ones (SWAP16).  a + b then holds, in each half (or each row of a pair), the sum over lanes i and i ^ 32
+// (i ^ 16) of what was a and of what was b: one addition reduces two values, and with a == b every
+// lane ends with its own sum.
+enum { SWAP32, SWAP16 };
+template <int W>
+__device__ __forceinline__ void lane_swap(unsigned& a, unsigned& b) {
+  const auto r = W == SWAP32 ? __builtin_amdgcn_permlane32_swap(a, b, false, false)
+                             : __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
 }
-__device__ __forceinline__ unsigned xor16(unsigned v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  return (threadIdx.x & 16) ? r[0] : r[1];
+template <int W>
+__device__ __forceinline__ float swap_add(float x, float y) {
+  unsigned a = __float_as_uint(x), b = __float_as_uint(y);
+  lane_swap<W>(a, b);
+  return __uint_as_float(a) + __uint_as_float(b);
+}
+template <int W>
+__device__ __forceinline__ double swap_add(double x, double y) {
+  const unsigned long long xb = (unsigned long long)__double_as_longlong(x);
+  const unsigned long long yb = (unsigned long long)__double_as_longlong(y);
+  unsigned al = (unsigned)xb, ah = (unsigned)(xb >> 32), bl = (unsigned)yb, bh = (unsigned)(yb >> 32);
+  lane_swap<W>(al, bl);
+  lane_swap<W>(ah, bh);
+  return __longlong_as_double((long long)((unsigned long long)ah << 32 | al)) +
+         __longlong_as_double((long long)((unsigned long long)bh << 32 | bl));
 }
 template <int CTRL>
 __device__ __forceinline__ unsigned dpp(unsigned v) {
@@ -32,29 +50,39 @@ __device__ __forceinline__ double map32(double v, F&& f) {
   const unsigned long long b = (unsigned long long)__double_as_longlong(v);
   return __longlong_as_double((long long)((unsigned long long)f((unsigned)(b >> 32)) << 32 | f((unsigned)b)));
 }
-// v + v of lane i ^ 32, and + v of lane i ^ 16.
+// Sum over each row of 16 lanes, in every lane: a butterfly over lanes i ^ 8, 4, 2, 1.  After the i ^ 8 step
+// a row repeats with period 8, so a rotation by 4 reads lane i ^ 4.
 template <typename T>
-__device__ __forceinline__ T add_xor32(T v) {
-  return v + map32(v, [](unsigned b) { return xor32(b); });
-}
-template <typename T>
-__device__ __forceinline__ T add_xor16(T v) {
-  return v + map32(v, [](unsigned b) { return xor16(b); });
-}
-// Sum over the wave, in every lane: a butterfly over lanes i ^ 32, 16, 8, 4, 2, 1.  Each step adds the
-// same two values in both lanes, so every lane ends with the same bits, and after the i ^ 8 step a
-// row of 16 repeats with period 8, so a rotation by 4 reads lane i ^ 4.  The moves are register-file
-// ones (swaps and DPP); as six ds_bpermute steps the sum took about 0.3 us, and several stand in a
-// PCG iteration's serial chain.
-template <typename T>
-__device__ __forceinline__ T wave_sum(T v) {
-  v = add_xor32(v);
-  v = add_xor16(v);
+__device__ __forceinline__ T row_sum(T v) {
   v += map32(v, [](unsigned b) { return dpp<kRor8>(b); });
   v += map32(v, [](unsigned b) { return dpp<kRor4>(b); });
   v += map32(v, [](unsigned b) { return dpp<kQuad2301>(b); });
   v += map32(v, [](unsigned b) { return dpp<kQuad1032>(b); });
   return v;
+}
+// Sum over the wave, in every lane: a butterfly over lanes i ^ 32, 16, 8, 4, 2, 1.  Each step adds the
+// same two values in both lanes, so every lane ends with the same bits.  The moves are register-file ones
+// (swaps and DPP); as six ds_bpermute steps the sum took about 0.3 us, and several stand in a PCG
+// iteration's serial chain.
+template <typename T>
+__device__ __forceinline__ T wave_sum(T v) {
+  v = swap_add<SWAP32>(v, v);
+  v = swap_add<SWAP16>(v, v);
+  return row_sum(v);
+}
+// wave_sum of a in lanes 0-31 and of b in lanes 32-63, for about the price of one.
+__device__ __forceinline__ double wave_sum2(double a, double b) {
+  double v = swap_add<SWAP32>(a, b);
+  v = swap_add<SWAP16>(v, v);
+  return row_sum(v);
+}
+// wave_sum of each group of H consecutive lanes, in each of its lanes (the other lanes' zeros left out, which
+// change nothing).
+template <int H>
+__device__ __forceinline__ double group_sum(double v) {
+  if (H == 64) v = swap_add<SWAP32>(v, v);
+  if (H >= 32) v = swap_add<SWAP16>(v, v);
+  return row_sum(v);
 }
 
 // A value that is the same in every lane, moved to scalar registers.

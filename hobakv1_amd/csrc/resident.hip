@@ -6,7 +6,8 @@
 // few hundred vertices, where nothing but the launches and their dependent loads is left.  The chip's
 // registers and LDS hold 168 MB, so here an instance's rows are dealt out to W workgroups of one
 // compute unit each, every workgroup loads its slots once, and an iteration moves only the
-// vector entries its rows couple to.
+// vector entries its rows couple to.  Measured per iteration: 10.6 us for the 40^3 lattice (FP64, 206
+// workgroups; FP32 10.1), 6.0 us for 10^3 (8 workgroups), 4.0 us for 4^3 (one).
 //
 // Arithmetic.  Every sum runs in the order of the two-kernel iteration: a row's blocks by the lane that
 // handles them there, p.t by SpMV workgroup (four slices), r.r and r.z by update workgroup (four
@@ -19,19 +20,29 @@
 // few rows past the range are computed twice, which costs less than handing t across workgroups.
 //   registers  the first kReg 64-slot steps of each wave (9 values and a 16-bit place per slot);
 //   LDS        the vector entries the slots couple to (FP64: p, which every workgroup keeps up to date
-//              itself from z; FP32: z), t, and as many further steps as fit; the steps past that
-//              are read from memory each iteration.
+//              itself from z; FP32: z), t, and as many further steps as fit, dealt so that the
+//              waves stream equally; the steps past that are read from memory each iteration.
+//
+// What bounds it.  With the matrix on chip an iteration is two waits plus a serial chain in which every
+// wave of a SIMD issues a few hundred instructions, so the loop is written for few instructions: places
+// are LDS byte offsets, a slice's three sums are reduced by swapping lanes between them, both dot
+// products share one lane reduction, rows past the end are handled by the buffer descriptors'
+// bounds, and addresses are formed anew instead of being kept where they would push the matrix out of
+// its registers.  That took the 40^3 FP64 iteration from 15.7 us to 10.6.
 //
 // Exchange.  Two all-to-all waits per iteration: on the p.t partial sums, and on the r.r / r.z partial
-// sums, which also order z.  A partial sum is published as two 8-byte words that carry half of its
-// bits and the iteration's tag each, so the wait and the read are one load, there is nothing to
+// sums, which also order z.  A partial sum is published as one 16-byte word that carries its bits in two
+// halves next to the iteration's tag, so the wait and the read are one load, there is nothing to
 // reset, and no address sees more than one writer.  Two copies alternate: a workgroup writes a copy
-// again only after every workgroup has published the step in between, hence has read it.  z and the
-// words are stored and loaded with agent-scope (L2-coherent) accesses; z's stores are
+// again only after every workgroup has published the step in between, hence has read it; likewise z is
+// overwritten only after every workgroup has published its p.t (or a zero), hence has read z.  While four
+// waves collect r.r and r.z, the other four wait for the few workgroups whose z this one needs and read it.
+// z and the words are stored and loaded device-coherently, past the dies' L2s; z's stores are
 // waited for before the partial sums that announce them.  All other data is private to a workgroup or
 // constant for the launch, so no cache is written back or invalidated: with a release and an acquire
-// the same wait costs about 10 us more over 256 workgroups.  Measured alone: 2.6 us for both waits over 8
-// workgroups, 6.6 us over 256.
+// the same wait costs about 10 us more over 256 workgroups.  One wait measured alone: 1.4 us over 8
+// workgroups, 2.5 us over 206 with 539 to 1077 words (3.2 us with 8-byte loads and 8-byte words; 2.3 us
+// with eight copies of each word or a second level of sums, which was not worth their code).
 //
 // Residency.  An instance's workgroups wait for each other, so all of them must run at once.
 // Workgroups take tickets, and tickets are dealt to instances in order, so at most the last instance
@@ -47,96 +58,137 @@ namespace hobak {
 namespace {
 
 typedef unsigned long long u64;
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x3 __attribute__((ext_vector_type(3)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kResThreads = 512;
 constexpr int kResWaves = kResThreads / 64;
-constexpr int kResLds = 160 * 1024 - 1024;    // dynamic; the rest holds the static arrays below
+constexpr int kResLds = 160 * 1024 - 1792;    // dynamic; the rest holds the static arrays below
+constexpr int kResMaxUpd = 512;               // update workgroups of an instance
 constexpr int kAbort = 1 << 30;
 constexpr u64 kJoinTicks = 20000000ull;       // 0.2 s of the 100 MHz wall clock
-constexpr u64 kWaitTicks = 500000000ull;      // 5 s; every peer is running, so this is never reached
+constexpr unsigned kWaitTicks = 500000000u;   // 5 s; every peer is running, so this is never reached
+constexpr int kAgentScope = 16;               // cache policy of a buffer access: coherent over the device's L2s
 
-// 64-slot steps of a wave held in registers: 162 registers of values and 5 or 9 of places, which
-// leaves about 80 of the 256 a wave may use at two waves per SIMD.
+// 64-slot steps of a wave held in registers: 162 or 144 registers of values and 5 or 8 of places, of the
+// 256 a wave may use at two waves per SIMD.
 template <typename T>
-constexpr int kReg = sizeof(T) == 8 ? 8 : 16;
+constexpr int kReg = sizeof(T) == 8 ? 9 : 16;
 
-__device__ __forceinline__ u64 ld_word(const HOBAK_GLOBAL u64* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+typedef __amdgpu_buffer_rsrc_t Rsrc;
+// A buffer descriptor of `bytes` bytes: accesses past them read zero and write nothing.
+__device__ __forceinline__ Rsrc buffer(void* p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)bytes, 0x00027000);
 }
-__device__ __forceinline__ void st_word(HOBAK_GLOBAL u64* p, u64 v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+template <typename T, int AUX = 0>
+__device__ __forceinline__ T buf_ld(Rsrc rs, unsigned off) {
+  if constexpr (sizeof(T) == 8) {
+    const u32x2 q = __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, AUX);
+    return __longlong_as_double((long long)((u64)q.y << 32 | q.x));
+  } else {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, AUX));
+  }
 }
-// A vector entry that other workgroups write or read in this launch (all: through the caches, when
-// the instance has one workgroup).
-__device__ __forceinline__ double ld_shared(const HOBAK_GLOBAL double* p, bool all) {
-  return all ? *p : __longlong_as_double((long long)ld_word((const HOBAK_GLOBAL u64*)p));
-}
-__device__ __forceinline__ float ld_shared(const HOBAK_GLOBAL float* p, bool all) {
-  return all ? *p
-             : __uint_as_float(__hip_atomic_load((const HOBAK_GLOBAL unsigned*)p, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT));
-}
-__device__ __forceinline__ void st_shared(HOBAK_GLOBAL double* p, double v, bool all) {
-  if (all)
-    *p = v;
-  else
-    st_word((HOBAK_GLOBAL u64*)p, (u64)__double_as_longlong(v));
-}
-__device__ __forceinline__ void st_shared(HOBAK_GLOBAL float* p, float v, bool all) {
-  if (all)
-    *p = v;
-  else
-    __hip_atomic_store((HOBAK_GLOBAL unsigned*)p, __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ void publish_word(HOBAK_GLOBAL u64* s, double v, unsigned tag) {
+template <int AUX>
+__device__ __forceinline__ void buf_st(Rsrc rs, unsigned off, double v) {
   const u64 b = (u64)__double_as_longlong(v);
-  st_word(s, (b & 0xffffffffull) | ((u64)tag << 32));
-  st_word(s + 1, (b >> 32) | ((u64)tag << 32));
+  const u32x2 q = {(unsigned)b, (unsigned)(b >> 32)};
+  __builtin_amdgcn_raw_buffer_store_b64(q, rs, off, 0, AUX);
+}
+template <int AUX>
+__device__ __forceinline__ void buf_st(Rsrc rs, unsigned off, float v) {
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rs, off, 0, AUX);
+}
+// The three entries of a vertex that another workgroup wrote in this launch.
+__device__ __forceinline__ void ld_vertex(Rsrc rs, unsigned off, double (&v)[3]) {
+  const u32x4 q = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, kAgentScope);
+  const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(rs, off + 16, 0, kAgentScope);
+  v[0] = __longlong_as_double((long long)((u64)q.y << 32 | q.x));
+  v[1] = __longlong_as_double((long long)((u64)q.w << 32 | q.z));
+  v[2] = __longlong_as_double((long long)((u64)w.y << 32 | w.x));
+}
+__device__ __forceinline__ void ld_vertex(Rsrc rs, unsigned off, float (&v)[3]) {
+  const u32x3 q = __builtin_amdgcn_raw_buffer_load_b96(rs, off, 0, kAgentScope);
+  v[0] = __uint_as_float(q.x);
+  v[1] = __uint_as_float(q.y);
+  v[2] = __uint_as_float(q.z);
 }
 
-// This lane's share (i0, i0 + 256, ...) of n published partial sums, added in ascending order; up to
-// five are in flight at once.
-__device__ __forceinline__ double poll_parts(const HOBAK_GLOBAL u64* s, int n, int i0, unsigned tag, int* failed) {
-  constexpr int KP = 5;
-  double v = 0.0;
-  for (int base = i0; base < n; base += 256 * KP) {
-    u64 lo[KP], hi[KP];
-    u64 t0 = 0;
-    for (int spin = 0;; spin++) {
-      bool ready = true;
+// A published value: its low and high word, each next to the tag of its iteration (8-byte halves are
+// stored and loaded whole, so both tags match only where both words are this iteration's).
+__device__ __forceinline__ void publish_word(Rsrc rs, unsigned i, double v, unsigned tag) {
+  const u64 b = (u64)__double_as_longlong(v);
+  const u32x4 q = {(unsigned)b, tag, (unsigned)(b >> 32), tag};
+  __builtin_amdgcn_raw_buffer_store_b128(q, rs, 16u * i, 0, kAgentScope);
+}
+
+// Spins until the K published values at byte offsets o[k] carry `tag`; gives up (false) after kWaitTicks.
+// All of a round's loads are in flight together.
+template <int K>
+__device__ __forceinline__ bool poll_words(Rsrc rs, const unsigned (&o)[K], unsigned tag, double (&v)[K]) {
+  u32x4 q[K];
+  unsigned t0 = 0;
+  for (int spin = 0;; spin++) {
+    asm volatile("" ::: "memory");  // each round loads anew
 #pragma unroll
-      for (int k = 0; k < KP; k++) {
-        const int i = base + 256 * k < n ? base + 256 * k : base;
-        lo[k] = ld_word(s + 2 * (size_t)i);
-        hi[k] = ld_word(s + 2 * (size_t)i + 1);
-      }
+    for (int k = 0; k < K; k++) q[k] = __builtin_amdgcn_raw_buffer_load_b128(rs, o[k], 0, kAgentScope);
+    unsigned miss = 0;
 #pragma unroll
-      for (int k = 0; k < KP; k++) ready = ready && (unsigned)(lo[k] >> 32) == tag && (unsigned)(hi[k] >> 32) == tag;
-      if (ready) break;
-      if ((spin & 255) == 255) {
-        const u64 now = wall_clock64();
-        if (t0 == 0) t0 = now;
-        if (now - t0 > kWaitTicks) {
-          *failed = 1;
-          return 0.0;
-        }
-      }
+    for (int k = 0; k < K; k++) miss |= (q[k].y ^ tag) | (q[k].w ^ tag);
+    if (miss == 0) break;
+    if ((spin & 255) == 255) {
+      const unsigned now = (unsigned)wall_clock64() | 1u;
+      if (t0 == 0) t0 = now;
+      if (now - t0 > kWaitTicks) return false;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < K; k++) v[k] = __longlong_as_double((long long)((u64)q[k].z << 32 | q[k].x));
+  return true;
+}
+
+// This lane's share (i0, i0 + 256, ...) of each of NK runs of n published values, KP of a run in flight at once,
+// added in ascending order; run k begins at byte base + k * 16 n.
+template <int NK, int KP>
+__device__ __forceinline__ void poll_parts(Rsrc rs, unsigned base, int n, int i0, unsigned tag, int* failed,
+                                           double (&sum)[NK]) {
+#pragma unroll
+  for (int k = 0; k < NK; k++) sum[k] = 0.0;
+  for (int b = i0; b < n; b += 256 * KP) {
+    unsigned o[NK * KP];
+    double v[NK * KP];
+#pragma unroll
+    for (int j = 0; j < KP; j++) {
+      o[j] = base + 16u * (unsigned)(j == 0 || b + 256 * j < n ? b + 256 * j : b);
+#pragma unroll
+      for (int k = 1; k < NK; k++) o[KP * k + j] = o[j] + 16u * (unsigned)(k * n);
+    }
+    if (!poll_words<NK * KP>(rs, o, tag, v)) {
+      *failed = 1;
+      return;
     }
 #pragma unroll
-    for (int k = 0; k < KP; k++)
-      if (base + 256 * k < n) v += __longlong_as_double((long long)((lo[k] & 0xffffffffull) | (hi[k] << 32)));
+    for (int k = 0; k < NK; k++)
+#pragma unroll
+      for (int j = 0; j < KP; j++)
+        if (j == 0 || b + 256 * j < n) sum[k] += v[KP * k + j];
   }
-  return v;
+}
+template <int NK>
+__device__ __forceinline__ void poll_sums(Rsrc rs, unsigned base, int n, int i0, unsigned tag, int* failed,
+                                          double (&sum)[NK]) {
+  if (n <= 256)
+    poll_parts<NK, 1>(rs, base, n, i0, tag, failed, sum);
+  else if (NK > 1 || n <= 512)
+    poll_parts<NK, 2>(rs, base, n, i0, tag, failed, sum);
+  else
+    poll_parts<NK, 5>(rs, base, n, i0, tag, failed, sum);
 }
 
 // A load at a 32-bit byte offset from a uniform base (hobak_check_offsets keeps instances in range).
 template <typename P>
 __device__ __forceinline__ P ld_off(const HOBAK_GLOBAL P* base, unsigned byte_off) {
   return *(const HOBAK_GLOBAL P*)((const HOBAK_GLOBAL char*)base + byte_off);
-}
-template <typename P>
-__device__ __forceinline__ HOBAK_GLOBAL P* at_off(HOBAK_GLOBAL P* base, unsigned byte_off) {
-  return (HOBAK_GLOBAL P*)((HOBAK_GLOBAL char*)base + byte_off);
 }
 
 // A pointer field of the record, as a global pointer in scalar registers.  The record is read after the
@@ -149,18 +201,29 @@ __device__ __forceinline__ HOBAK_GLOBAL P* uptr(P* p) {
   return (HOBAK_GLOBAL P*)(((u64)hi << 32) | lo);
 }
 
+// nonfinite() from the exponent bits alone (no constants held in registers).
+__device__ __forceinline__ bool not_finite(double v) {
+  return ((unsigned)((u64)__double_as_longlong(v) >> 52) & 0x7ffu) == 0x7ffu;
+}
+
 __device__ __forceinline__ int al16(int x) { return (x + 15) & ~15; }
 
-template <typename T, int R>
+template <typename T, int R, int H>
 __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __restrict__ I, int lb, int W,
                                                int iters, char* lds) {
   constexpr bool kF32 = sizeof(T) < sizeof(double);
   constexpr int NR = kReg<T>;
+  constexpr unsigned ts = sizeof(T);
+  constexpr int sh = H == 64 ? 6 : H == 32 ? 5 : 4, L = 64 / H;
   constexpr int UR = 84 * R;                  // rows of an update workgroup
-  constexpr int kStepBytes = 64 * 9 * (int)sizeof(T);
+  constexpr int ZS = kF32 ? 16 : 24;          // bytes of a vertex in the LDS vector
+  constexpr int GF = 4;                       // other workgroups' columns a thread has in flight at once
+  constexpr int kStepBytes = 64 * 9 * (int)ts;
   __shared__ double red[2][5][4];             // wave sums of the two reductions
   __shared__ int scan[kResWaves], rest_of[kResWaves];
   __shared__ int sh_flag, sh_failed;
+  __shared__ unsigned ubits[kResMaxUpd / 32];  // the update workgroups whose z this one reads, as bits ...
+  __shared__ unsigned short need[kResMaxUpd];  // ... and as a list
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -169,22 +232,25 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   if (S->done) return;
   const int nrows = uniform_i(I->nv);
   const size_t ns = (size_t)uniform_i(I->nslots);
-  const int sh = uniform_i(I->shift), H = 1 << sh;
   const int NU = uniform_i(I->nb[K_UPD]), NQ = uniform_i(I->nb[K_SPMV]);
   const auto slice_off = uptr(I->slice_off);
   const auto col = uptr(I->col);
   const auto A = uptr((const T*)I->A);
-  const auto mi = uptr((const T*)I->minv);
   const auto ainv = uptr((const T*)I->agg_inv);
   const auto pinned = uptr(I->pinned);
-  auto xg = uptr((T*)I->x);
-  auto rg = uptr((T*)I->r);
-  auto zg = uptr((T*)I->z);
-  auto p0 = uptr((T*)I->p0);
-  auto tg = uptr((T*)I->t);
-  auto words = uptr(I->xwords);
-  const auto prr = uptr(I->part_rr), prz = uptr(I->part_rz), pug = uptr(I->part_upd_g);
+  // fields that only a launch's first or last iteration needs are read where they are used: held through the
+  // loop, they would not leave enough scalar registers
+  auto rec = [&]() {
+    auto J = I;
+    asm volatile("" : "+s"(J));
+    return J;
+  };
   const int precond = uniform_i(I->precond);
+  const unsigned vec_bytes = 3u * ts * (unsigned)nrows;
+  const Rsrc rs_r = buffer((void*)uptr((T*)I->r), vec_bytes), rs_x = buffer((void*)uptr((T*)I->x), vec_bytes);
+  const Rsrc rs_z = buffer((void*)uptr((T*)I->z), vec_bytes);
+  const Rsrc rs_m = buffer((void*)uptr((T*)I->minv), (precond == 0 ? 1u : 3u) * vec_bytes);
+  const Rsrc rs_w = buffer((void*)uptr(I->xwords), 32u * (unsigned)(NQ + NU) + 160u * (unsigned)NU);
   const bool coarse = kF32 && uniform_i(I->coarse) != 0;
   const bool local = kF32 && uniform_i(I->agg) != 0;
   const int nval = coarse ? 5 : 2;
@@ -205,19 +271,26 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   }
   const bool solo = W == 1;
   // this workgroup's update workgroups, rows, SpMV workgroups and slices
-  const int u0 = (int)((long)lb * NU / W), u1 = (int)((long)(lb + 1) * NU / W);
+  const int u0 = uniform_i(lb * NU / W), u1 = uniform_i((lb + 1) * NU / W);  // (NU <= kResMaxUpd)
   const int nu = u1 - u0, nch = 4 * nu;
-  const int ua = u0 * UR, ub = min(u1 * UR, nrows);
+  const int ua = u0 * UR, ub = min(u1 * UR, nrows), nown = ub - ua;
   const int nslices = (nrows + H - 1) >> sh;
-  const int q0 = (ua + 4 * H - 1) >> (sh + 2), q1 = (ub + 4 * H - 1) >> (sh + 2);
+  auto first_q = [&](int row) { return (row + 4 * H - 1) >> (sh + 2); };  // the first SpMV workgroup from row on
+  const int q0 = first_q(ua), q1 = first_q(ub);
   const int nq = q1 - q0;
+  // A workgroup in whose rows no SpMV workgroup begins publishes a zero in its place, so that nobody passes the
+  // wait on p.t, and overwrites z, before every workgroup has read it: np words in all, this one's at qe
+  const bool none = tid < W && first_q(tid * NU / W * UR) == first_q(min((tid + 1) * NU / W * UR, nrows));
+  const int np = NQ + __syncthreads_count(none), qe = NQ + __syncthreads_count(none && tid < lb);
   const int sa = ua >> sh;
   int sb = (ub + H - 1) >> sh;
   if (nq > 0) sb = max(sb, min(4 * q1, nslices));
   const int nsl = sb - sa;
   const int row0 = sa << sh;
   const int nrl = min(sb << sh, nrows) - row0;
-  // the wave's slices sa + wave + 8 j: lane j holds the j-th one's first slot and step count
+  const int nrp = nsl << sh;  // the rows of whole slices
+  // the wave's slices sa + wave + 8 j: lane j holds the j-th one's first slot and step count (no slice is
+  // empty: resident_pack)
   const int nslw = nsl > wave ? (nsl - wave + kResWaves - 1) / kResWaves : 0;
   int l_beg = 0, l_nit = 0;
   if (lane < nslw) {
@@ -230,41 +303,24 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   for (int off = 32; off > 0; off >>= 1) steps += __shfl_xor(steps, off, 64);
   steps = __builtin_amdgcn_readfirstlane(steps);
   const int nrest = steps > NR ? steps - NR : 0;
-  // LDS layout, first part (sizes known from the ranges)
-  int off = 0;
-  double* ptsl = (double*)(lds + off);  // p.t of each slice
-  off += 8 * nsl;
-  double* uw = (double*)(lds + off);    // sums of each chunk
-  off += 8 * 5 * nch;
-  double* lp = (double*)(lds + off);    // solo: the partial sums
-  off += 8 * (nq + 5 * nu);
-  off = al16(off);
-  T* Tv = (T*)(lds + off);              // t (FP32: t_old between iterations)
-  off += (int)sizeof(T) * 3 * nrl;
-  T *Pv = nullptr, *Sv = Tv, *Dv = nullptr;
-  if (kF32) {
-    Pv = (T*)(lds + off);               // p of the own rows
-    Sv = Pv + 3 * nrl;                  // the rows' sums before the diagonal term and t_old
-    Dv = Sv + 3 * nrl;                  // the difference form's diagonal
-    off += (int)sizeof(T) * 9 * nrl;
-  }
-  off = al16(off);
-  const int nw = (nrows + 31) >> 5;     // the column set as a bitmap, at the top while it is built
+  // the column set as a bitmap, at the top of the LDS while the layout is not known
+  const int nw = (nrows + 31) >> 5;
   const int bm_off = kResLds - 2 * al16(4 * nw);
   unsigned* bm = (unsigned*)(lds + bm_off);
   unsigned* pre = (unsigned*)(lds + bm_off + al16(4 * nw));
   if (lane == 0) rest_of[wave] = nrest;
   if (tid == 0) sh_failed = 0;
-  bool fits = nslw <= 64 && off <= bm_off;
+  bool fits = steps <= 64 && bm_off >= 0;
   fits = __syncthreads_and(fits);
-  int NC = 0, rest_base = 0, rest_all = 0;
+  int NC = 0, rest_base = 0, rest_all = 0, nneed = 0;
   for (int w = 0; w < kResWaves; w++) {
-    if (w < wave) rest_base += rest_of[w];
-    rest_all += rest_of[w];
+    const int n = uniform_i(rest_of[w]);
+    if (w < wave) rest_base += n;
+    rest_all += n;
   }
-  int* clist = (int*)(lds + off);
-  T* zp = nullptr;
-  unsigned short* idxr = nullptr;
+  // LDS layout: vector entries, t (FP64: also the rows' z between update and next_p), FP32: p, the rows'
+  // sums and the diagonal; partial sums; places of the steps not in registers; the column list; steps
+  int off_t = 0, off_p = 0, off_s = 0, off_d = 0, off_pt = 0, off_u = 0, off_lp = 0, off_ix = 0, off_cl = 0, off_m = 0;
   if (fits) {
     for (int i = tid; i < nw; i += kResThreads) bm[i] = 0u;
     __syncthreads();
@@ -289,20 +345,29 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
     __syncthreads();
     int run = inc - cnt;
     for (int w = 0; w < kResWaves; w++) {
-      if (w < wave) run += scan[w];
-      NC += scan[w];
+      const int n = uniform_i(scan[w]);
+      if (w < wave) run += n;
+      NC += n;
     }
-    // second part: the column list, the vector entries, the places of the steps not in registers
-    off += al16(4 * NC);
-    zp = (T*)(lds + off);
-    off += al16((kF32 ? 16 : 24) * NC);
-    idxr = (unsigned short*)(lds + off);
-    off += 128 * rest_all;
-    fits = NC < 65536 && off <= bm_off;
+    const int vec = 3 * (int)ts * nrp;
+    off_t = al16(ZS * NC);
+    off_s = off_t;
+    off_p = off_t + vec;
+    if (kF32) {
+      off_s = off_p + vec;
+      off_d = off_s + vec;
+    }
+    off_pt = al16(off_t + (kF32 ? 4 : 1) * vec);
+    off_u = off_pt + 8 * nsl;
+    off_lp = off_u + 8 * 5 * nch;
+    off_ix = al16(off_lp + (solo ? 8 * (nq + 5 * nu) : 0));
+    off_cl = off_ix + 128 * rest_all;
+    off_m = al16(off_cl + 4 * NC);
+    fits = ZS * NC <= 65536 && off_m <= bm_off;
     if (fits)
       for (int i = wa; i < wb; i++) {
         pre[i] = run;
-        for (unsigned m = bm[i]; m; m &= m - 1) clist[run++] = 32 * i + __ffs(m) - 1;
+        for (unsigned m = bm[i]; m; m &= m - 1) ((int*)(lds + off_cl))[run++] = 32 * i + __ffs(m) - 1;
       }
     __syncthreads();
   }
@@ -315,17 +380,45 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
       __hip_atomic_fetch_or(arr, kAbort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (fits) {
+    int* const clist = (int*)(lds + off_cl);
+    T* const Tv = (T*)(lds + off_t);
+    T* const Sv = (T*)(lds + off_s);
+    T* const Pv = (T*)(lds + off_p);
+    T* const Dv = (T*)(lds + off_d);
+    double* const ptsl = (double*)(lds + off_pt);  // p.t of each slice
+    double* const uw = (double*)(lds + off_u);     // sums of each chunk
+    double* const lp = (double*)(lds + off_lp);    // solo: the partial sums
+    unsigned short* const idxr = (unsigned short*)(lds + off_ix);
     auto rank = [&](int c) -> int { return pre[c >> 5] + __popc(bm[c >> 5] & ((1u << (c & 31)) - 1u)); };
-    const int own0 = rank(row0);
-    // the register steps and their places; a step past the wave's last one multiplies zeros
+    // the own rows' entries in the vector; the other workgroups' are [0, flo) and [flo + nown, NC)
+    const int own0 = uniform_i(rank(row0)), flo = uniform_i(rank(ua)), nf = NC - nown;
+    auto foreign = [&](int k) -> int { return k < flo ? k : k + nown; };
+    for (int i = tid; i < kResMaxUpd / 32; i += kResThreads) ubits[i] = 0u;
+    __syncthreads();
+    for (int k = tid; k < nf; k += kResThreads) {
+      const int u = clist[foreign(k)] / UR;
+      atomicOr(&ubits[u >> 5], 1u << (u & 31));
+    }
+    __syncthreads();
+    for (int w = 0; w < (NU + 31) >> 5; w++) {
+      const unsigned m = (unsigned)uniform_i((int)ubits[w]);
+      if (tid >> 5 == w && (m >> (tid & 31) & 1u))
+        need[nneed + __popc(m & ((1u << (tid & 31)) - 1u))] = (unsigned short)tid;
+      nneed += __popc(m);
+    }
+    // the register steps and the places of their columns (byte offsets); a step past the wave's last one
+    // multiplies zeros
     T m[NR][9];
     unsigned ix[(NR + 1) / 2];
-    u64 ends = 0;  // bit k: step k (of the register steps) is the last one of its slice
+    u64 ends = 0;  // bit k: step k is the last one of its slice
     int cj = 0, cs = 0;  // cursor: the wave's slice and the step in it
-    auto skip_empty = [&](int& js) {
-      while (js < nslw && __builtin_amdgcn_readlane(l_nit, js) == 0) js++;
+    auto advance = [&](int k) {
+      if (++cs == __builtin_amdgcn_readlane(l_nit, cj)) {
+        ends |= 1ull << k;
+        cs = 0;
+        cj++;
+      }
     };
-    skip_empty(cj);
 #pragma unroll
     for (int k = 0; k < NR; k++) {
       int id = 0;
@@ -333,15 +426,10 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
       for (int e = 0; e < 9; e++) m[k][e] = T(0);
       if (k < steps) {
         const unsigned slot = (unsigned)(__builtin_amdgcn_readlane(l_beg, cj) + 64 * cs + lane);
-        id = rank(ld_off(col, 4u * slot));
+        id = ZS * rank(ld_off(col, 4u * slot));
 #pragma unroll
-        for (int e = 0; e < 9; e++) m[k][e] = ld_off(A + e * ns, (unsigned)sizeof(T) * slot);
-        if (++cs == __builtin_amdgcn_readlane(l_nit, cj)) {
-          ends |= 1ull << k;
-          cs = 0;
-          cj++;
-          skip_empty(cj);
-        }
+        for (int e = 0; e < 9; e++) m[k][e] = ld_off(A + e * ns, ts * slot);
+        advance(k);
       }
       if (k & 1)
         ix[k >> 1] |= (unsigned)id << 16;
@@ -351,46 +439,55 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
     const int rest_cj = cj, rest_cs = cs;  // where the steps past the registers begin
     for (int k = 0; k < nrest; k++) {
       const size_t slot = (size_t)(__builtin_amdgcn_readlane(l_beg, cj) + 64 * cs + lane);
-      idxr[64 * (rest_base + k) + lane] = (unsigned short)rank(col[slot]);
-      if (++cs == __builtin_amdgcn_readlane(l_nit, cj)) {
-        cs = 0;
-        cj++;
-        skip_empty(cj);
-      }
+      idxr[64 * (rest_base + k) + lane] = (unsigned short)(ZS * rank(col[slot]));
+      advance(NR + k);
     }
     __syncthreads();  // the bitmap is not read past here: its space goes to the LDS steps
-    off = al16(off);
-    const int share = (kResLds - off) / kStepBytes / kResWaves;  // LDS steps of each wave
-    const int nlds = min(nrest, share);
-    T* ml = (T*)(lds + off) + (size_t)wave * share * (64 * 9);
+    // LDS steps of each wave: all but the last `streamed` of its steps past the registers, for the least
+    // `streamed` that fits (the slowest wave of the slowest workgroup sets the pace)
+    const int cap = (kResLds - off_m) / kStepBytes;
+    int streamed = -1, taken = 0, before = 0;
+    do {
+      streamed++;
+      taken = before = 0;
+      for (int w = 0; w < kResWaves; w++) {
+        const int n = max(uniform_i(rest_of[w]) - streamed, 0);
+        if (w < wave) before += n;
+        taken += n;
+      }
+    } while (taken > cap);
+    const int nlds = uniform_i(max(nrest - streamed, 0));
+    T* const ml = (T*)(lds + off_m) + (size_t)uniform_i(before) * (64 * 9);
     cj = rest_cj;
     cs = rest_cs;
     for (int k = 0; k < nlds; k++) {
       const size_t slot = (size_t)(__builtin_amdgcn_readlane(l_beg, cj) + 64 * cs + lane);
 #pragma unroll
       for (int e = 0; e < 9; e++) ml[(9 * k + e) * 64 + lane] = A[e * ns + slot];
-      if (++cs == __builtin_amdgcn_readlane(l_nit, cj)) {
-        cs = 0;
-        cj++;
-        skip_empty(cj);
-      }
+      advance(NR + k);
     }
+    const int str_cj = cj, str_cs = cs;  // where the steps past the LDS begin
+    // (z only ever by device-coherent loads here: an ordinary one would leave its line, with other workgroups'
+    // rows, in this die's L2, where the coherent ones would then find it)
+    const auto p0 = gbl((const T*)rec()->p0), tg = gbl((const T*)rec()->t);
     for (int i = tid; i < 3 * nrl; i += kResThreads) {
       const size_t g = 3 * (size_t)row0 + i;
       if (kF32) {
         Tv[i] = first ? T(0) : tg[g];
         Pv[i] = first ? T(0) : p0[g];
-        Sv[i] = T(0);
         Dv[i] = (T)gbl(I->dg)[g];
       } else {
-        Tv[i] = T(0);
+        Tv[i] = buf_ld<T, kAgentScope>(rs_z, ts * (unsigned)g);
       }
     }
-    if (!kF32 && !first)
-      for (int i = tid; i < NC; i += kResThreads) {
+    if (kF32)
+      for (int i = tid; i < 3 * nown; i += kResThreads)
+        ((T*)lds)[4 * (flo + i / 3) + i % 3] = buf_ld<T, kAgentScope>(rs_z, ts * (unsigned)(3 * ua + i));
+    else
+      for (int i = tid; i < NC; i += kResThreads) {  // (in the first iteration beta is 0)
         const size_t g = 3 * (size_t)clist[i];
 #pragma unroll
-        for (int c = 0; c < 3; c++) zp[3 * i + c] = p0[g + c];
+        for (int c = 0; c < 3; c++) ((T*)lds)[3 * i + c] = first ? T(0) : p0[g + c];
       }
     // wait for the instance's other workgroups
     if (tid == 0) {
@@ -408,50 +505,108 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
     }
     __syncthreads();
     if (sh_flag) {
-      const int half = tid >> 8, i0 = tid & 255;
-      const int tid_ = tid, lane_ = lane;
-      const auto wpt = words;                          // p.t: [copy][NQ]
-      const auto wup = words + 4 * (size_t)NQ;         // update sums: [copy][5][NU]
+      // words: p.t [copy][NQ + NU], then the update sums [copy][5][NU]
+      const unsigned wup = 32u * (unsigned)(NQ + NU), wstride = 80u * (unsigned)NU;
+      // the update's rows of this lane: chunk `wave` of the workgroup, R rows 21 apart; the 64th lane has none
+      int urow = lane < 63 ? (4 * u0 + wave) * 21 * R + lane / 3 : 0x7fffff;
+      int c = lane - 3 * (lane / 3);
+      unsigned gofs = lane < 63 ? ts * (unsigned)(3 * urow + c) : 0x7ffff000u;
+      int srow = (wave << sh) + (lane & (H - 1));  // this lane's row in the wave's first slice
+      int tid_ = tid;
+      T* const zown = (T*)(lds + ZS * own0);
       int it = 0;
       for (; it < iters; it++) {
         const unsigned tag = epoch + 1u + (unsigned)it;  // this iteration's words
-        // opaque copies: row numbers and addresses are formed anew in each iteration instead of being
-        // kept in registers that the matrix needs
-        int tid = tid_, lane = lane_;
-        asm volatile("" : "+v"(tid), "+v"(lane));
-        // finish the previous iteration: |r|^2, r.z (and the coarse correction's sums of r)
-        double beta = 0.0;
-        if (!first) {
-          for (int k0 = 0; k0 < nval; k0 += 2) {
-            const int kind = k0 + half;
-            double v = 0.0;
-            if (kind < nval) {
-              if (it == 0) {  // left by the launch before
-                const auto src = kind == 0 ? prr : kind == 1 ? prz : pug + (size_t)(kind - 2) * NU;
-                for (int i = i0; i < NU; i += 256) v += src[i];
-              } else if (solo) {
-                for (int i = i0; i < NU; i += 256) v += lp[nq + kind * nu + i];
-              } else if (i0 < NU) {
-                v = poll_parts(wup + 2 * (size_t)(5 * ((tag - 1u) & 1u) + kind) * NU, NU, i0, tag - 1u, &sh_failed);
+        const unsigned wprev = wup + ((tag - 1u) & 1u) * wstride;
+        // opaque to the compiler: addresses derived from these are formed anew in each iteration
+        // instead of being kept in registers that the matrix needs
+        asm volatile("" : "+v"(tid_), "+v"(urow), "+v"(c), "+v"(srow), "+v"(gofs));
+        const int tid = tid_, lane = tid & 63;
+        const int left0 = nrows - urow;                  // rows q with 21 q < left0 exist
+        const unsigned gofs_m = precond == 0 || lane == 63 ? gofs : 3u * gofs;
+        const int lofs = 3 * (urow - row0) + c;          // in T entries of the rows' vectors
+        // The previous iteration's |r|^2 and r.z (and the coarse correction's sums of r) are collected by
+        // waves 0-3; meanwhile waves 4-7 wait for the few update workgroups whose z this one reads, and
+        // read it.
+        T zf[GF][3] = {};
+        if (wave < 4) {
+          if (!first) {
+            double v[2];
+            if (it == 0) {  // left by the launch before
+              v[0] = v[1] = 0.0;
+              for (int i = tid; i < NU; i += 256) {
+                v[0] += gbl(rec()->part_rr)[i];
+                v[1] += gbl(rec()->part_rz)[i];
+              }
+            } else if (solo) {
+              v[0] = v[1] = 0.0;
+              for (int i = tid; i < NU; i += 256) {
+                v[0] += lp[nq + i];
+                v[1] += lp[nq + nu + i];
+              }
+            } else {
+              poll_sums<2>(rs_w, wprev, NU, tid, tag - 1u, &sh_failed, v);
+            }
+            const double s = wave_sum2(v[0], v[1]);
+            if ((lane & 31) == 0) red[0][lane >> 5][wave] = s;
+            if (coarse) {
+              for (int k = 2; k < 5; k++) {
+                double g[1] = {0.0};
+                if (it == 0) {
+                  for (int i = tid; i < NU; i += 256) g[0] += gbl(rec()->part_upd_g)[(size_t)(k - 2) * NU + i];
+                } else if (solo) {
+                  for (int i = tid; i < NU; i += 256) g[0] += lp[nq + k * nu + i];
+                } else {
+                  poll_sums<1>(rs_w, wprev + 16u * (unsigned)(k * NU), NU, tid, tag - 1u, &sh_failed, g);
+                }
+                const double gs = wave_sum(g[0]);
+                if (lane == 0) red[0][k][wave] = gs;
               }
             }
-            v = wave_sum(v);
-            if (lane == 0 && kind < nval) red[0][kind][wave & 3] = v;
           }
-          __syncthreads();
-          if (sh_failed) {
-            done = 1;
-            status = 2;
-            break;
+        } else if (nf > 0) {
+          if (it > 0)
+            for (int i = lane; i < nneed; i += 64) {
+              const unsigned o[1] = {wprev + 16u * need[i]};
+              double v[1];
+              if (!poll_words<1>(rs_w, o, tag - 1u, v)) sh_failed = 1;
+            }
+          asm volatile("" ::: "memory");
+          if (kF32) {
+            for (int k = tid - 256; k < nf; k += 256 * GF) {
+#pragma unroll
+              for (int j = 0; j < GF; j++)
+                ld_vertex(rs_z, 3u * ts * (unsigned)clist[foreign(min(k + 256 * j, nf - 1))], zf[j]);
+#pragma unroll
+              for (int j = 0; j < GF; j++) {
+                const float4 q = make_float4((float)zf[j][0], (float)zf[j][1], (float)zf[j][2], 0.f);
+                *(float4*)(lds + ZS * foreign(min(k + 256 * j, nf - 1))) = q;
+              }
+            }
+          } else {
+#pragma unroll
+            for (int j = 0; j < GF; j++)
+              if (256 * j < nf)
+                ld_vertex(rs_z, 3u * ts * (unsigned)clist[foreign(min(tid - 256 + 256 * j, nf - 1))], zf[j]);
           }
+        }
+        __syncthreads();
+        if (sh_failed) {
+          done = 1;
+          status = 2;
+          break;
+        }
+        double beta = 0.0;
+        if (!first) {
           double tot[5];
 #pragma unroll
           for (int k = 0; k < 5; k++) {
             tot[k] = 0.0;
-            if (k < nval)
+            if (k < 2 || coarse) {
 #pragma unroll
               for (int w = 0; w < 4; w++) tot[k] += red[0][k][w];
-            tot[k] = uniform_f(tot[k]);
+              tot[k] = uniform_f(tot[k]);
+            }
           }
           const double rrv = tot[0];
           double rz = tot[1];
@@ -462,7 +617,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
             rz += tot[2] * ce0 + tot[3] * ce1 + tot[4] * ce2;
           }
           resNorm2 = rrv;
-          if (nonfinite(rrv) || !(rz == rz)) {
+          if (not_finite(rrv) || !(rz == rz)) {
             done = 1;
             status = 2;
             break;
@@ -483,52 +638,79 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           }
         }
         const T bt = (T)beta;
-        // the vector entries the slots couple to: z, or (FP64) p = z + beta p_old
-        for (int b0 = tid; b0 < NC; b0 += 4 * kResThreads) {
-          int cc[4];
-          T zv[4][3];
+        if (!kF32) {  // p = z + beta p_old at every column (the own rows' z is in Tv)
+          if (wave >= 4) {
 #pragma unroll
-          for (int j = 0; j < 4; j++) cc[j] = clist[min(b0 + j * kResThreads, NC - 1)];
+            for (int j0 = 0; j0 < GF; j0 += 2) {
+              if (256 * j0 >= nf) break;
+              T pv[2][3];
+              int k[2];
 #pragma unroll
-          for (int j = 0; j < 4; j++)
+              for (int j = 0; j < 2; j++) {
+                k[j] = tid - 256 + 256 * (j0 + j);
+                const T* q = (const T*)(lds + ZS * foreign(min(k[j], nf - 1)));
 #pragma unroll
-            for (int c = 0; c < 3; c++) zv[j][c] = ld_shared(at_off(zg + c, 3u * (unsigned)sizeof(T) * (unsigned)cc[j]), solo);
+                for (int e = 0; e < 3; e++) pv[j][e] = q[e];
+              }
 #pragma unroll
-          for (int j = 0; j < 4; j++) {
-            const int i = b0 + j * kResThreads;
-            if (i >= NC) continue;
-            if (kF32) {
-              *(float4*)(zp + 4 * i) = make_float4((float)zv[j][0], (float)zv[j][1], (float)zv[j][2], 0.f);
-            } else {
+              for (int j = 0; j < 2; j++)
+                if (k[j] < nf) {
+                  T* q = (T*)(lds + ZS * foreign(k[j]));
 #pragma unroll
-              for (int c = 0; c < 3; c++) zp[3 * i + c] = first ? zv[j][c] : fma(bt, zp[3 * i + c], zv[j][c]);
+                  for (int e = 0; e < 3; e++) q[e] = first ? zf[j0 + j][e] : fma(bt, pv[j][e], zf[j0 + j][e]);
+                }
+            }
+            for (int k = tid - 256 + 256 * GF; k < nf; k += 256) {
+              T v[3];
+              ld_vertex(rs_z, 3u * ts * (unsigned)clist[foreign(k)], v);
+              T* q = (T*)(lds + ZS * foreign(k));
+#pragma unroll
+              for (int e = 0; e < 3; e++) q[e] = first ? v[e] : fma(bt, q[e], v[e]);
+            }
+          } else {
+            T* q = (T*)(lds + ZS * flo);
+            const T* zs = Tv + 3 * (ua - row0);
+            for (int i = tid; i < 3 * nown; i += 4 * 256) {
+              T pv[4], zv[4];
+#pragma unroll
+              for (int j = 0; j < 4; j++) {
+                const int k = min(i + 256 * j, 3 * nown - 1);
+                pv[j] = q[k];
+                zv[j] = zs[k];
+              }
+#pragma unroll
+              for (int j = 0; j < 4; j++)
+                if (j == 0 || i + 256 * j < 3 * nown) q[i + 256 * j] = first ? zv[j] : fma(bt, pv[j], zv[j]);
             }
           }
+          __syncthreads();
         }
-        __syncthreads();
-        // A times those entries, slice by slice
+        // A times those entries, slice by slice, into Sv
         {
-          int js = 0;
           T s0 = T(0), s1 = T(0), s2 = T(0), d0 = T(0), d1 = T(0), d2 = T(0);
+          // the slice sums' place: the component and row this lane writes, in bytes
+          const int scomp = H == 16 ? min(lane >> 4, 2) : H == 32 ? lane >> 5 : 0;
+          unsigned so = (unsigned)off_s + ts * (unsigned)(3 * srow + scomp);
+          int orow = srow;
           auto own_entry = [&]() {  // FP32: the row's own z, which its columns are relative to
-            if (!kF32 || js >= nslw) return;
-            const int r = ((sa + wave + kResWaves * js) << sh) + (lane & (H - 1));
-            const bool live = r < nrows;
-            const T* o = zp + 4 * (own0 + (live ? r : row0) - row0);
-            d0 = live ? o[0] : T(0);
-            d1 = live ? o[1] : T(0);
-            d2 = live ? o[2] : T(0);
-          };
-          auto gather = [&](int id, T(&v)[3]) {
             if (kF32) {
-              const float4 q = *(const float4*)(zp + 4 * id);
+              const float4 q = *(const float4*)((char*)zown + ZS * min(orow, nrl - 1));
+              d0 = (T)q.x;
+              d1 = (T)q.y;
+              d2 = (T)q.z;
+            }
+          };
+          auto gather = [&](unsigned o, T(&v)[3]) {
+            if (kF32) {
+              const float4 q = *(const float4*)(lds + o);
               v[0] = (T)q.x;
               v[1] = (T)q.y;
               v[2] = (T)q.z;
             } else {
-              v[0] = zp[3 * id];
-              v[1] = zp[3 * id + 1];
-              v[2] = zp[3 * id + 2];
+              const T* q = (const T*)(lds + o);
+              v[0] = q[0];
+              v[1] = q[1];
+              v[2] = q[2];
             }
           };
           auto accumulate = [&](const T(&a)[9], const T(&v)[3]) {
@@ -537,45 +719,50 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
             s1 = row3(s1, a[3], a[4], a[5], p0v, p1v, p2v);
             s2 = row3(s2, a[6], a[7], a[8], p0v, p1v, p2v);
           };
+          // the lanes of a row add their sums (i ^ 16 first, then i ^ 32), several components at once
           auto finish_slice = [&]() {
-            if (H == 8) {
-              s0 += map32(s0, [](unsigned b) { return dpp<kRor8>(b); });
-              s1 += map32(s1, [](unsigned b) { return dpp<kRor8>(b); });
-              s2 += map32(s2, [](unsigned b) { return dpp<kRor8>(b); });
-            }
-            if (H <= 16) {
-              s0 = add_xor16(s0);
-              s1 = add_xor16(s1);
-              s2 = add_xor16(s2);
-            }
-            if (H <= 32) {
-              s0 = add_xor32(s0);
-              s1 = add_xor32(s1);
-              s2 = add_xor32(s2);
-            }
-            const int rl = ((wave + kResWaves * js) << sh) + lane;
-            if (lane < H && rl < nrl) {
-              Sv[3 * rl] = s0;
-              Sv[3 * rl + 1] = s1;
-              Sv[3 * rl + 2] = s2;
+            if (H == 16) {
+              const T a = swap_add<SWAP16>(s0, s1), b = swap_add<SWAP16>(s2, s2);
+              *(T*)(lds + so) = swap_add<SWAP32>(a, b);
+            } else if (H == 32) {
+              *(T*)(lds + so) = swap_add<SWAP32>(s0, s1);
+              const T b = swap_add<SWAP32>(s2, s2);
+              if (scomp == 0) *(T*)(lds + so + 2 * ts) = b;
+            } else {
+              T* q = (T*)(lds + so);
+              q[0] = s0;
+              q[1] = s1;
+              q[2] = s2;
             }
             s0 = s1 = s2 = T(0);
-            js++;
-            skip_empty(js);
+            so += 3 * ts * H * kResWaves;
+            orow += H * kResWaves;
             own_entry();
           };
-          skip_empty(js);
           own_entry();
+          // the first streamed step's values arrive during the others
+          T sa9[9] = {};
+          unsigned slot = 0;
+          auto fetch = [&]() {
+            size_t ns_ = ns;
+            asm volatile("" : "+s"(ns_));
+#pragma unroll
+            for (int e = 0; e < 9; e++) sa9[e] = ld_off(A + e * ns_, ts * slot);
+          };
+          if (nlds < nrest) {
+            slot = (unsigned)(__builtin_amdgcn_readlane(l_beg, str_cj) + 64 * str_cs + lane);
+            fetch();
+          }
           // the register steps in groups whose gathers are issued together (those past the wave's
           // last step multiply zeros)
-          constexpr int G = kF32 ? 4 : 2;
+          constexpr int G = kF32 ? 4 : 3;
 #pragma unroll
           for (int k0 = 0; k0 < NR; k0 += G) {
             if (k0 < steps) {
               T v[G][3];
 #pragma unroll
               for (int k = k0; k < k0 + G && k < NR; k++)
-                gather((int)((k & 1) ? ix[k >> 1] >> 16 : ix[k >> 1] & 0xffffu), v[k - k0]);
+                gather((k & 1) ? ix[k >> 1] >> 16 : ix[k >> 1] & 0xffffu, v[k - k0]);
 #pragma unroll
               for (int k = k0; k < k0 + G && k < NR; k++) {
                 accumulate(m[k], v[k - k0]);
@@ -583,38 +770,58 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
               }
             }
           }
-          int kj = rest_cj, ks = rest_cs;
-          for (int k = 0; k < nrest; k++) {
-            T a[9];
-            if (k < nlds) {
+          for (int k = 0; k < nlds; k++) {
+            T a[9], v[3];
 #pragma unroll
-              for (int e = 0; e < 9; e++) a[e] = ml[(9 * k + e) * 64 + lane];
-            } else {
-              const unsigned slot = (unsigned)(__builtin_amdgcn_readlane(l_beg, kj) + 64 * ks + lane);
-#pragma unroll
-              for (int e = 0; e < 9; e++) a[e] = ld_off(A + e * ns, (unsigned)sizeof(T) * slot);
-            }
-            T v[3];
-            gather((int)idxr[64 * (rest_base + k) + lane], v);
+            for (int e = 0; e < 9; e++) a[e] = ml[(9 * k + e) * 64 + lane];
+            gather(idxr[64 * (rest_base + k) + lane], v);
             accumulate(a, v);
-            if (++ks == __builtin_amdgcn_readlane(l_nit, kj)) {
-              ks = 0;
-              kj++;
-              skip_empty(kj);
-              finish_slice();
+            if ((ends >> (NR + k)) & 1) finish_slice();
+          }
+          if (nlds < nrest) {
+            int kj = str_cj;
+            for (int k = nlds; k < nrest; k++) {
+              T v[3];
+              gather(idxr[64 * (rest_base + k) + lane], v);
+              accumulate(sa9, v);
+              slot += 64;
+              const bool last = (ends >> (NR + k)) & 1;
+              if (last && ++kj < nslw) slot = (unsigned)(__builtin_amdgcn_readlane(l_beg, kj) + lane);
+              if (k + 1 < nrest) fetch();
+              if (last) finish_slice();
             }
           }
         }
-        // t and p of the rows, and p.t of each slice
-        for (int j = 0; j < nslw; j++) {
-          const int ls = wave + kResWaves * j;
-          const int rl = (ls << sh) + lane;
+        // the first chunk's r, x and preconditioner, which the update needs: they arrive while p.t is awaited (past
+        // the wave's chunks: rows that are not used, or past the end)
+        T rv0[R], xv[R], m0[R], m1[R], m2[R];
+        unsigned char pn[R];
+        auto load = [&](unsigned go, unsigned gm, int left, int row) {
+#pragma unroll
+          for (int q = 0; q < R; q++) {
+            pn[q] = 1;
+            if (local && 21 * q < left) pn[q] = ld_off(pinned, (unsigned)(row + 21 * q));
+            rv0[q] = buf_ld<T>(rs_r, go + 63 * q * ts);
+            xv[q] = buf_ld<T>(rs_x, go + 63 * q * ts);
+            if (precond == 0) {
+              m0[q] = buf_ld<T>(rs_m, gm + 63 * q * ts);
+            } else {
+              m0[q] = buf_ld<T>(rs_m, gm + 189 * q * ts);
+              m1[q] = buf_ld<T>(rs_m, gm + 189 * q * ts + ts);
+              m2[q] = buf_ld<T>(rs_m, gm + 189 * q * ts + 2 * ts);
+            }
+          }
+        };
+        // t and p of the rows, and p.t of each slice, L slices of the wave at a time
+        for (int j0 = 0; j0 < nslw; j0 += L) {
+          const int j = j0 + (lane >> sh);
+          const int rl = srow + j * (H * kResWaves);
           double pt = 0.0;
-          if (lane < H && rl < nrl) {
+          if (j < nslw && rl < nrl) {
             T s0 = Sv[3 * rl], s1 = Sv[3 * rl + 1], s2 = Sv[3 * rl + 2];
             if (kF32) {
-              const T* o = zp + 4 * (own0 + rl);
-              T z0 = o[0], z1 = o[1], z2 = o[2];
+              const float4 o = *(const float4*)((char*)zown + ZS * rl);
+              T z0 = (T)o.x, z1 = (T)o.y, z2 = (T)o.z;
               if (coarse) {
                 z0 += (T)ce0;
                 z1 += (T)ce1;
@@ -639,65 +846,39 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
               Pv[3 * rl + 2] = z2;
               pt = dot3((double)z0, (double)z1, (double)z2, (double)s0, (double)s1, (double)s2);
             } else {
-              const T* o = zp + 3 * (own0 + rl);
+              const T* o = zown + 3 * rl;
               pt = dot3((double)o[0], (double)o[1], (double)o[2], (double)s0, (double)s1, (double)s2);
             }
           }
-          pt = wave_sum(pt);
-          if (lane == 0) ptsl[ls] = pt;
+          pt = group_sum<H>(pt);
+          if (j < nslw && (lane & (H - 1)) == 0) ptsl[wave + kResWaves * j] = pt;
         }
         __syncthreads();
-        if (tid < nq) {
+        if (tid < max(nq, 1)) {
           double s = 0.0;
+          if (nq > 0) {
 #pragma unroll
-          for (int w = 0; w < 4; w++) {
-            const int sl = 4 * (q0 + tid) + w;
-            s += sl < nslices ? ptsl[sl - sa] : 0.0;
+            for (int w = 0; w < 4; w++) {
+              const int sl = 4 * (q0 + tid) + w;
+              s += sl < nslices ? ptsl[sl - sa] : 0.0;
+            }
           }
           if (solo)
             lp[tid] = s;
           else
-            publish_word(wpt + 2 * ((size_t)(tag & 1u) * NQ + q0 + tid), s, tag);
+            publish_word(rs_w, (tag & 1u) * (unsigned)(NQ + NU) + (unsigned)(nq > 0 ? q0 + tid : qe), s, tag);
         }
         if (solo) __syncthreads();
-        // alpha, then x, r and z of the own rows, chunk by chunk; the first chunk's loads are issued
-        // before the wait for p.t
-        const int c = lane - 3 * (lane / 3);
-        const int bse = lane - c;
-        T rv0[R], xv[R], m0[R], m1[R], m2[R];
-        unsigned char pn[R];
-        auto load = [&](int cl) {
-#pragma unroll
-          for (int q = 0; q < R; q++) {
-            const int row = ((4 * u0 + cl) * R + q) * 21 + lane / 3;
-            rv0[q] = xv[q] = m0[q] = m1[q] = m2[q] = T(0);
-            pn[q] = 1;
-            if (lane < 63 && row < nrows) {
-              const unsigned i = (unsigned)(3 * row + c);
-              if (local) pn[q] = ld_off(pinned, (unsigned)row);
-              constexpr unsigned ts = sizeof(T);
-              rv0[q] = ld_off(rg, ts * i);
-              xv[q] = ld_off(xg, ts * i);
-              if (precond == 0) {
-                m0[q] = ld_off(mi, ts * i);
-              } else {
-                m0[q] = ld_off(mi, 3 * ts * i);
-                m1[q] = ld_off(mi + 1, 3 * ts * i);
-                m2[q] = ld_off(mi + 2, 3 * ts * i);
-              }
-            }
-          }
-        };
-        if (wave < nch) load(wave);
-        if (half == 0) {
-          double v = 0.0;
+        load(gofs, gofs_m, left0, urow);
+        if (wave < 4) {
+          double v[1] = {0.0};
           if (solo) {
-            for (int i = i0; i < NQ; i += 256) v += lp[i];
-          } else if (i0 < NQ) {
-            v = poll_parts(wpt + 2 * (size_t)(tag & 1u) * NQ, NQ, i0, tag, &sh_failed);
+            for (int i = tid; i < NQ; i += 256) v[0] += lp[i];
+          } else {
+            poll_sums<1>(rs_w, 16u * (tag & 1u) * (unsigned)(NQ + NU), np, tid, tag, &sh_failed, v);
           }
-          v = wave_sum(v);
-          if (lane == 0) red[1][0][wave] = v;
+          v[0] = wave_sum(v[0]);
+          if (lane == 0) red[1][0][wave] = v[0];
         }
         __syncthreads();
         if (sh_failed) {
@@ -705,30 +886,24 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           status = 2;
           break;
         }
+        // alpha, then x, r and z of the own rows, chunk by chunk
         double ptt = 0.0;
 #pragma unroll
         for (int w = 0; w < 4; w++) ptt += red[1][0][w];
         const T alpha = (T)(absNew / uniform_f(ptt));
         for (int cl = wave; cl < nch; cl += kResWaves) {
-          if (cl != wave) load(cl);
+          const int ch = (cl - wave) * 21 * R;  // rows past the first chunk's
+          const unsigned go = gofs + 3u * ts * (unsigned)ch;
+          const int left = left0 - ch, lo = lofs + 3 * ch;
           T rq[R], zq[R];
           double rr2 = 0.0, rz = 0.0, gc = 0.0;
 #pragma unroll
           for (int q = 0; q < R; q++) {
-            const int row = ((4 * u0 + cl) * R + q) * 21 + lane / 3;
-            const bool live = lane < 63 && row < nrows;
-            const unsigned i = (unsigned)(3 * row + c);
             T rv = T(0);
-            if (live) {
-              const int rl = row - row0;
-              const T pv = kF32 ? Pv[3 * rl + c] : zp[3 * (own0 + rl) + c];
-              *at_off(xg, (unsigned)sizeof(T) * i) = fma(alpha, pv, xv[q]);
-              rv = fma(-alpha, Tv[3 * rl + c], rv0[q]);
-              *at_off(rg, (unsigned)sizeof(T) * i) = rv;
-            }
-            const T r0 = __shfl(rv, bse, 64);
-            const T r1 = __shfl(rv, bse + 1, 64);
-            const T r2 = __shfl(rv, bse + 2, 64);
+            if (21 * q < left) rv = fma(-alpha, Tv[lo + 63 * q], rv0[q]);
+            const T r0 = __shfl(rv, lane - c, 64);
+            const T r1 = __shfl(rv, lane - c + 1, 64);
+            const T r2 = __shfl(rv, lane - c + 2, 64);
             rq[q] = rv;
             zq[q] = precond == 0 ? m0[q] * rv : fma(m2[q], r2, fma(m0[q], r0, m1[q] * r1));
           }
@@ -738,42 +913,57 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           }
 #pragma unroll
           for (int q = 0; q < R; q++) {
-            const int row = ((4 * u0 + cl) * R + q) * 21 + lane / 3;
-            if (lane < 63 && row < nrows) {
-              st_shared(at_off(zg, (unsigned)sizeof(T) * (unsigned)(3 * row + c)), zq[q], solo);
+            buf_st<kAgentScope>(rs_z, go + 63 * q * ts, zq[q]);
+            if (21 * q < left) {
               rr2 = fma((double)rq[q], (double)rq[q], rr2);
               rz = fma((double)rq[q], (double)zq[q], rz);
               gc += (double)rq[q];
             }
           }
-          const double v0 = wave_sum(rr2), v1 = wave_sum(rz);
-          if (lane == 0) {
-            uw[cl] = v0;
-            uw[nch + cl] = v1;
-          }
+          const double v2 = wave_sum2(rr2, rz);
+          if ((lane & 31) == 0) uw[(lane >> 5) * nch + cl] = v2;
           if (coarse) {
+            const double g2 = wave_sum2(c == 0 ? gc : 0.0, c == 1 ? gc : 0.0), g = wave_sum(c == 2 ? gc : 0.0);
+            if ((lane & 31) == 0) uw[(2 + (lane >> 5)) * nch + cl] = g2;
+            if (lane == 0) uw[4 * nch + cl] = g;
+          }
 #pragma unroll
-            for (int k = 0; k < 3; k++) {
-              const double g = wave_sum(c == k ? gc : 0.0);
-              if (lane == 0) uw[(2 + k) * nch + cl] = g;
+          for (int q = 0; q < R; q++) {
+            buf_st<0>(rs_r, go + 63 * q * ts, rq[q]);
+            if (21 * q < left) {
+              const int l = lo + 63 * q;
+              const T pv = kF32 ? Pv[l] : zown[l];
+              buf_st<0>(rs_x, go + 63 * q * ts, fma(alpha, pv, xv[q]));
+              if (kF32)
+                zown[4 * (urow + ch + 21 * q - row0) + c] = zq[q];
+              else
+                Tv[l] = zq[q];
             }
+          }
+          if (cl + kResWaves < nch) {
+            constexpr int step = kResWaves * 21 * R;
+            load(go + 3u * ts * step, gofs_m + (precond == 0 ? 3u : 9u) * ts * (unsigned)(ch + step), left - step,
+                 urow + ch + step);
           }
         }
         // z is complete before the sums that announce it are published
-        __builtin_amdgcn_s_waitcnt(0);
+        if (!solo) __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         if (tid < nval * nu) {
-          const int kind = tid / nu, u = tid - kind * nu;
+          int kind = 0, ku = tid;  // the update sum this thread publishes
+          for (; ku >= nu; kind++) ku -= nu;
           double s = 0.0;
 #pragma unroll
-          for (int w = 0; w < 4; w++) s += uw[kind * nch + 4 * u + w];
+          for (int w = 0; w < 4; w++) s += uw[kind * nch + 4 * ku + w];
           if (solo)
-            lp[nq + kind * nu + u] = s;
+            lp[nq + kind * nu + ku] = s;
           else
-            publish_word(wup + 2 * ((size_t)(5 * (tag & 1u) + kind) * NU + u0 + u), s, tag);
+            publish_word(rs_w, 2u * (unsigned)(NQ + NU) + (5u * (tag & 1u) + (unsigned)kind) * (unsigned)NU + (unsigned)(u0 + ku),
+                         s, tag);
           if (it == iters - 1) {  // the next launch finishes this iteration from these
-            auto dst = kind == 0 ? prr : kind == 1 ? prz : pug + (size_t)(kind - 2) * NU;
-            dst[u0 + u] = s;
+            const auto J = rec();
+            auto dst = kind == 0 ? J->part_rr : kind == 1 ? J->part_rz : J->part_upd_g + (size_t)(kind - 2) * NU;
+            gbl(dst)[u0 + ku] = s;
           }
         }
         if (solo) __syncthreads();
@@ -781,11 +971,11 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
       }
       __syncthreads();
       if (!done)  // the solve goes on in another launch: its p and t
-        for (int i = tid; i < 3 * (ub - ua); i += kResThreads) {
+        for (int i = tid; i < 3 * nown; i += kResThreads) {
           const size_t g = 3 * (size_t)ua + i;
           const int l = 3 * (ua - row0) + i;
-          p0[g] = kF32 ? Pv[l] : zp[3 * own0 + l];
-          if (kF32) tg[g] = Tv[l];
+          gbl((T*)rec()->p0)[g] = kF32 ? Pv[l] : zown[l];
+          if (kF32) gbl((T*)rec()->t)[g] = Tv[l];
         }
       if (lb == 0 && tid == 0) {
 #pragma unroll
@@ -825,7 +1015,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
 
 // b: boff[i] counts the workgroups of instance i.  tickets: [0] the next ticket, [1] workgroups done;
 // both zero between launches.
-template <typename T, int R>
+template <typename T, int R, int H>
 __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void cg_resident_kernel(
     Batch b, int* tickets, int iters) {
   extern __shared__ __align__(16) char lds[];
@@ -834,8 +1024,9 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 
     sh_ticket = __hip_atomic_fetch_add(tickets, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
   int lb, W;
-  const HOBAK_GLOBAL InstDev* I = seg_find(b, __builtin_amdgcn_readfirstlane(sh_ticket), lb, W);
-  resident_solve<T, R>(I, lb, W, iters, lds);
+  const HOBAK_GLOBAL InstDev* I =
+      uptr((const InstDev*)seg_find(b, __builtin_amdgcn_readfirstlane(sh_ticket), lb, W));
+  resident_solve<T, R, H>(I, uniform_i(lb), uniform_i(W), iters, lds);
   if (threadIdx.x == 0 &&
       __hip_atomic_fetch_add(tickets + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == b.total - 1) {
     __hip_atomic_store(tickets, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -843,30 +1034,41 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 
   }
 }
 
-template <typename T, int R>
-hipError_t resident_r(const Batch& b, int* tickets, int iters, hipStream_t s) {
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&cg_resident_kernel<T, R>),
+template <typename T, int R, int H>
+hipError_t resident_rh(const Batch& b, int* tickets, int iters, hipStream_t s) {
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&cg_resident_kernel<T, R, H>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, kResLds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((cg_resident_kernel<T, R>), dim3(b.total), dim3(kResThreads), kResLds, s, b, tickets, iters);
+  hipLaunchKernelGGL((cg_resident_kernel<T, R, H>), dim3(b.total), dim3(kResThreads), kResLds, s, b, tickets, iters);
   return hipGetLastError();
+}
+template <typename T, int R>
+hipError_t resident_r(const Batch& b, int shift, int* tickets, int iters, hipStream_t s) {
+  switch (shift) {
+    case 4: return resident_rh<T, R, 16>(b, tickets, iters, s);
+    case 5: return resident_rh<T, R, 32>(b, tickets, iters, s);
+    case 6: return resident_rh<T, R, 64>(b, tickets, iters, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 }  // namespace
 
-size_t resident_words(int nb_spmv, int nb_upd) { return 4 * (size_t)nb_spmv + 20 * (size_t)nb_upd; }
+size_t resident_words(int nb_spmv, int nb_upd) { return 4 * (size_t)(nb_spmv + nb_upd) + 20 * (size_t)nb_upd; }
+bool resident_layout(int shift, int groups, int nb_upd) {
+  return shift >= 4 && shift <= 6 && (groups == 2 || groups == 4) && nb_upd <= kResMaxUpd;
+}
 
 template <typename T>
-hipError_t launch_cg_resident(const Batch& b, int groups, int* tickets, int iters, hipStream_t s) {
+hipError_t launch_cg_resident(const Batch& b, int shift, int groups, int* tickets, int iters, hipStream_t s) {
   if (b.total <= 0) return hipSuccess;
   switch (groups) {
-    case 1: return resident_r<T, 1>(b, tickets, iters, s);
-    case 2: return resident_r<T, 2>(b, tickets, iters, s);
-    case 4: return resident_r<T, 4>(b, tickets, iters, s);
+    case 2: return resident_r<T, 2>(b, shift, tickets, iters, s);
+    case 4: return resident_r<T, 4>(b, shift, tickets, iters, s);
     default: return hipErrorInvalidValue;
   }
 }
-template hipError_t launch_cg_resident<double>(const Batch&, int, int*, int, hipStream_t);
-template hipError_t launch_cg_resident<float>(const Batch&, int, int*, int, hipStream_t);
+template hipError_t launch_cg_resident<double>(const Batch&, int, int, int*, int, hipStream_t);
+template hipError_t launch_cg_resident<float>(const Batch&, int, int, int*, int, hipStream_t);
 
 }  // namespace hobak

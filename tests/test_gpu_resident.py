@@ -75,6 +75,16 @@ def test_batch_past_the_device(precision):
     _same(scs, precision, residents=(512, 32), workload="batch", steps=1)
 
 
+@pytest.mark.parametrize("precision", [F64, F32])
+def test_workgroups_in_whose_rows_no_spmv_workgroup_begins(precision):
+    """(16, 5, 4) cells: 510 rows, update workgroups of 168 and SpMV workgroups of 256; such a workgroup still
+    takes part in the wait on p.t, so that z is not overwritten before it has read it."""
+    scs = [_lattice((16, 5, 4), seed=k) for k in range(24)]
+    for pad in (0, 60):  # one update workgroup's rows each, then packed
+        _same(scs + [_lattice((24, 24, 20), seed=90 + k) for k in range(pad // 4)], precision, workload="batch",
+              steps=2)
+
+
 def test_serving_layout_streams_past_the_chip():
     """Four row groups and 64-row slices, unpinned, large enough that steps are streamed."""
     scs = [scenes.serving_instance(k, seed=7) for k in range(6)]
