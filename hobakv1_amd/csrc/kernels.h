@@ -376,6 +376,12 @@ hipError_t launch_status(const Batch& b, InstStatus* out, hipStream_t s);
 template <typename T>
 hipError_t launch_force_gather(const Batch& b, int cap, hipStream_t s, const void* stage_f_ext = nullptr,
                                double* out_ext = nullptr);
+// A state from or to pinned host memory in the caller's numbering (iperm: a caller's vertex -> ours, or null:
+// the same); a null host pointer leaves that half.
+hipError_t launch_state_in(const double* hu, const double* hv, double* u, double* v, const int* iperm, int nv,
+                           hipStream_t s);
+hipError_t launch_state_out(const double* u, const double* v, double* hu, double* hv, const int* iperm, int nv,
+                            hipStream_t s);
 hipError_t launch_copy(const void* src, void* dst, size_t bytes, hipStream_t s);
 
 }  // namespace hobak

@@ -2203,6 +2203,38 @@ hipError_t launch_force_gather(const Batch& b, int cap, hipStream_t s, const voi
   SEG_LAUNCH((force_gather_kernel<T>), b, cap, s, stage_f_ext, out_ext);
 }
 
+// One lane per DOF of u and, above 3 nv, of v; the host side is walked in order (the bus wants whole lines).
+// Bound by the bus's latency at these sizes.
+template <bool IN>
+__global__ __launch_bounds__(kBlock) void state_kernel(double* hu, double* hv, double* u, double* v,
+                                                       const int* iperm, int nv) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  const int n = 3 * nv;
+  if (i >= 2 * n) return;
+  const int d = i < n ? i : i - n;
+  auto h = gbl(i < n ? hu : hv);
+  if (!h) return;
+  const int row = d / 3;
+  const size_t j = 3 * (size_t)(iperm ? gbl(iperm)[row] : row) + (d - 3 * row);
+  auto g = gbl(i < n ? u : v);
+  if (IN)
+    g[j] = h[d];
+  else
+    h[d] = g[j];
+}
+hipError_t launch_state_in(const double* hu, const double* hv, double* u, double* v, const int* iperm, int nv,
+                           hipStream_t s) {
+  hipLaunchKernelGGL(state_kernel<true>, dim3(cdiv(6L * nv, kBlock)), dim3(kBlock), 0, s, const_cast<double*>(hu),
+                     const_cast<double*>(hv), u, v, iperm, nv);
+  return hipGetLastError();
+}
+hipError_t launch_state_out(const double* u, const double* v, double* hu, double* hv, const int* iperm, int nv,
+                            hipStream_t s) {
+  hipLaunchKernelGGL(state_kernel<false>, dim3(cdiv(6L * nv, kBlock)), dim3(kBlock), 0, s, hu, hv,
+                     const_cast<double*>(u), const_cast<double*>(v), iperm, nv);
+  return hipGetLastError();
+}
+
 hipError_t launch_copy(const void* src, void* dst, size_t bytes, hipStream_t s) {
   const size_t n = bytes / sizeof(double4);
   hipLaunchKernelGGL(copy_kernel, dim3(4096), dim3(kBlock), 0, s, (const double4*)src, (double4*)dst, n);
