@@ -53,7 +53,7 @@ struct Plan;
 constexpr double kEps = 2.220446049250313e-16;  // Eigen's default CG tolerance (machine epsilon)
 constexpr int kMaxPlans = 32;
 constexpr int kMaxSamples = 512;
-constexpr int kResidentIters = 512;
+constexpr int kResidentIters = 2048;  // a solve of more iterations goes on in a second launch, after the whole batch
 }  // namespace
 
 struct hobak_ctx {
@@ -662,7 +662,10 @@ int agg_on(const hobak_ctx* ctx, const hobak_inst* I) {
 
 // Update workgroups' rows that one workgroup of the resident PCG takes when compute units are short: as
 // many as keep its slots in registers and LDS (84 FP64 or 147 FP32 64-slot steps, beside the
-// columns and vectors of a lattice), with an eighth past that streamed; 0 where the instance does
+// columns and vectors of a lattice), with up to 30% past that streamed: streaming a few steps costs less
+// than the waits of the next whole run of rows.  48-instance FP64 batch, 128 FP32 and 24 served
+// sessions at 12.5%, 30%, 50%, 75% past the chip: 12.0, 11.7, 12.4, 12.9 ms; 20.6, 19.9, 20.7, 20.7;
+// 20.8, 18.0, 18.0, 20.9.  0 where the instance does
 // not qualify: its update workgroups loop over several runs of rows (more rows than the cap covers), the
 // kernel has no variant for its layout, a slice has no blocks (vertices no tet uses), or it needs more
 // workgroups than there are compute units.
@@ -671,9 +674,9 @@ int resident_pack(const hobak_ctx* ctx, const hobak_inst* I) {
   if ((long)nu * rows < I->nv || !resident_layout(I->P.shift, I->groups, nu)) return 0;
   for (int s = 0; s < I->P.nslices; s++)
     if (I->P.slice_off[s + 1] == I->P.slice_off[s]) return 0;
-  const double steps = (I->tsize == 8 ? 84 : 147) * 1.125;
+  const double steps = (I->tsize == 8 ? 84 : 147) * 1.3;
   const double per_row = (double)I->P.nslots / I->nv / 64.0;
-  const int fit = std::max(1, (int)((steps / per_row - 2.5 * I->P.H) / rows));
+  const int fit = std::max(1, (int)((steps / per_row - I->P.H) / rows));
   const int need = (nu + ctx->cus - 1) / ctx->cus;
   return need <= 2 * fit ? std::max(fit, need) : 0;
 }
@@ -1264,7 +1267,8 @@ int tick_impl(hobak_sched* S) {
     I->work_seen = w;
     if (M.status_host[i].res_abort != I->abort_seen) {  // did not fit, or could not run at once
       I->abort_seen = M.status_host[i].res_abort;
-      I->res_pack /= 2;
+      I->res_pack /= 2;  // more workgroups, each with fewer rows, while the device has that many
+      if (I->res_pack > 0 && (I->h.nb[K_UPD] + I->res_pack - 1) / I->res_pack > ctx->cus) I->res_pack = 0;
     }
   }
   S->stat[8] += work_bytes;

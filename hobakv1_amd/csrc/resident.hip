@@ -53,6 +53,8 @@
 #include "kernels.h"
 #include "pcg_device.h"
 
+#include <algorithm>
+
 namespace hobak {
 
 namespace {
@@ -63,8 +65,14 @@ typedef unsigned u32x3 __attribute__((ext_vector_type(3)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kResThreads = 512;
 constexpr int kResWaves = kResThreads / 64;
-constexpr int kResLds = 160 * 1024 - 1792;    // dynamic; the rest holds the static arrays below
+constexpr int kResLds = 160 * 1024 - 2048;    // dynamic; the rest holds the static arrays below
 constexpr int kResMaxUpd = 512;               // update workgroups of an instance
+// Up to this many SpMV workgroups (of four slices), a workgroup publishes p.t only of the slices that begin in
+// its rows: the sum of those that follow a group's first one, and each of the others of a group that begins in
+// another workgroup's rows by itself, so that the four are still added in order.  Without that it computes
+// the rest of its last group's rows a second time, up to 255 rows past its own 168 to 336 with 64-row slices.  A
+// lane then polls up to four words, so the rule ends where lanes would have more than one group each.
+constexpr int kSplitMax = 255;
 constexpr int kAbort = 1 << 30;
 constexpr u64 kJoinTicks = 20000000ull;       // 0.2 s of the 100 MHz wall clock
 constexpr unsigned kWaitTicks = 500000000u;   // 5 s; every peer is running, so this is never reached
@@ -224,6 +232,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   __shared__ int sh_flag, sh_failed;
   __shared__ unsigned ubits[kResMaxUpd / 32];  // the update workgroups whose z this one reads, as bits ...
   __shared__ unsigned short need[kResMaxUpd];  // ... and as a list
+  __shared__ unsigned char apart[256];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -250,7 +259,10 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   const Rsrc rs_r = buffer((void*)uptr((T*)I->r), vec_bytes), rs_x = buffer((void*)uptr((T*)I->x), vec_bytes);
   const Rsrc rs_z = buffer((void*)uptr((T*)I->z), vec_bytes);
   const Rsrc rs_m = buffer((void*)uptr((T*)I->minv), (precond == 0 ? 1u : 3u) * vec_bytes);
-  const Rsrc rs_w = buffer((void*)uptr(I->xwords), 32u * (unsigned)(NQ + NU) + 160u * (unsigned)NU);
+  // whether p.t words are single slices' where a group of four straddles two workgroups (see kSplitMax)
+  const bool split = H >= 32 && W > 1 && NQ <= kSplitMax;
+  const unsigned npt = split ? 4u * (unsigned)(NQ + 1) : (unsigned)(NQ + NU);  // p.t words of a copy
+  const Rsrc rs_w = buffer((void*)uptr(I->xwords), 32u * npt + 160u * (unsigned)NU);
   const bool coarse = kF32 && uniform_i(I->coarse) != 0;
   const bool local = kF32 && uniform_i(I->agg) != 0;
   const int nval = coarse ? 5 : 2;
@@ -276,15 +288,28 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   const int ua = u0 * UR, ub = min(u1 * UR, nrows), nown = ub - ua;
   const int nslices = (nrows + H - 1) >> sh;
   auto first_q = [&](int row) { return (row + 4 * H - 1) >> (sh + 2); };  // the first SpMV workgroup from row on
+  auto first_s = [&](int row) { return (row + H - 1) >> sh; };         // the first slice from row on
   const int q0 = first_q(ua), q1 = first_q(ub);
   const int nq = q1 - q0;
-  // A workgroup in whose rows no SpMV workgroup begins publishes a zero in its place, so that nobody passes the
-  // wait on p.t, and overwrites z, before every workgroup has read it: np words in all, this one's at qe
-  const bool none = tid < W && first_q(tid * NU / W * UR) == first_q(min((tid + 1) * NU / W * UR, nrows));
+  // A workgroup in whose rows no SpMV workgroup (split: no slice) begins publishes a zero in its place, so
+  // that nobody passes the wait on p.t, and overwrites z, before every workgroup has read it: np words in
+  // all, this one's at qe
+  const int ra = tid * NU / W * UR, rb = min((tid + 1) * NU / W * UR, nrows);
+  const bool none = tid < W && (split ? first_s(ra) == first_s(rb) : first_q(ra) == first_q(rb));
   const int np = NQ + __syncthreads_count(none), qe = NQ + __syncthreads_count(none && tid < lb);
-  const int sa = ua >> sh;
-  int sb = (ub + H - 1) >> sh;
-  if (nq > 0) sb = max(sb, min(4 * q1, nslices));
+  const int sa = ua >> sh, so = first_s(ua);
+  int sb = first_s(ub);
+  const int nown_s = sb - so;  // the slices that begin in its rows
+  if (!split && nq > 0) sb = max(sb, min(4 * q1, nslices));
+  if (tid < 256) {  // bits j: slice 4 tid + j is published by another workgroup than slice 4 tid
+    auto owner = [&](int s) { return ((s * H / UR + 1) * W - 1) / NU; };
+    unsigned m = 0;
+    if (split && tid < NQ)
+#pragma unroll
+      for (int j = 1; j < 4; j++)
+        if (4 * tid + j < nslices && owner(4 * tid + j) != owner(4 * tid)) m |= 1u << j;
+    apart[tid] = (unsigned char)m;
+  }
   const int nsl = sb - sa;
   const int row0 = sa << sh;
   const int nrl = min(sb << sh, nrows) - row0;
@@ -360,7 +385,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
     off_pt = al16(off_t + (kF32 ? 4 : 1) * vec);
     off_u = off_pt + 8 * nsl;
     off_lp = off_u + 8 * 5 * nch;
-    off_ix = al16(off_lp + (solo ? 8 * (nq + 5 * nu) : 0));
+    off_ix = al16(off_lp + (solo ? 8 * (nq + 5 * nu) : split ? 2 * nsl : 0));
     off_cl = off_ix + 128 * rest_all;
     off_m = al16(off_cl + 4 * NC);
     fits = ZS * NC <= 65536 && off_m <= bm_off;
@@ -388,6 +413,8 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
     double* const ptsl = (double*)(lds + off_pt);  // p.t of each slice
     double* const uw = (double*)(lds + off_u);     // sums of each chunk
     double* const lp = (double*)(lds + off_lp);    // solo: the partial sums
+    // split: what to publish for each slice: the word, and in bits 12 to 14 how many slices it sums (5: a zero)
+    unsigned short* const pubs = (unsigned short*)(lds + off_lp);
     unsigned short* const idxr = (unsigned short*)(lds + off_ix);
     auto rank = [&](int c) -> int { return pre[c >> 5] + __popc(bm[c >> 5] & ((1u << (c & 31)) - 1u)); };
     // the own rows' entries in the vector; the other workgroups' are [0, flo) and [flo + nown, NC)
@@ -443,6 +470,16 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
       advance(NR + k);
     }
     __syncthreads();  // the bitmap is not read past here: its space goes to the LDS steps
+    if (split)
+      for (int i = tid; i < nsl; i += kResThreads) {
+        const int s = sa + i;
+        unsigned e = 0;
+        if (nown_s == 0)
+          e = i == 0 ? 5u << 12 | 4u * (unsigned)qe : 0u;
+        else if (s >= so && ((s & 3) == 0 || (s & ~3) < so))
+          e = (unsigned)((s & 3) == 0 ? min(4, sb - s) : 1) << 12 | (unsigned)s;
+        pubs[i] = (unsigned short)e;
+      }
     // LDS steps of each wave: all but the last `streamed` of its steps past the registers, for the least
     // `streamed` that fits (the slowest wave of the slowest workgroup sets the pace)
     const int cap = (kResLds - off_m) / kStepBytes;
@@ -505,8 +542,8 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
     }
     __syncthreads();
     if (sh_flag) {
-      // words: p.t [copy][NQ + NU], then the update sums [copy][5][NU]
-      const unsigned wup = 32u * (unsigned)(NQ + NU), wstride = 80u * (unsigned)NU;
+      // words: p.t [copy][npt], then the update sums [copy][5][NU]
+      const unsigned wup = 32u * npt, wstride = 80u * (unsigned)NU;
       // the update's rows of this lane: chunk `wave` of the workgroup, R rows 21 apart; the 64th lane has none
       int urow = lane < 63 ? (4 * u0 + wave) * 21 * R + lane / 3 : 0x7fffff;
       int c = lane - 3 * (lane / 3);
@@ -854,7 +891,15 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           if (j < nslw && (lane & (H - 1)) == 0) ptsl[wave + kResWaves * j] = pt;
         }
         __syncthreads();
-        if (tid < max(nq, 1)) {
+        if (split) {
+          if (tid < nsl && (pubs[tid] >> 12) != 0) {
+            const int e = pubs[tid], n = e >> 12;
+            double v = n <= 4 ? ptsl[tid] : 0.0;
+#pragma unroll
+            for (int w = 1; w < 4; w++) v += w < n && n <= 4 ? ptsl[tid + w] : 0.0;
+            publish_word(rs_w, (tag & 1u) * npt + (unsigned)(e & 0xfff), v, tag);
+          }
+        } else if (tid < max(nq, 1)) {
           double s = 0.0;
           if (nq > 0) {
 #pragma unroll
@@ -866,7 +911,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           if (solo)
             lp[tid] = s;
           else
-            publish_word(rs_w, (tag & 1u) * (unsigned)(NQ + NU) + (unsigned)(nq > 0 ? q0 + tid : qe), s, tag);
+            publish_word(rs_w, (tag & 1u) * npt + (unsigned)(nq > 0 ? q0 + tid : qe), s, tag);
         }
         if (solo) __syncthreads();
         load(gofs, gofs_m, left0, urow);
@@ -874,8 +919,32 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           double v[1] = {0.0};
           if (solo) {
             for (int i = tid; i < NQ; i += 256) v[0] += lp[i];
+          } else if (split) {
+            if (tid < np) {
+              const unsigned m = apart[tid], o0 = 16u * (tag & 1u) * npt + 64u * (unsigned)tid;
+              if (kF32) {
+                const unsigned o[4] = {o0, o0 + (m & 2u) * 8u, o0 + (m & 4u) * 8u, o0 + (m & 8u) * 6u};
+                double g[4];
+                if (!poll_words<4>(rs_w, o, tag, g)) sh_failed = 1;
+                v[0] = g[0];
+#pragma unroll
+                for (int j = 1; j < 4; j++)
+                  if (m >> j & 1u) v[0] += g[j];
+              } else {
+                unsigned o[1] = {o0};
+                double g[1];
+                unsigned left = m | 1u;
+                while (left) {  // (the others are usually there by the time the first one is)
+                  const unsigned j = (unsigned)__ffs((int)left) - 1u;
+                  o[0] = o0 + 16u * j;
+                  if (!poll_words<1>(rs_w, o, tag, g)) sh_failed = 1;
+                  v[0] += g[0];
+                  left &= left - 1u;
+                }
+              }
+            }
           } else {
-            poll_sums<1>(rs_w, 16u * (tag & 1u) * (unsigned)(NQ + NU), np, tid, tag, &sh_failed, v);
+            poll_sums<1>(rs_w, 16u * (tag & 1u) * npt, np, tid, tag, &sh_failed, v);
           }
           v[0] = wave_sum(v[0]);
           if (lane == 0) red[1][0][wave] = v[0];
@@ -958,7 +1027,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           if (solo)
             lp[nq + kind * nu + ku] = s;
           else
-            publish_word(rs_w, 2u * (unsigned)(NQ + NU) + (5u * (tag & 1u) + (unsigned)kind) * (unsigned)NU + (unsigned)(u0 + ku),
+            publish_word(rs_w, 2u * npt + (5u * (tag & 1u) + (unsigned)kind) * (unsigned)NU + (unsigned)(u0 + ku),
                          s, tag);
           if (it == iters - 1) {  // the next launch finishes this iteration from these
             const auto J = rec();
@@ -1054,7 +1123,10 @@ hipError_t resident_r(const Batch& b, int shift, int* tickets, int iters, hipStr
 
 }  // namespace
 
-size_t resident_words(int nb_spmv, int nb_upd) { return 4 * (size_t)(nb_spmv + nb_upd) + 20 * (size_t)nb_upd; }
+size_t resident_words(int nb_spmv, int nb_upd) {
+  const size_t npt = nb_spmv <= kSplitMax ? 4 * (size_t)(nb_spmv + 1) : 0;
+  return 4 * std::max(npt, (size_t)nb_spmv + nb_upd) + 20 * (size_t)nb_upd;
+}
 bool resident_layout(int shift, int groups, int nb_upd) {
   return shift >= 4 && shift <= 6 && (groups == 2 || groups == 4) && nb_upd <= kResMaxUpd;
 }

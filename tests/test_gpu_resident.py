@@ -122,3 +122,10 @@ def test_unconnected_vertices_and_many_columns():
     sc.rest, sc.tets = sc.rest[perm], inv[sc.tets].astype(np.int32)
     sc.v0 = sc.v0.reshape(-1, 3)[perm].ravel()
     _same([sc], F64, steps=1)
+
+
+@pytest.mark.parametrize("dims", [(30, 31, 31), (30, 31, 32)])
+def test_row_counts_about_the_limit_of_single_slice_words(dims):
+    """31,744 and 32,736 rows: 248 and 256 SpMV workgroups of four 32-row slices, either side of the 255 up to
+    which a group that straddles two workgroups is published slice by slice."""
+    _same([_lattice(dims)], F32, steps=1)
