@@ -53,6 +53,7 @@ struct Plan;
 constexpr double kEps = 2.220446049250313e-16;  // Eigen's default CG tolerance (machine epsilon)
 constexpr int kMaxPlans = 32;
 constexpr int kMaxSamples = 512;
+constexpr int kResBig = 1 << 20;      // hobak_inst::res_pack of an instance on every compute unit
 constexpr int kResidentIters = 2048;  // a solve of more iterations goes on in a second launch, after the whole batch
 }  // namespace
 
@@ -666,14 +667,17 @@ int agg_on(const hobak_ctx* ctx, const hobak_inst* I) {
 // than the waits of the next whole run of rows.  48-instance FP64 batch, 128 FP32 and 24 served
 // sessions at 12.5%, 30%, 50%, 75% past the chip: 12.0, 11.7, 12.4, 12.9 ms; 20.6, 19.9, 20.7, 20.7;
 // 20.8, 18.0, 18.0, 20.9.  0 where the instance does
-// not qualify: its update workgroups loop over several runs of rows (more rows than the cap covers), the
-// kernel has no variant for its layout, a slice has no blocks (vertices no tet uses), or it needs more
-// workgroups than there are compute units.
+// not qualify: the kernel has no variant for its layout, a slice has no blocks (vertices no tet uses), or it
+// needs more workgroups than there are compute units.  kResBig: its update workgroups loop over several
+// runs of rows (more rows than the cap covers) and it takes the reduced-precision form for that, on every
+// compute unit.
 int resident_pack(const hobak_ctx* ctx, const hobak_inst* I) {
   const int nu = I->h.nb[K_UPD], rows = 84 * I->groups;
-  if ((long)nu * rows < I->nv || !resident_layout(I->P.shift, I->groups, nu)) return 0;
   for (int s = 0; s < I->P.nslices; s++)
     if (I->P.slice_off[s + 1] == I->P.slice_off[s]) return 0;
+  if ((long)nu * rows < I->nv)
+    return I->tsize < 8 && resident_layout_big(I->P.shift, I->groups, nu, ctx->cus) ? kResBig : 0;
+  if (!resident_layout(I->P.shift, I->groups, nu)) return 0;
   const double steps = (I->tsize == 8 ? 84 : 147) * 1.3;
   const double per_row = (double)I->P.nslots / I->nv / 64.0;
   const int fit = std::max(1, (int)((steps / per_row - I->P.H) / rows));
@@ -936,8 +940,10 @@ bool stream_matrix(const hobak_ctx* ctx, double solving_bytes) {
 int resident_tables(hobak_ctx* ctx, const std::vector<hobak_inst*>& m, Batch& b) {
   const int n = (int)m.size();
   long packed = 0;
+  const bool big = m[0]->res_pack == kResBig;
   for (auto* I : m) packed += (I->h.nb[K_UPD] + I->res_pack - 1) / I->res_pack;
   auto workgroups = [&](const hobak_inst* I) {
+    if (big) return ctx->cus;
     const int nu = I->h.nb[K_UPD];
     const int least = (nu + I->res_pack - 1) / I->res_pack;
     const long w = std::min<long>(nu, std::max<long>(least, least * (long)ctx->cus / packed));
@@ -1168,7 +1174,7 @@ int tick_impl(hobak_sched* S) {
   int nsolving = 0;
   double solving_bytes = 0.0;
   long solving_wgs = 0;
-  std::vector<hobak_inst*> solving, resident;
+  std::vector<hobak_inst*> solving, resident, resident_big;
   const int k = ctx->chunk_iters;
   int every = 0;
   if (S->sampling && S->ephemeral) {
@@ -1187,7 +1193,10 @@ int tick_impl(hobak_sched* S) {
   // that group over every solving instance in the two-kernel form, which the samples time
   const bool may_reside = ctx->resident > 0 && ctx->grid_cap == 0;
   for (auto& r : S->active)
-    if (r.stage == 1 && may_reside && r.I->res_pack > 0) resident.push_back(r.I);
+    if (r.stage == 1 && may_reside && r.I->res_pack > 0) {
+      resident.push_back(r.I);
+      if (r.I->res_pack == kResBig) resident_big.push_back(r.I);
+    }
   const bool sample_first = !resident.empty() && sampled_group();
   int sweeps = 1;
   for (auto& r : S->active) {
@@ -1231,13 +1240,18 @@ int tick_impl(hobak_sched* S) {
   }
   if (!resident.empty()) {
     const Range r_res("hobak resident pcg");
-    Batch rb;
-    TRY(resident_tables(ctx, resident, rb));
+    Batch rb{}, rbig{};
+    std::vector<hobak_inst*> rest;
+    for (auto* I : resident)
+      if (I->res_pack != kResBig) rest.push_back(I);
+    if (!rest.empty()) TRY(resident_tables(ctx, rest, rb));
+    if (!resident_big.empty()) TRY(resident_tables(ctx, resident_big, rbig));
     Plan PR;
     const bool all = (int)resident.size() == M.n;
     if (!all) TRY(plan_transient(ctx, resident, PR));
     for (int j = 0; j < sweeps; j++) {
-      HIPCHK(ctx, launch_cg_resident<T>(rb, M.shift, M.groups, ctx->tickets, ctx->resident, s));
+      HIPCHK(ctx, launch_cg_resident<T>(rb, M.shift, M.groups, false, ctx->tickets, ctx->resident, s));
+      if (rbig.n) HIPCHK(ctx, launch_cg_resident<T>(rbig, M.shift, M.groups, true, ctx->tickets, ctx->resident, s));
       TRY(launch_solve_ends<T>(ctx, all ? M : PR));
     }
     S->stat[1] += sweeps;
@@ -1267,7 +1281,7 @@ int tick_impl(hobak_sched* S) {
     I->work_seen = w;
     if (M.status_host[i].res_abort != I->abort_seen) {  // did not fit, or could not run at once
       I->abort_seen = M.status_host[i].res_abort;
-      I->res_pack /= 2;  // more workgroups, each with fewer rows, while the device has that many
+      I->res_pack = I->res_pack == kResBig ? 0 : I->res_pack / 2;  // more workgroups, each with fewer rows, while the device has that many
       if (I->res_pack > 0 && (I->h.nb[K_UPD] + I->res_pack - 1) / I->res_pack > ctx->cus) I->res_pack = 0;
     }
   }

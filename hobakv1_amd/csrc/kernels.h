@@ -360,9 +360,11 @@ hipError_t launch_cg_spmv_p(const Batch& b, int shift, int pad, int stream, int 
 // least 1 and at most nb[K_UPD], all of which must fit on the device at once; needs every update
 // workgroup to hold one run of rows (nb[K_UPD] below the cap).  tickets: two zero ints.
 template <typename T>
-hipError_t launch_cg_resident(const Batch& b, int shift, int groups, int* tickets, int iters, hipStream_t s);
+hipError_t launch_cg_resident(const Batch& b, int shift, int groups, bool big, int* tickets, int iters, hipStream_t s);
 // Whether the resident PCG has a variant for this slice height, update layout and row count.
 bool resident_layout(int shift, int groups, int nb_upd);
+// The same of the form for more rows than the update workgroups cover in one run each, on `wgs` workgroups.
+bool resident_layout_big(int shift, int groups, int nb_upd, int wgs);
 // 8-byte words of InstDev::xwords.
 size_t resident_words(int nb_spmv, int nb_upd);
 hipError_t launch_refine_begin(const Batch& b, int cap, hipStream_t s);

@@ -9,7 +9,7 @@
 // vector entries its rows couple to.  Measured per iteration: 10.6 us for the 40^3 lattice (FP64, 206
 // workgroups; FP32 10.1), 6.0 us for 10^3 (8 workgroups), 4.0 us for 4^3 (one).
 //
-// Arithmetic.  Every sum runs in the order of the two-kernel iteration: a row's blocks by the lane that
+// Arithmetic (all but BIG).  Every sum runs in the order of the two-kernel iteration: a row's blocks by the lane that
 // handles them there, p.t by SpMV workgroup (four slices), r.r and r.z by update workgroup (four
 // chunks of 21 R rows), and the totals over those partial sums by the same 256-lane tree.  The results
 // are therefore bitwise those of the two-kernel iteration, whatever W is, and a solve may pass from
@@ -22,6 +22,16 @@
 //   LDS        the vector entries the slots couple to (FP64: p, which every workgroup keeps up to date
 //              itself from z; FP32: z), t, and as many further steps as fit, dealt so that the
 //              waves stream equally; the steps past that are read from memory each iteration.
+//
+// BIG is the reduced-precision form for more rows than the update workgroups cover in one run each (86,016
+// with two row groups), where the two-kernel form is bound by reading 160 MB of matrix and 30 MB of vectors an
+// iteration: 46 us for 303,242 vertices.  It runs on every compute unit, which hold about half the
+// matrix and stream the rest: 30 us, of which 13 for the streamed half (9 TB/s) and 5 for the update's
+// vectors.  Its rows are dealt in single chunks of 21 R, and each workgroup publishes one word per sum; the
+// sums are so added in another order than the two-kernel form's (the same in every launch).  They
+// are FP64 sums behind FP32 step lengths, which that has not changed in any run.  FP64 solves keep the
+// two-kernel form there: their results depend on the order to 1e-8 (one iteration more or less at the end),
+// and the update workgroups' runs of rows lie too far apart for one workgroup's columns.
 //
 // What bounds it.  With the matrix on chip an iteration is two waits plus a serial chain in which every
 // wave of a SIMD issues a few hundred instructions, so the loop is written for few instructions: places
@@ -82,6 +92,10 @@ constexpr int kAgentScope = 16;               // cache policy of a buffer access
 // 256 a wave may use at two waves per SIMD.
 template <typename T>
 constexpr int kReg = sizeof(T) == 8 ? 9 : 16;
+// Streamed steps whose values are on their way at once: every workgroup of the BIG form streams about half its
+// steps (72x61x66 step: 19.4 ms with one a wave under way, 19.0 with two).
+template <bool BIG>
+constexpr int kAhead = BIG ? 2 : 1;
 
 typedef __amdgpu_buffer_rsrc_t Rsrc;
 // A buffer descriptor of `bytes` bytes: accesses past them read zero and write nothing.
@@ -89,12 +103,12 @@ __device__ __forceinline__ Rsrc buffer(void* p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)bytes, 0x00027000);
 }
 template <typename T, int AUX = 0>
-__device__ __forceinline__ T buf_ld(Rsrc rs, unsigned off) {
+__device__ __forceinline__ T buf_ld(Rsrc rs, unsigned off, int soff = 0) {
   if constexpr (sizeof(T) == 8) {
-    const u32x2 q = __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, AUX);
+    const u32x2 q = __builtin_amdgcn_raw_buffer_load_b64(rs, off, soff, AUX);
     return __longlong_as_double((long long)((u64)q.y << 32 | q.x));
   } else {
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, AUX));
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, soff, AUX));
   }
 }
 template <int AUX>
@@ -216,14 +230,15 @@ __device__ __forceinline__ bool not_finite(double v) {
 
 __device__ __forceinline__ int al16(int x) { return (x + 15) & ~15; }
 
-template <typename T, int R, int H>
+template <typename T, int R, int H, bool BIG>
 __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __restrict__ I, int lb, int W,
                                                int iters, char* lds) {
   constexpr bool kF32 = sizeof(T) < sizeof(double);
-  constexpr int NR = kReg<T>;
+  constexpr int NR = kReg<T>, ND = kAhead<BIG>;
   constexpr unsigned ts = sizeof(T);
   constexpr int sh = H == 64 ? 6 : H == 32 ? 5 : 4, L = 64 / H;
-  constexpr int UR = 84 * R;                  // rows of an update workgroup
+  constexpr int UC = BIG ? 1 : 4;             // 21 R-row chunks of a unit of rows
+  constexpr int UR = 21 * R * UC;             // its rows: an update workgroup's, or one chunk's
   constexpr int ZS = kF32 ? 16 : 24;          // bytes of a vertex in the LDS vector
   constexpr int GF = 4;                       // other workgroups' columns a thread has in flight at once
   constexpr int kStepBytes = 64 * 9 * (int)ts;
@@ -241,7 +256,9 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   if (S->done) return;
   const int nrows = uniform_i(I->nv);
   const size_t ns = (size_t)uniform_i(I->nslots);
-  const int NU = uniform_i(I->nb[K_UPD]), NQ = uniform_i(I->nb[K_SPMV]);
+  const int NB = uniform_i(I->nb[K_UPD]), NQ = uniform_i(I->nb[K_SPMV]);
+  const int NU = BIG ? (nrows + UR - 1) / UR : NB;  // units of rows ...
+  const int NX = BIG ? W : NU;                      // ... and words of each update sum
   const auto slice_off = uptr(I->slice_off);
   const auto col = uptr(I->col);
   const auto A = uptr((const T*)I->A);
@@ -260,9 +277,11 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   const Rsrc rs_z = buffer((void*)uptr((T*)I->z), vec_bytes);
   const Rsrc rs_m = buffer((void*)uptr((T*)I->minv), (precond == 0 ? 1u : 3u) * vec_bytes);
   // whether p.t words are single slices' where a group of four straddles two workgroups (see kSplitMax)
-  const bool split = H >= 32 && W > 1 && NQ <= kSplitMax;
-  const unsigned npt = split ? 4u * (unsigned)(NQ + 1) : (unsigned)(NQ + NU);  // p.t words of a copy
-  const Rsrc rs_w = buffer((void*)uptr(I->xwords), 32u * npt + 160u * (unsigned)NU);
+  const bool split = !BIG && H >= 32 && W > 1 && NQ <= kSplitMax;
+  const unsigned npt = BIG ? (unsigned)W : split ? 4u * (unsigned)(NQ + 1) : (unsigned)(NQ + NU);  // p.t words of a copy
+  const Rsrc rs_w = buffer((void*)uptr(I->xwords), 32u * npt + 160u * (unsigned)NX);
+  // (BIG: at most 64 steps of 512 x 256 threads, so the planes together stay below 2^30 bytes)
+  const Rsrc rs_a = buffer((void*)uptr((T*)I->A), (unsigned)(9 * ns * ts));
   const bool coarse = kF32 && uniform_i(I->coarse) != 0;
   const bool local = kF32 && uniform_i(I->agg) != 0;
   const int nval = coarse ? 5 : 2;
@@ -281,10 +300,10 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
     ai1 = uniform_f(ctl->ac_inv[1]);
     ai2 = uniform_f(ctl->ac_inv[2]);
   }
-  const bool solo = W == 1;
-  // this workgroup's update workgroups, rows, SpMV workgroups and slices
-  const int u0 = uniform_i(lb * NU / W), u1 = uniform_i((lb + 1) * NU / W);  // (NU <= kResMaxUpd)
-  const int nu = u1 - u0, nch = 4 * nu;
+  const bool solo = !BIG && W == 1;
+  // this workgroup's units, rows, SpMV workgroups and slices
+  const int u0 = uniform_i(lb * NU / W), u1 = uniform_i((lb + 1) * NU / W);  // (NU W < 2^31: nv < 2^25)
+  const int nu = u1 - u0, nch = UC * nu;
   const int ua = u0 * UR, ub = min(u1 * UR, nrows), nown = ub - ua;
   const int nslices = (nrows + H - 1) >> sh;
   auto first_q = [&](int row) { return (row + 4 * H - 1) >> (sh + 2); };  // the first SpMV workgroup from row on
@@ -296,11 +315,11 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   // all, this one's at qe
   const int ra = tid * NU / W * UR, rb = min((tid + 1) * NU / W * UR, nrows);
   const bool none = tid < W && (split ? first_s(ra) == first_s(rb) : first_q(ra) == first_q(rb));
-  const int np = NQ + __syncthreads_count(none), qe = NQ + __syncthreads_count(none && tid < lb);
+  const int np = BIG ? W : NQ + __syncthreads_count(none), qe = BIG ? 0 : NQ + __syncthreads_count(none && tid < lb);
   const int sa = ua >> sh, so = first_s(ua);
   int sb = first_s(ub);
   const int nown_s = sb - so;  // the slices that begin in its rows
-  if (!split && nq > 0) sb = max(sb, min(4 * q1, nslices));
+  if (!BIG && !split && nq > 0) sb = max(sb, min(4 * q1, nslices));
   if (tid < 256) {  // bits j: slice 4 tid + j is published by another workgroup than slice 4 tid
     auto owner = [&](int s) { return ((s * H / UR + 1) * W - 1) / NU; };
     unsigned m = 0;
@@ -328,14 +347,14 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   for (int off = 32; off > 0; off >>= 1) steps += __shfl_xor(steps, off, 64);
   steps = __builtin_amdgcn_readfirstlane(steps);
   const int nrest = steps > NR ? steps - NR : 0;
-  // the column set as a bitmap, at the top of the LDS while the layout is not known
+  // the column set as a bitmap, at the bottom of the LDS, below what is written while it is needed
   const int nw = (nrows + 31) >> 5;
-  const int bm_off = kResLds - 2 * al16(4 * nw);
-  unsigned* bm = (unsigned*)(lds + bm_off);
-  unsigned* pre = (unsigned*)(lds + bm_off + al16(4 * nw));
+  const int bm_end = 2 * al16(4 * nw);
+  unsigned* bm = (unsigned*)lds;
+  unsigned* pre = (unsigned*)(lds + al16(4 * nw));
   if (lane == 0) rest_of[wave] = nrest;
   if (tid == 0) sh_failed = 0;
-  bool fits = steps <= 64 && bm_off >= 0;
+  bool fits = steps <= 64 && bm_end <= kResLds;
   fits = __syncthreads_and(fits);
   int NC = 0, rest_base = 0, rest_all = 0, nneed = 0;
   for (int w = 0; w < kResWaves; w++) {
@@ -385,10 +404,10 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
     off_pt = al16(off_t + (kF32 ? 4 : 1) * vec);
     off_u = off_pt + 8 * nsl;
     off_lp = off_u + 8 * 5 * nch;
-    off_ix = al16(off_lp + (solo ? 8 * (nq + 5 * nu) : split ? 2 * nsl : 0));
+    off_ix = max(al16(off_lp + (solo ? 8 * (nq + 5 * nu) : split ? 2 * nsl : 0)), bm_end);
     off_cl = off_ix + 128 * rest_all;
     off_m = al16(off_cl + 4 * NC);
-    fits = ZS * NC <= 65536 && off_m <= bm_off;
+    fits = ZS * NC <= 65536 && off_m <= kResLds;
     if (fits)
       for (int i = wa; i < wb; i++) {
         pre[i] = run;
@@ -423,11 +442,12 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
     for (int i = tid; i < kResMaxUpd / 32; i += kResThreads) ubits[i] = 0u;
     __syncthreads();
     for (int k = tid; k < nf; k += kResThreads) {
-      const int u = clist[foreign(k)] / UR;
+      int u = clist[foreign(k)] / UR;
+      if (BIG) u = ((u + 1) * W - 1) / NU;  // the workgroup that owns the unit
       atomicOr(&ubits[u >> 5], 1u << (u & 31));
     }
     __syncthreads();
-    for (int w = 0; w < (NU + 31) >> 5; w++) {
+    for (int w = 0; w < (NX + 31) >> 5; w++) {
       const unsigned m = (unsigned)uniform_i((int)ubits[w]);
       if (tid >> 5 == w && (m >> (tid & 31) & 1u))
         need[nneed + __popc(m & ((1u << (tid & 31)) - 1u))] = (unsigned short)tid;
@@ -469,7 +489,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
       idxr[64 * (rest_base + k) + lane] = (unsigned short)(ZS * rank(col[slot]));
       advance(NR + k);
     }
-    __syncthreads();  // the bitmap is not read past here: its space goes to the LDS steps
+    __syncthreads();  // the bitmap is not read past here: the vectors take its space
     if (split)
       for (int i = tid; i < nsl; i += kResThreads) {
         const int s = sa + i;
@@ -543,9 +563,9 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
     __syncthreads();
     if (sh_flag) {
       // words: p.t [copy][npt], then the update sums [copy][5][NU]
-      const unsigned wup = 32u * npt, wstride = 80u * (unsigned)NU;
+      const unsigned wup = 32u * npt, wstride = 80u * (unsigned)NX;
       // the update's rows of this lane: chunk `wave` of the workgroup, R rows 21 apart; the 64th lane has none
-      int urow = lane < 63 ? (4 * u0 + wave) * 21 * R + lane / 3 : 0x7fffff;
+      int urow = lane < 63 ? (UC * u0 + wave) * 21 * R + lane / 3 : 0x7fffff;
       int c = lane - 3 * (lane / 3);
       unsigned gofs = lane < 63 ? ts * (unsigned)(3 * urow + c) : 0x7ffff000u;
       int srow = (wave << sh) + (lane & (H - 1));  // this lane's row in the wave's first slice
@@ -571,7 +591,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
             double v[2];
             if (it == 0) {  // left by the launch before
               v[0] = v[1] = 0.0;
-              for (int i = tid; i < NU; i += 256) {
+              for (int i = tid; i < NB; i += 256) {
                 v[0] += gbl(rec()->part_rr)[i];
                 v[1] += gbl(rec()->part_rz)[i];
               }
@@ -582,7 +602,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
                 v[1] += lp[nq + nu + i];
               }
             } else {
-              poll_sums<2>(rs_w, wprev, NU, tid, tag - 1u, &sh_failed, v);
+              poll_sums<2>(rs_w, wprev, NX, tid, tag - 1u, &sh_failed, v);
             }
             const double s = wave_sum2(v[0], v[1]);
             if ((lane & 31) == 0) red[0][lane >> 5][wave] = s;
@@ -590,11 +610,11 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
               for (int k = 2; k < 5; k++) {
                 double g[1] = {0.0};
                 if (it == 0) {
-                  for (int i = tid; i < NU; i += 256) g[0] += gbl(rec()->part_upd_g)[(size_t)(k - 2) * NU + i];
+                  for (int i = tid; i < NB; i += 256) g[0] += gbl(rec()->part_upd_g)[(size_t)(k - 2) * NB + i];
                 } else if (solo) {
                   for (int i = tid; i < NU; i += 256) g[0] += lp[nq + k * nu + i];
                 } else {
-                  poll_sums<1>(rs_w, wprev + 16u * (unsigned)(k * NU), NU, tid, tag - 1u, &sh_failed, g);
+                  poll_sums<1>(rs_w, wprev + 16u * (unsigned)(k * NX), NX, tid, tag - 1u, &sh_failed, g);
                 }
                 const double gs = wave_sum(g[0]);
                 if (lane == 0) red[0][k][wave] = gs;
@@ -777,18 +797,29 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
             own_entry();
           };
           own_entry();
-          // the first streamed step's values arrive during the others
-          T sa9[9] = {};
+          // the first streamed steps' values arrive during the others (BIG: past the last one, nothing is read)
+          T sa9[ND][9] = {};
           unsigned slot = 0;
-          auto fetch = [&]() {
+          int kj = str_cj;
+          auto fetch = [&](T(&a)[9], int k) {
             size_t ns_ = ns;
             asm volatile("" : "+s"(ns_));
+            if constexpr (BIG) {
+              const unsigned o = k < nrest ? ts * slot : 0x7ffff000u;
 #pragma unroll
-            for (int e = 0; e < 9; e++) sa9[e] = ld_off(A + e * ns_, ts * slot);
+              for (int e = 0; e < 9; e++) a[e] = buf_ld<T>(rs_a, o, (int)((unsigned)e * ts * (unsigned)ns_));
+            } else {
+#pragma unroll
+              for (int e = 0; e < 9; e++) a[e] = ld_off(A + e * ns_, ts * slot);
+            }
+            slot += 64;
+            if (k < nrest && ((ends >> (NR + k)) & 1) && ++kj < nslw)
+              slot = (unsigned)(__builtin_amdgcn_readlane(l_beg, kj) + lane);
           };
           if (nlds < nrest) {
             slot = (unsigned)(__builtin_amdgcn_readlane(l_beg, str_cj) + 64 * str_cs + lane);
-            fetch();
+#pragma unroll
+            for (int d = 0; d < ND; d++) fetch(sa9[d], nlds + d);
           }
           // the register steps in groups whose gathers are issued together (those past the wave's
           // last step multiply zeros)
@@ -815,17 +846,17 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
             accumulate(a, v);
             if ((ends >> (NR + k)) & 1) finish_slice();
           }
-          if (nlds < nrest) {
-            int kj = str_cj;
-            for (int k = nlds; k < nrest; k++) {
-              T v[3];
-              gather(idxr[64 * (rest_base + k) + lane], v);
-              accumulate(sa9, v);
-              slot += 64;
-              const bool last = (ends >> (NR + k)) & 1;
-              if (last && ++kj < nslw) slot = (unsigned)(__builtin_amdgcn_readlane(l_beg, kj) + lane);
-              if (k + 1 < nrest) fetch();
-              if (last) finish_slice();
+          for (int k0 = nlds; k0 < nrest; k0 += ND) {
+#pragma unroll
+            for (int d = 0; d < ND; d++) {
+              const int k = k0 + d;
+              if (d == 0 || k < nrest) {
+                T v[3];
+                gather(idxr[64 * (rest_base + k) + lane], v);
+                accumulate(sa9[d], v);
+                if (BIG || k + ND < nrest) fetch(sa9[d], k + ND);
+                if ((ends >> (NR + k)) & 1) finish_slice();
+              }
             }
           }
         }
@@ -887,11 +918,20 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
               pt = dot3((double)o[0], (double)o[1], (double)o[2], (double)s0, (double)s1, (double)s2);
             }
           }
+          // (the slices at the ends hold other workgroups' rows too)
+          if (BIG && (row0 + rl < ua || row0 + rl >= ub)) pt = 0.0;
           pt = group_sum<H>(pt);
           if (j < nslw && (lane & (H - 1)) == 0) ptsl[wave + kResWaves * j] = pt;
         }
         __syncthreads();
-        if (split) {
+        if (BIG) {
+          if (wave == 0) {
+            double s = 0.0;
+            for (int i = lane; i < nsl; i += 64) s += ptsl[i];
+            s = wave_sum(s);
+            if (lane == 0) publish_word(rs_w, (tag & 1u) * npt + (unsigned)lb, s, tag);
+          }
+        } else if (split) {
           if (tid < nsl && (pubs[tid] >> 12) != 0) {
             const int e = pubs[tid], n = e >> 12;
             double v = n <= 4 ? ptsl[tid] : 0.0;
@@ -977,7 +1017,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
             zq[q] = precond == 0 ? m0[q] * rv : fma(m2[q], r2, fma(m0[q], r0, m1[q] * r1));
           }
           if constexpr (kF32) {
-            if (local) agg_correct<T, R>(ainv, 4 * u0 + cl < (nrows + 21 * R - 1) / (21 * R) ? 4 * u0 + cl : 0,
+            if (local) agg_correct<T, R>(ainv, UC * u0 + cl < (nrows + 21 * R - 1) / (21 * R) ? UC * u0 + cl : 0,
                                          c, rq, pn, zq);
           }
 #pragma unroll
@@ -1018,7 +1058,19 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
         // z is complete before the sums that announce it are published
         if (!solo) __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        if (tid < nval * nu) {
+        if (BIG) {
+          if (wave < nval) {
+            double s = 0.0;
+            for (int i = lane; i < nch; i += 64) s += uw[wave * nch + i];
+            s = wave_sum(s);
+            if (lane == 0) publish_word(rs_w, 2u * npt + (5u * (tag & 1u) + (unsigned)wave) * (unsigned)NX + (unsigned)lb, s, tag);
+            if (it == iters - 1) {  // the next launch adds all NB of them
+              const auto J = rec();
+              auto dst = gbl(wave == 0 ? J->part_rr : wave == 1 ? J->part_rz : J->part_upd_g + (size_t)(wave - 2) * NB);
+              for (int i = lb + W * lane; i < NB; i += 64 * W) dst[i] = lane == 0 ? s : 0.0;
+            }
+          }
+        } else if (tid < nval * nu) {
           int kind = 0, ku = tid;  // the update sum this thread publishes
           for (; ku >= nu; kind++) ku -= nu;
           double s = 0.0;
@@ -1084,7 +1136,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
 
 // b: boff[i] counts the workgroups of instance i.  tickets: [0] the next ticket, [1] workgroups done;
 // both zero between launches.
-template <typename T, int R, int H>
+template <typename T, int R, int H, bool BIG>
 __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void cg_resident_kernel(
     Batch b, int* tickets, int iters) {
   extern __shared__ __align__(16) char lds[];
@@ -1095,7 +1147,7 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 
   int lb, W;
   const HOBAK_GLOBAL InstDev* I =
       uptr((const InstDev*)seg_find(b, __builtin_amdgcn_readfirstlane(sh_ticket), lb, W));
-  resident_solve<T, R, H>(I, uniform_i(lb), uniform_i(W), iters, lds);
+  resident_solve<T, R, H, BIG>(I, uniform_i(lb), uniform_i(W), iters, lds);
   if (threadIdx.x == 0 &&
       __hip_atomic_fetch_add(tickets + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == b.total - 1) {
     __hip_atomic_store(tickets, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1103,20 +1155,21 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 
   }
 }
 
-template <typename T, int R, int H>
+template <typename T, int R, int H, bool BIG>
 hipError_t resident_rh(const Batch& b, int* tickets, int iters, hipStream_t s) {
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&cg_resident_kernel<T, R, H>),
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&cg_resident_kernel<T, R, H, BIG>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, kResLds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((cg_resident_kernel<T, R, H>), dim3(b.total), dim3(kResThreads), kResLds, s, b, tickets, iters);
+  hipLaunchKernelGGL((cg_resident_kernel<T, R, H, BIG>), dim3(b.total), dim3(kResThreads), kResLds, s, b, tickets,
+                     iters);
   return hipGetLastError();
 }
-template <typename T, int R>
+template <typename T, int R, bool BIG>
 hipError_t resident_r(const Batch& b, int shift, int* tickets, int iters, hipStream_t s) {
   switch (shift) {
-    case 4: return resident_rh<T, R, 16>(b, tickets, iters, s);
-    case 5: return resident_rh<T, R, 32>(b, tickets, iters, s);
-    case 6: return resident_rh<T, R, 64>(b, tickets, iters, s);
+    case 4: return resident_rh<T, R, 16, BIG>(b, tickets, iters, s);
+    case 5: return resident_rh<T, R, 32, BIG>(b, tickets, iters, s);
+    case 6: return resident_rh<T, R, 64, BIG>(b, tickets, iters, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1130,17 +1183,24 @@ size_t resident_words(int nb_spmv, int nb_upd) {
 bool resident_layout(int shift, int groups, int nb_upd) {
   return shift >= 4 && shift <= 6 && (groups == 2 || groups == 4) && nb_upd <= kResMaxUpd;
 }
+bool resident_layout_big(int shift, int groups, int nb_upd, int wgs) {
+  return shift >= 4 && shift <= 6 && (groups == 2 || groups == 4) && wgs <= std::min(nb_upd, 256);
+}
 
 template <typename T>
-hipError_t launch_cg_resident(const Batch& b, int shift, int groups, int* tickets, int iters, hipStream_t s) {
+hipError_t launch_cg_resident(const Batch& b, int shift, int groups, bool big, int* tickets, int iters, hipStream_t s) {
   if (b.total <= 0) return hipSuccess;
+  if constexpr (sizeof(T) < sizeof(double)) {
+    if (big) return groups == 2 ? resident_r<T, 2, true>(b, shift, tickets, iters, s) : resident_r<T, 4, true>(b, shift, tickets, iters, s);
+  }
+  if (big) return hipErrorInvalidValue;
   switch (groups) {
-    case 2: return resident_r<T, 2>(b, shift, tickets, iters, s);
-    case 4: return resident_r<T, 4>(b, shift, tickets, iters, s);
+    case 2: return resident_r<T, 2, false>(b, shift, tickets, iters, s);
+    case 4: return resident_r<T, 4, false>(b, shift, tickets, iters, s);
     default: return hipErrorInvalidValue;
   }
 }
-template hipError_t launch_cg_resident<double>(const Batch&, int, int, int*, int, hipStream_t);
-template hipError_t launch_cg_resident<float>(const Batch&, int, int, int*, int, hipStream_t);
+template hipError_t launch_cg_resident<double>(const Batch&, int, int, bool, int*, int, hipStream_t);
+template hipError_t launch_cg_resident<float>(const Batch&, int, int, bool, int*, int, hipStream_t);
 
 }  // namespace hobak

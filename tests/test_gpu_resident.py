@@ -129,3 +129,23 @@ def test_row_counts_about_the_limit_of_single_slice_words(dims):
     """31,744 and 32,736 rows: 248 and 256 SpMV workgroups of four 32-row slices, either side of the 255 up to
     which a group that straddles two workgroups is published slice by slice."""
     _same([_lattice(dims)], F32, steps=1)
+
+
+@pytest.mark.parametrize("precision,pin,tuning", [
+    (F64, True, {}), (F32, True, {}), (F32, False, {}), (F32, False, dict(slice_rows=16)),
+    (F32, True, dict(slice_rows=64, update_groups=4))])
+def test_more_rows_than_the_update_workgroups_cover(precision, pin, tuning):
+    """256 update workgroups of 168 (or 336) rows and 49,248 (or 91,125) rows: the form on every compute unit, which
+    streams what does not fit and publishes one word per workgroup.  Its sums run in another order, so the
+    bar is the parity bar, for one launch, for many, and in a batch beside an ordinary instance.  FP64
+    solves take the two-kernel form there."""
+    dims = (44, 44, 44) if "update_groups" in tuning else (35, 37, 35)
+    big, small = _lattice(dims, pin=pin), _lattice((6, 5, 7))
+    tuning = dict(update_wgs=256, **tuning)
+    want, ws = _steps([big], precision, 0, steps=1, tuning=tuning)
+    for n, scs in ((512, [big]), (6, [big]), (512, [small, big])):
+        print(f"  nt {big.nt} precision {precision} {tuning} {n} {len(scs)}", flush=True)
+        got, gs = _steps(scs, precision, n, steps=1, tuning=tuning)
+        x, y = big.rest.ravel() + got[-1][0], big.rest.ravel() + want[0][0]
+        assert np.linalg.norm(x - y) <= 1e-9 * np.linalg.norm(y), n
+        assert gs[0][-1][0] == ws[0][0][0] and abs(gs[0][-1][1][0] - ws[0][0][1][0]) <= 1, (n, gs, ws)
