@@ -75,6 +75,7 @@ struct hobak_ctx {
   int agg = 0;                         // reduced-precision form: spatial order and local aggregates (2: also with the coarse correction)
   int resident = kResidentIters;       // resident PCG: iterations per launch, 0 off
   int cus = 0;                         // compute units of the device
+  bool dies = true;                    // small batches of the resident PCG run on one die each
   int* tickets = nullptr;              // resident PCG launches of this context's stream
   hipStream_t stream = nullptr;
   size_t budget = 0;
@@ -933,11 +934,35 @@ bool stream_matrix(const hobak_ctx* ctx, double solving_bytes) {
   return solving_bytes > (double)ctx->spmv_stream_mb * (1 << 20);
 }
 
+// Workgroups of an instance that runs on one die: one per update workgroup's rows up to a die's compute units, and
+// two update workgroups' rows each past that; 0 where it does not fit.  The exchange within a die's L2 is worth
+// the twice longer rows but not more: steps of 30, 56 and 94 update workgroups in FP32 took 0.96, 1.14 and
+// 1.77 ms on one die and 1.10, 1.31 and 1.65 ms over all of them; 30, 39 and 56 in FP64 1.04, 1.39 and
+// 1.48 ms, and 1.21, 1.38 and 1.57.
+int die_workgroups(const hobak_inst* I) {
+  const int nu = I->h.nb[K_UPD], per = (nu + kResDieWgs - 1) / kResDieWgs;
+  return I->res_pack != kResBig && per <= std::min(I->res_pack, 2) ? (nu + per - 1) / per : 0;
+}
+// Whether the instances run on one die each, and if so the most workgroups of any: at most as many as there are
+// dies, each within one.
+int resident_per_die(const hobak_ctx* ctx, const std::vector<hobak_inst*>& m) {
+  if (!ctx->dies || ctx->cus != kResDies * kResDieWgs || (int)m.size() > kResDies) return 0;
+  int most = 0;
+  for (auto* I : m) {
+    const int w = die_workgroups(I);
+    if (w == 0) return 0;
+    most = std::max(most, w);
+  }
+  return most > 1 ? most : 0;  // (a workgroup by itself exchanges nothing)
+}
+
 // The resident PCG's launch tables in the arena: the instances, largest first (their solves take the
 // most iterations, and what runs last should be short), and the workgroups of each.  An instance takes
 // as few workgroups as hold its matrix on chip (res_pack) when the batch fills the device's
 // compute units that way, and up to one per update workgroup's rows while compute units are left.
-int resident_tables(hobak_ctx* ctx, const std::vector<hobak_inst*>& m, Batch& b) {
+// `die_wgs`: 0, or the most workgroups of any instance where each instance runs on one die (see
+// resident_per_die), which gives them their number.
+int resident_tables(hobak_ctx* ctx, const std::vector<hobak_inst*>& m, int die_wgs, Batch& b) {
   const int n = (int)m.size();
   long packed = 0;
   const bool big = m[0]->res_pack == kResBig;
@@ -945,6 +970,7 @@ int resident_tables(hobak_ctx* ctx, const std::vector<hobak_inst*>& m, Batch& b)
   auto workgroups = [&](const hobak_inst* I) {
     if (big) return ctx->cus;
     const int nu = I->h.nb[K_UPD];
+    if (die_wgs) return die_workgroups(I);
     const int least = (nu + I->res_pack - 1) / I->res_pack;
     const long w = std::min<long>(nu, std::max<long>(least, least * (long)ctx->cus / packed));
     const int per = (int)((nu + w - 1) / w);
@@ -1198,7 +1224,7 @@ int tick_impl(hobak_sched* S) {
       if (r.I->res_pack == kResBig) resident_big.push_back(r.I);
     }
   const bool sample_first = !resident.empty() && sampled_group();
-  int sweeps = 1;
+  int sweeps = 1, die_wgs = 0;
   for (auto& r : S->active) {
     if (r.stage != 1) continue;
     const bool res = may_reside && r.I->res_pack > 0;
@@ -1244,13 +1270,17 @@ int tick_impl(hobak_sched* S) {
     std::vector<hobak_inst*> rest;
     for (auto* I : resident)
       if (I->res_pack != kResBig) rest.push_back(I);
-    if (!rest.empty()) TRY(resident_tables(ctx, rest, rb));
-    if (!resident_big.empty()) TRY(resident_tables(ctx, resident_big, rbig));
+    if (!rest.empty()) die_wgs = resident_per_die(ctx, rest);
+    if (!rest.empty()) TRY(resident_tables(ctx, rest, die_wgs, rb));
+    if (!resident_big.empty()) TRY(resident_tables(ctx, resident_big, 0, rbig));
     Plan PR;
     const bool all = (int)resident.size() == M.n;
     if (!all) TRY(plan_transient(ctx, resident, PR));
     for (int j = 0; j < sweeps; j++) {
-      HIPCHK(ctx, launch_cg_resident<T>(rb, M.shift, M.groups, false, ctx->tickets, ctx->resident, s));
+      if (die_wgs)
+        HIPCHK(ctx, launch_cg_resident_die<T>(rb, M.shift, M.groups, die_wgs, ctx->tickets, ctx->resident, s));
+      else
+        HIPCHK(ctx, launch_cg_resident<T>(rb, M.shift, M.groups, false, ctx->tickets, ctx->resident, s));
       if (rbig.n) HIPCHK(ctx, launch_cg_resident<T>(rbig, M.shift, M.groups, true, ctx->tickets, ctx->resident, s));
       TRY(launch_solve_ends<T>(ctx, all ? M : PR));
     }
@@ -1278,8 +1308,14 @@ int tick_impl(hobak_sched* S) {
     const unsigned w = M.status_host[i].spmv_work;
     work_bytes += (double)(unsigned)(w - I->work_seen) * spmv_bytes_of(I);
     if (!resident.empty()) res_launches = std::max(res_launches, w - I->work_seen);
+    // (an instance still solving that did not advance: its die had no compute units for it)
+    const bool stuck = die_wgs && w == I->work_seen && M.status_host[i].phase == PHASE_SOLVING &&
+                       std::find(resident.begin(), resident.end(), I) != resident.end();
     I->work_seen = w;
-    if (M.status_host[i].res_abort != I->abort_seen) {  // did not fit, or could not run at once
+    if (die_wgs && (stuck || M.status_host[i].res_abort != I->abort_seen)) {
+      ctx->dies = false;
+      I->abort_seen = M.status_host[i].res_abort;
+    } else if (M.status_host[i].res_abort != I->abort_seen) {  // did not fit, or could not run at once
       I->abort_seen = M.status_host[i].res_abort;
       I->res_pack = I->res_pack == kResBig ? 0 : I->res_pack / 2;  // more workgroups, each with fewer rows, while the device has that many
       if (I->res_pack > 0 && (I->h.nb[K_UPD] + I->res_pack - 1) / I->res_pack > ctx->cus) I->res_pack = 0;
@@ -1595,8 +1631,8 @@ int hobak_ctx_create(int device, size_t hbm_budget_bytes, hobak_ctx** out) {
   }
   bool ok = true;
   for (auto& e : ctx->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
-  ok = ok && hipMalloc((void**)&ctx->tickets, 2 * sizeof(int)) == hipSuccess &&
-       hipMemset(ctx->tickets, 0, 2 * sizeof(int)) == hipSuccess;
+  ok = ok && hipMalloc((void**)&ctx->tickets, (1 + kResDies) * sizeof(int)) == hipSuccess &&
+       hipMemset(ctx->tickets, 0, (1 + kResDies) * sizeof(int)) == hipSuccess;
   if (!ok || arena_ensure(ctx, 1 << 20) != HOBAK_OK || scratch_of_device(device, &ctx->scratch) != HOBAK_OK) {
     hobak_ctx_destroy(ctx);
     return HOBAK_E_HIP;

@@ -358,9 +358,14 @@ hipError_t launch_cg_spmv_p(const Batch& b, int shift, int pad, int stream, int 
 // Up to `iters` PCG iterations (from scalar set 0, which holds the current set again at the end) with
 // the matrices held on chip (resident.hip); b's prefix table counts each instance's workgroups, at
 // least 1 and at most nb[K_UPD], all of which must fit on the device at once; needs every update
-// workgroup to hold one run of rows (nb[K_UPD] below the cap).  tickets: two zero ints.
+// workgroup to hold one run of rows (nb[K_UPD] below the cap).  tickets: 1 + kResDies zero ints.
 template <typename T>
 hipError_t launch_cg_resident(const Batch& b, int shift, int groups, bool big, int* tickets, int iters, hipStream_t s);
+// The same for at most kResDies instances, each on the workgroups of one die (at most `wgs`, the most any takes),
+// which exchange through its L2.  An instance whose die gets no workgroups is left untouched.
+constexpr int kResDies = 8, kResDieWgs = 32;
+template <typename T>
+hipError_t launch_cg_resident_die(const Batch& b, int shift, int groups, int wgs, int* tickets, int iters, hipStream_t s);
 // Whether the resident PCG has a variant for this slice height, update layout and row count.
 bool resident_layout(int shift, int groups, int nb_upd);
 // The same of the form for more rows than the update workgroups cover in one run each, on `wgs` workgroups.

@@ -54,6 +54,13 @@
 // workgroups, 2.5 us over 206 with 539 to 1077 words (3.2 us with 8-byte loads and 8-byte words; 2.3 us
 // with eight copies of each word or a second level of sums, which was not worth their code).
 //
+// One die.  Up to eight instances of at most 32 workgroups each are placed on one die (XCD) each, where z and the
+// words go to the die's own L2 by ordinary stores: both waits then take about 1000 cycles less of an
+// iteration's 13,000 (10^3 FP64 step 783 -> 686 us, 17x9x23 BDF 2.37 -> 2.03 ms).  The loads are the same, past the
+// compute unit's cache (a load of workgroup scope may be served from that cache and never see the
+// word).  Workgroups learn their die from the hardware; an instance whose workgroups turn out to be on several, or
+// whose die gets none, is left untouched, and the context uses the general form from then on.
+//
 // Residency.  An instance's workgroups wait for each other, so all of them must run at once.
 // Workgroups take tickets, and tickets are dealt to instances in order, so at most the last instance
 // whose workgroups have begun is incomplete and every other one makes progress.  Before a workgroup
@@ -87,6 +94,9 @@ constexpr int kAbort = 1 << 30;
 constexpr u64 kJoinTicks = 20000000ull;       // 0.2 s of the 100 MHz wall clock
 constexpr unsigned kWaitTicks = 500000000u;   // 5 s; every peer is running, so this is never reached
 constexpr int kAgentScope = 16;               // cache policy of a buffer access: coherent over the device's L2s
+constexpr int kDieScope = 0;                  // of a store: to this die's L2, where loads of the other policy find it
+constexpr int kArrived = 1023;                // Ctl::res_arrive: workgroups here; from kDieBit on, their dies as bits
+constexpr int kDieBit = 16;
 
 // 64-slot steps of a wave held in registers: 162 or 144 registers of values and 5 or 8 of places, of the
 // 256 a wave may use at two waves per SIMD.
@@ -138,10 +148,11 @@ __device__ __forceinline__ void ld_vertex(Rsrc rs, unsigned off, float (&v)[3]) 
 
 // A published value: its low and high word, each next to the tag of its iteration (8-byte halves are
 // stored and loaded whole, so both tags match only where both words are this iteration's).
+template <int SC>
 __device__ __forceinline__ void publish_word(Rsrc rs, unsigned i, double v, unsigned tag) {
   const u64 b = (u64)__double_as_longlong(v);
   const u32x4 q = {(unsigned)b, tag, (unsigned)(b >> 32), tag};
-  __builtin_amdgcn_raw_buffer_store_b128(q, rs, 16u * i, 0, kAgentScope);
+  __builtin_amdgcn_raw_buffer_store_b128(q, rs, 16u * i, 0, SC);
 }
 
 // Spins until the K published values at byte offsets o[k] carry `tag`; gives up (false) after kWaitTicks.
@@ -228,14 +239,18 @@ __device__ __forceinline__ bool not_finite(double v) {
   return ((unsigned)((u64)__double_as_longlong(v) >> 52) & 0x7ffu) == 0x7ffu;
 }
 
+// The die (XCD, with an L2 of its own) this wave runs on: HW_REG_XCC_ID, bits 0 to 3.
+__device__ __forceinline__ int die_of_wave() { return __builtin_amdgcn_s_getreg(20 | 3 << 11) & 7; }
+
 __device__ __forceinline__ int al16(int x) { return (x + 15) & ~15; }
 
-template <typename T, int R, int H, bool BIG>
+template <typename T, int R, int H, bool BIG, bool ONE>
 __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __restrict__ I, int lb, int W,
                                                int iters, char* lds) {
   constexpr bool kF32 = sizeof(T) < sizeof(double);
   constexpr int NR = kReg<T>, ND = kAhead<BIG>;
   constexpr unsigned ts = sizeof(T);
+  constexpr int SC = ONE ? kDieScope : kAgentScope;  // the exchange between workgroups
   constexpr int sh = H == 64 ? 6 : H == 32 ? 5 : 4, L = 64 / H;
   constexpr int UC = BIG ? 1 : 4;             // 21 R-row chunks of a unit of rows
   constexpr int UR = 21 * R * UC;             // its rows: an update workgroup's, or one chunk's
@@ -418,9 +433,10 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   // announce this workgroup (or that its instance cannot run here)
   auto arr = (HOBAK_GLOBAL int*)&ctl->res_arrive;
   if (tid == 0) {
-    if (fits)
+    if (fits) {
+      if (ONE) __hip_atomic_fetch_or(arr, 1 << (kDieBit + die_of_wave()), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_fetch_add(arr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else
+    } else
       __hip_atomic_fetch_or(arr, kAbort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (fits) {
@@ -550,7 +566,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
     if (tid == 0) {
       const u64 t0 = wall_clock64();
       int v = __hip_atomic_load(arr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      while (!(v & kAbort) && v < W) {
+      while (!(v & kAbort) && (v & kArrived) < W) {
         if (wall_clock64() - t0 > kJoinTicks)
           __hip_atomic_compare_exchange_strong(arr, &v, v | kAbort, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT);
@@ -558,6 +574,9 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           __builtin_amdgcn_s_sleep(1);
         v = __hip_atomic_load(arr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
+      // (every workgroup's die is in before it is counted, so all of them see the same ones here)
+      if (ONE && !(v & kAbort) && __popc(v >> kDieBit) != 1)
+        v = __hip_atomic_fetch_or(arr, kAbort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) | kAbort;
       sh_flag = (v & kAbort) ? 0 : 1;
     }
     __syncthreads();
@@ -929,7 +948,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
             double s = 0.0;
             for (int i = lane; i < nsl; i += 64) s += ptsl[i];
             s = wave_sum(s);
-            if (lane == 0) publish_word(rs_w, (tag & 1u) * npt + (unsigned)lb, s, tag);
+            if (lane == 0) publish_word<SC>(rs_w, (tag & 1u) * npt + (unsigned)lb, s, tag);
           }
         } else if (split) {
           if (tid < nsl && (pubs[tid] >> 12) != 0) {
@@ -937,7 +956,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
             double v = n <= 4 ? ptsl[tid] : 0.0;
 #pragma unroll
             for (int w = 1; w < 4; w++) v += w < n && n <= 4 ? ptsl[tid + w] : 0.0;
-            publish_word(rs_w, (tag & 1u) * npt + (unsigned)(e & 0xfff), v, tag);
+            publish_word<SC>(rs_w, (tag & 1u) * npt + (unsigned)(e & 0xfff), v, tag);
           }
         } else if (tid < max(nq, 1)) {
           double s = 0.0;
@@ -951,7 +970,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           if (solo)
             lp[tid] = s;
           else
-            publish_word(rs_w, (tag & 1u) * npt + (unsigned)(nq > 0 ? q0 + tid : qe), s, tag);
+            publish_word<SC>(rs_w, (tag & 1u) * npt + (unsigned)(nq > 0 ? q0 + tid : qe), s, tag);
         }
         if (solo) __syncthreads();
         load(gofs, gofs_m, left0, urow);
@@ -1022,7 +1041,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           }
 #pragma unroll
           for (int q = 0; q < R; q++) {
-            buf_st<kAgentScope>(rs_z, go + 63 * q * ts, zq[q]);
+            buf_st<SC>(rs_z, go + 63 * q * ts, zq[q]);
             if (21 * q < left) {
               rr2 = fma((double)rq[q], (double)rq[q], rr2);
               rz = fma((double)rq[q], (double)zq[q], rz);
@@ -1063,7 +1082,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
             double s = 0.0;
             for (int i = lane; i < nch; i += 64) s += uw[wave * nch + i];
             s = wave_sum(s);
-            if (lane == 0) publish_word(rs_w, 2u * npt + (5u * (tag & 1u) + (unsigned)wave) * (unsigned)NX + (unsigned)lb, s, tag);
+            if (lane == 0) publish_word<SC>(rs_w, 2u * npt + (5u * (tag & 1u) + (unsigned)wave) * (unsigned)NX + (unsigned)lb, s, tag);
             if (it == iters - 1) {  // the next launch adds all NB of them
               const auto J = rec();
               auto dst = gbl(wave == 0 ? J->part_rr : wave == 1 ? J->part_rz : J->part_upd_g + (size_t)(wave - 2) * NB);
@@ -1079,7 +1098,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           if (solo)
             lp[nq + kind * nu + ku] = s;
           else
-            publish_word(rs_w, 2u * npt + (5u * (tag & 1u) + (unsigned)kind) * (unsigned)NU + (unsigned)(u0 + ku),
+            publish_word<SC>(rs_w, 2u * npt + (5u * (tag & 1u) + (unsigned)kind) * (unsigned)NU + (unsigned)(u0 + ku),
                          s, tag);
           if (it == iters - 1) {  // the next launch finishes this iteration from these
             const auto J = rec();
@@ -1147,12 +1166,38 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 
   int lb, W;
   const HOBAK_GLOBAL InstDev* I =
       uptr((const InstDev*)seg_find(b, __builtin_amdgcn_readfirstlane(sh_ticket), lb, W));
-  resident_solve<T, R, H, BIG>(I, uniform_i(lb), uniform_i(W), iters, lds);
+  resident_solve<T, R, H, BIG, false>(I, uniform_i(lb), uniform_i(W), iters, lds);
   if (threadIdx.x == 0 &&
       __hip_atomic_fetch_add(tickets + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == b.total - 1) {
     __hip_atomic_store(tickets, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(tickets + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+}
+
+// The same for up to eight instances, instance i on die i alone: the grid holds as many workgroups for each die as
+// the largest instance takes, and those past an instance's, or of a die without one, leave at once.
+// tickets: [0] workgroups done, [1 + i] instance i's next ticket; all zero between launches.
+template <typename T, int R, int H>
+__global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void cg_resident_die_kernel(
+    Batch b, int* tickets, int iters) {
+  extern __shared__ __align__(16) char lds[];
+  __shared__ int sh_ticket;
+  const int i = __builtin_amdgcn_readfirstlane(die_of_wave());
+  if (i < b.n) {
+    const int W = uniform_i(b.n == 1 ? b.total : gbl(b.boff)[i + 1] - gbl(b.boff)[i]);
+    if (threadIdx.x == 0)
+      sh_ticket = __hip_atomic_fetch_add(tickets + 1 + i, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int lb = uniform_i(sh_ticket);
+    if (lb < W) {
+      const HOBAK_GLOBAL InstDev* I = uptr(b.n == 1 ? b.one : gbl(b.inst)[i]);
+      resident_solve<T, R, H, false, true>(I, lb, W, iters, lds);
+    }
+  }
+  if (threadIdx.x == 0 &&
+      __hip_atomic_fetch_add(tickets, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1)
+    for (int k = 0; k <= kResDies; k++)
+      __hip_atomic_store(tickets + k, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <typename T, int R, int H, bool BIG>
@@ -1164,6 +1209,25 @@ hipError_t resident_rh(const Batch& b, int* tickets, int iters, hipStream_t s) {
                      iters);
   return hipGetLastError();
 }
+template <typename T, int R, int H>
+hipError_t resident_die(const Batch& b, int wgs, int* tickets, int iters, hipStream_t s) {
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&cg_resident_die_kernel<T, R, H>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, kResLds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((cg_resident_die_kernel<T, R, H>), dim3(kResDies * wgs), dim3(kResThreads), kResLds, s, b, tickets,
+                     iters);
+  return hipGetLastError();
+}
+template <typename T, int R>
+hipError_t resident_die_r(const Batch& b, int shift, int wgs, int* tickets, int iters, hipStream_t s) {
+  switch (shift) {
+    case 4: return resident_die<T, R, 16>(b, wgs, tickets, iters, s);
+    case 5: return resident_die<T, R, 32>(b, wgs, tickets, iters, s);
+    case 6: return resident_die<T, R, 64>(b, wgs, tickets, iters, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 template <typename T, int R, bool BIG>
 hipError_t resident_r(const Batch& b, int shift, int* tickets, int iters, hipStream_t s) {
   switch (shift) {
@@ -1200,6 +1264,17 @@ hipError_t launch_cg_resident(const Batch& b, int shift, int groups, bool big, i
     default: return hipErrorInvalidValue;
   }
 }
+template <typename T>
+hipError_t launch_cg_resident_die(const Batch& b, int shift, int groups, int wgs, int* tickets, int iters, hipStream_t s) {
+  if (b.n < 1 || b.n > kResDies || wgs < 1) return hipErrorInvalidValue;
+  switch (groups) {
+    case 2: return resident_die_r<T, 2>(b, shift, wgs, tickets, iters, s);
+    case 4: return resident_die_r<T, 4>(b, shift, wgs, tickets, iters, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+template hipError_t launch_cg_resident_die<double>(const Batch&, int, int, int, int*, int, hipStream_t);
+template hipError_t launch_cg_resident_die<float>(const Batch&, int, int, int, int*, int, hipStream_t);
 template hipError_t launch_cg_resident<double>(const Batch&, int, int, bool, int*, int, hipStream_t);
 template hipError_t launch_cg_resident<float>(const Batch&, int, int, bool, int*, int, hipStream_t);
 

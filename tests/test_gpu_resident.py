@@ -149,3 +149,32 @@ def test_more_rows_than_the_update_workgroups_cover(precision, pin, tuning):
         x, y = big.rest.ravel() + got[-1][0], big.rest.ravel() + want[0][0]
         assert np.linalg.norm(x - y) <= 1e-9 * np.linalg.norm(y), n
         assert gs[0][-1][0] == ws[0][0][0] and abs(gs[0][-1][1][0] - ws[0][0][1][0]) <= 1, (n, gs, ws)
+
+
+@pytest.mark.parametrize("precision", [F64, F32])
+def test_one_die_and_all_of_them_in_turn(precision):
+    """Up to eight instances run on one die each, more of them over the device; the same instances in turn in both,
+    with solves that end in one launch and in several, at the row counts about one and two update workgroups'
+    rows a workgroup (5,376 and 10,752 rows)."""
+    dims = [(6, 5, 4), (16, 16, 17), (17, 17, 15), (21, 21, 20), (21, 21, 21), (3, 30, 5), (8, 8, 8), (9, 8, 7)]
+    scs = [_lattice(d, seed=k) for k, d in enumerate(dims)] + [_lattice((5, 5, 5), seed=20 + k) for k in range(3)]
+
+    def run(resident):
+        ctx = lib.Context(0, precision="fp64" if precision == F64 else "fp32", workload="batch")
+        ctx.set_tuning(resident=resident)
+        insts = [lib.Instance(ctx, sc, precision=precision) for sc in scs]
+        its = []
+        for group in (insts[:1], insts[:8], insts, insts[3:4], insts[4:5], insts[1:8], insts):
+            its += [s["pcg_iters"] for s in lib.step_batch(ctx, group, True)]
+        out = [i.state() for i in insts]
+        for i in insts:
+            i.close()
+        ctx.close()
+        return out, its
+
+    want, wi = run(0)
+    for n in (512, 10):
+        got, gi = run(n)
+        assert gi == wi, n
+        for i, ((u, v), (uw, vw)) in enumerate(zip(got, want)):
+            assert np.array_equal(u, uw) and np.array_equal(v, vw), (n, i)
