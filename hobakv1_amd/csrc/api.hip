@@ -450,7 +450,7 @@ struct hobak_inst {
   // perm[p]; iperm is the inverse.  Empty: the caller's numbering.  ocol_idx / orow_ptr are the
   // block pattern in the caller's numbering and oslot the slot of each of its blocks.
   std::vector<int> perm, iperm, orow_ptr, ocol_idx, oslot;
-  int* iperm_dev = nullptr;  // iperm on the device, where states cross the staging (see stage_get)
+  int* iperm_dev = nullptr;  // iperm on the device, which relabels states on their way in and out
   std::vector<std::pair<void*, size_t>> allocs;
   size_t bytes = 0;
   InstDev h{};              // host mirror of the device record
@@ -586,7 +586,9 @@ void to_caller_order(const hobak_inst* I, double* v) {
 // A state crosses as one kernel that reads or writes the pinned memory over the bus, in either direction, and
 // relabels on the way: 14 us in and 27 us out for a mean instance of a 128-instance batch (4 to 24 cells an axis,
 // relabelled) and 11 and 20 us for 125 vertices, where two pageable copies and a host-side relabelling took 39 and
-// 38, and 26 and 47.  Larger states gain nothing: there the host's own copy into the staging is what takes time.
+// 38, and 26 and 47.  Larger states gain nothing from the staging: there the host's own copy into it is what takes
+// time.  They are copied whole and relabelled by the same kernel on the device: 3.66 and 16.1 ms for a 68,921- and a
+// 303,242-vertex FP32 step with its state in and out, which relabelled on the host took 3.9 and 19.0 ms.
 constexpr size_t kStageBytes = 4 << 20, kStageState = 1 << 20;
 char* stage_get(hobak_ctx* ctx, size_t bytes) {
   if (bytes > kStageState) return nullptr;
@@ -1911,8 +1913,8 @@ int hobak_inst_create(hobak_ctx* ctx, const double* rest_xyz, int32_t nv, const 
     I->dev = (InstDev*)rec;
     h.ctl = ctl_of(I->dev);
   }
-  const bool staged = !I->iperm.empty() && 2 * sizeof(double) * (size_t)I->dofs <= kStageState;
-  if (staged) ALLOC(I->iperm_dev, nv);
+  const bool relabelled = !I->iperm.empty();
+  if (relabelled) ALLOC(I->iperm_dev, nv);
 #undef ALLOC
 #undef ALLOCT
   h.rest = rest;
@@ -1956,7 +1958,7 @@ int hobak_inst_create(hobak_ctx* ctx, const double* rest_xyz, int32_t nv, const 
       (rc = upload(I, vol, vol_h.data(), vol_h.size())) ||
       (rc = upload(I, t4d, t4.data(), t4.size())) ||
       (rc = upload(I, slice_off, P.slice_off.data(), P.slice_off.size())) ||
-      (staged && (rc = upload(I, I->iperm_dev, I->iperm.data(), (size_t)nv))) ||
+      (relabelled && (rc = upload(I, I->iperm_dev, I->iperm.data(), (size_t)nv))) ||
       (rc = upload(I, row_len, P.row_len.data(), P.row_len.size())) ||
       (rc = upload(I, col, P.col.data(), P.col.size())) ||
       (rc = upload(I, slot_row, P.slot_row.data(), P.slot_row.size())) ||
@@ -2163,9 +2165,15 @@ int hobak_inst_set_state(hobak_inst* I, const double* u, const double* v) {
     HIPCHK(I->ctx, launch_state_in(u ? stage : nullptr, v ? stage + I->dofs : nullptr, I->h.u, I->h.v, I->iperm_dev,
                                    I->nv, I->ctx->stream));
   } else {
-    std::vector<double> ub, vb;
-    if (u) TRY(upload(I, I->h.u, to_device_order(I, u, ub), (size_t)I->dofs));
-    if (v) TRY(upload(I, I->h.v, to_device_order(I, v, vb), (size_t)I->dofs));
+    // relabelled states pass through tmp64, which nothing holds between calls
+    for (int k = 0; k < 2; k++) {
+      const double* src = k ? v : u;
+      double* dst = k ? I->h.v : I->h.u;
+      if (!src) continue;
+      TRY(upload(I, I->iperm_dev ? I->h.tmp64 : dst, src, (size_t)I->dofs));
+      if (I->iperm_dev)
+        HIPCHK(I->ctx, launch_state_in(I->h.tmp64, nullptr, dst, nullptr, I->iperm_dev, I->nv, I->ctx->stream));
+    }
     HIPCHK(I->ctx, hipStreamSynchronize(I->ctx->stream));
   }
   for (auto& p : I->pred) p = -1;
@@ -2185,11 +2193,14 @@ int hobak_inst_get_state(hobak_inst* I, double* u, double* v) {
     I->ctx->stage_off = 0;
     return HOBAK_OK;
   }
-  if (u) HIPCHK(I->ctx, hipMemcpyAsync(u, I->h.u, sizeof(double) * I->dofs, hipMemcpyDeviceToHost, s));
-  if (v) HIPCHK(I->ctx, hipMemcpyAsync(v, I->h.v, sizeof(double) * I->dofs, hipMemcpyDeviceToHost, s));
+  for (int k = 0; k < 2; k++) {
+    double* dst = k ? v : u;
+    double* src = k ? I->h.v : I->h.u;
+    if (!dst) continue;
+    if (I->iperm_dev) HIPCHK(I->ctx, launch_state_out(src, nullptr, I->h.tmp64, nullptr, I->iperm_dev, I->nv, s));
+    HIPCHK(I->ctx, hipMemcpyAsync(dst, I->iperm_dev ? I->h.tmp64 : src, bytes, hipMemcpyDeviceToHost, s));
+  }
   HIPCHK(I->ctx, hipStreamSynchronize(s));
-  to_caller_order(I, u);
-  to_caller_order(I, v);
   return HOBAK_OK;
 }
 
