@@ -116,19 +116,25 @@ __device__ __forceinline__ bool nonfinite(double v) { return !(v == v) || v > DB
 // in a fixed lane order to the same value in every lane, then z += (P_I^T A P_I)^-1 g at the free
 // rows.  pn[q] != 0: row q is pinned or past the end.  Every lane of the wave takes part.
 template <typename T, int R>
-__device__ __forceinline__ void agg_correct(const HOBAK_GLOBAL T* ainv, int ch, int c, const T (&rq)[R],
-                                            const unsigned char (&pn)[R], T (&zq)[R]) {
+__device__ __forceinline__ void agg_apply(const T (&m)[3], int c, const T (&rq)[R], const unsigned char (&pn)[R],
+                                          T (&zq)[R]) {
   T s = T(0);
 #pragma unroll
   for (int q = 0; q < R; q++) s += pn[q] ? T(0) : rq[q];
   const T g0 = wave_sum(c == 0 ? s : T(0));
   const T g1 = wave_sum(c == 1 ? s : T(0));
   const T g2 = wave_sum(c == 2 ? s : T(0));
-  const HOBAK_GLOBAL T* m = ainv + 9 * (size_t)ch + 3 * c;
   const T e = fma(m[2], g2, fma(m[1], g1, m[0] * g0));
 #pragma unroll
   for (int q = 0; q < R; q++)
     if (!pn[q]) zq[q] += e;
+}
+template <typename T, int R>
+__device__ __forceinline__ void agg_correct(const HOBAK_GLOBAL T* ainv, int ch, int c, const T (&rq)[R],
+                                            const unsigned char (&pn)[R], T (&zq)[R]) {
+  const HOBAK_GLOBAL T* p = ainv + 9 * (size_t)ch + 3 * c;
+  const T m[3] = {p[0], p[1], p[2]};
+  agg_apply<T, R>(m, c, rq, pn, zq);
 }
 
 }  // namespace hobak

@@ -317,7 +317,11 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   }
   const bool solo = !BIG && W == 1;
   // this workgroup's units, rows, SpMV workgroups and slices
-  const int u0 = uniform_i(lb * NU / W), u1 = uniform_i((lb + 1) * NU / W);  // (NU W < 2^31: nv < 2^25)
+  // (as many units each, the last fewer: a 336-row workgroup then begins on a 16-row slice and has at most 24 of them,
+  // three a wave; dealt evenly, most began half a slice off and the 25th slice of some, with the columns
+  // past 1024 that it couples to, set the pace of all: 40^3 FP64 step 5.07 -> 4.85 ms.  BIG: NU W < 2^31, nv < 2^25)
+  const int per = (NU + W - 1) / W;
+  const int u0 = uniform_i(BIG ? lb * NU / W : min(lb * per, NU)), u1 = uniform_i(BIG ? (lb + 1) * NU / W : min((lb + 1) * per, NU));
   const int nu = u1 - u0, nch = UC * nu;
   const int ua = u0 * UR, ub = min(u1 * UR, nrows), nown = ub - ua;
   const int nslices = (nrows + H - 1) >> sh;
@@ -328,7 +332,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   // A workgroup in whose rows no SpMV workgroup (split: no slice) begins publishes a zero in its place, so
   // that nobody passes the wait on p.t, and overwrites z, before every workgroup has read it: np words in
   // all, this one's at qe
-  const int ra = tid * NU / W * UR, rb = min((tid + 1) * NU / W * UR, nrows);
+  const int ra = min(tid * per * UR, nrows), rb = min((tid + 1) * per * UR, nrows);
   const bool none = tid < W && (split ? first_s(ra) == first_s(rb) : first_q(ra) == first_q(rb));
   const int np = BIG ? W : NQ + __syncthreads_count(none), qe = BIG ? 0 : NQ + __syncthreads_count(none && tid < lb);
   const int sa = ua >> sh, so = first_s(ua);
@@ -336,7 +340,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   const int nown_s = sb - so;  // the slices that begin in its rows
   if (!BIG && !split && nq > 0) sb = max(sb, min(4 * q1, nslices));
   if (tid < 256) {  // bits j: slice 4 tid + j is published by another workgroup than slice 4 tid
-    auto owner = [&](int s) { return ((s * H / UR + 1) * W - 1) / NU; };
+    auto owner = [&](int s) { return s * H / (UR * per); };
     unsigned m = 0;
     if (split && tid < NQ)
 #pragma unroll
@@ -882,8 +886,18 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
         // the first chunk's r, x and preconditioner, which the update needs: they arrive while p.t is awaited (past
         // the wave's chunks: rows that are not used, or past the end)
         T rv0[R], xv[R], m0[R], m1[R], m2[R];
+        // this component's row of the chunk's aggregate inverse; with four row groups it costs more registers than the
+        // latency is worth (24 served sessions 16.8 instead of 16.6 ms; 40^3 FP32 with two: 3.39 instead of 3.56)
+        constexpr bool kInverse = kF32 && R == 2;
+        T ai[3] = {};
         unsigned char pn[R];
-        auto load = [&](unsigned go, unsigned gm, int left, int row) {
+        auto load = [&](unsigned go, unsigned gm, int left, int row, int ch) {
+          if constexpr (kInverse)
+            if (local && ch * 21 * R < nrows) {
+              const unsigned o = ts * (unsigned)(9 * ch + 3 * c);
+#pragma unroll
+              for (int k = 0; k < 3; k++) ai[k] = ld_off(ainv, o + (unsigned)k * ts);
+            }
 #pragma unroll
           for (int q = 0; q < R; q++) {
             pn[q] = 1;
@@ -973,7 +987,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
             publish_word<SC>(rs_w, (tag & 1u) * npt + (unsigned)(nq > 0 ? q0 + tid : qe), s, tag);
         }
         if (solo) __syncthreads();
-        load(gofs, gofs_m, left0, urow);
+        load(gofs, gofs_m, left0, urow, UC * u0 + wave);
         if (wave < 4) {
           double v[1] = {0.0};
           if (solo) {
@@ -1036,8 +1050,12 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
             zq[q] = precond == 0 ? m0[q] * rv : fma(m2[q], r2, fma(m0[q], r0, m1[q] * r1));
           }
           if constexpr (kF32) {
-            if (local) agg_correct<T, R>(ainv, UC * u0 + cl < (nrows + 21 * R - 1) / (21 * R) ? UC * u0 + cl : 0,
-                                         c, rq, pn, zq);
+            if (local) {
+              if constexpr (kInverse)
+                agg_apply<T, R>(ai, c, rq, pn, zq);
+              else
+                agg_correct<T, R>(ainv, UC * u0 + cl < (nrows + 21 * R - 1) / (21 * R) ? UC * u0 + cl : 0, c, rq, pn, zq);
+            }
           }
 #pragma unroll
           for (int q = 0; q < R; q++) {
@@ -1071,7 +1089,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           if (cl + kResWaves < nch) {
             constexpr int step = kResWaves * 21 * R;
             load(go + 3u * ts * step, gofs_m + (precond == 0 ? 3u : 9u) * ts * (unsigned)(ch + step), left - step,
-                 urow + ch + step);
+                 urow + ch + step, UC * u0 + cl + kResWaves);
           }
         }
         // z is complete before the sums that announce it are published
