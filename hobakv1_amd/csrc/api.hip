@@ -1634,7 +1634,7 @@ int hobak_ctx_create(int device, size_t hbm_budget_bytes, hobak_ctx** out) {
   bool ok = true;
   for (auto& e : ctx->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
   ok = ok && hipMalloc((void**)&ctx->tickets, (1 + kResDies) * sizeof(int)) == hipSuccess &&
-       hipMemset(ctx->tickets, 0, (1 + kResDies) * sizeof(int)) == hipSuccess;
+       hipMemsetAsync(ctx->tickets, 0, (1 + kResDies) * sizeof(int), ctx->stream) == hipSuccess;
   if (!ok || arena_ensure(ctx, 1 << 20) != HOBAK_OK || scratch_of_device(device, &ctx->scratch) != HOBAK_OK) {
     hobak_ctx_destroy(ctx);
     return HOBAK_E_HIP;
@@ -1905,13 +1905,15 @@ int hobak_inst_create(hobak_ctx* ctx, const double* rest_xyz, int32_t nv, const 
     ALLOC(h.part_row_c, 6 * (size_t)h.nb[K_ROW]);
     ALLOC(h.part_upd_g, 3 * (size_t)h.nb[K_UPD]);
   }
-  if (I->res_pack > 0) ALLOC(h.xwords, resident_words(h.nb[K_SPMV], h.nb[K_UPD]));
   if (I->spatial) ALLOCT(h.agg_inv, 9 * (size_t)((nv + 21 * I->groups - 1) / (21 * I->groups)));
   {
-    char* rec = nullptr;  // the record and, kCtlOffset bytes after it, the control block
-    if ((rc = dalloc(I, &rec, kCtlOffset + sizeof(Ctl), 1)) != HOBAK_OK) return bail(rc);
+    char* rec = nullptr;  // the record, kCtlOffset bytes after it the control block, and the published words
+    const size_t words_at = kCtlOffset + (sizeof(Ctl) + 255) / 256 * 256;
+    const size_t words = I->res_pack > 0 ? resident_words(h.nb[K_SPMV], h.nb[K_UPD]) : 0;
+    if ((rc = dalloc(I, &rec, words_at + 8 * words, 1)) != HOBAK_OK) return bail(rc);
     I->dev = (InstDev*)rec;
     h.ctl = ctl_of(I->dev);
+    h.xwords = words ? (unsigned long long*)(rec + words_at) : nullptr;
   }
   const bool relabelled = !I->iperm.empty();
   if (relabelled) ALLOC(I->iperm_dev, nv);

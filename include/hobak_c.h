@@ -302,7 +302,9 @@ int hobak_kernel_stats(hobak_inst* inst, double* spmv_avg_ms, int64_t* spmv_coun
  *                          form, which holds an instance's matrix in registers and LDS for the whole
  *                          launch; instances that do not fit the device that way run the
  *                          two-kernel form, as does everything while GRID_CAP is set.  Results do not
- *                          depend on it.  Default 512; 0 never */
+ *                          depend on it, but for FP32_REFINE instances of more rows than the update
+ *                          workgroups cover in one run each (86,016 by default), whose sums of products
+ *                          round in another order than the two-kernel form's.  Default 2048; 0 never */
 #define HOBAK_TUNE_SLICE_ROWS 0
 #define HOBAK_TUNE_POLL_CHUNK 2
 #define HOBAK_TUNE_MAX_CHUNKS 3
