@@ -1225,7 +1225,11 @@ int tick_impl(hobak_sched* S) {
       resident.push_back(r.I);
       if (r.I->res_pack == kResBig) resident_big.push_back(r.I);
     }
-  const bool sample_first = !resident.empty() && sampled_group();
+  // (a step of resident instances whose samples would all fall inside its one launch has its second
+  // iteration sampled instead)
+  const bool brief = !resident.empty() && S->ephemeral && every > 0 && S->samples.empty() && !sampled_group();
+  const bool sample_first = !resident.empty() && (brief || sampled_group());
+  const int group_iters = brief ? 2 : k;
   int sweeps = 1, die_wgs = 0;
   for (auto& r : S->active) {
     if (r.stage != 1) continue;
@@ -1248,19 +1252,19 @@ int tick_impl(hobak_sched* S) {
     const bool compact = nsolving < M.n && solving_wgs * 100 <= (long)ctx->compact_pct * M.b[K_SPMV].total;
     Plan PG;
     if (compact) TRY(plan_transient(ctx, solving, PG));
-    if (graphs && !compact && (!M.chunk_exec[st] || M.chunk_k[st] != k)) {
+    if (graphs && !compact && !brief && (!M.chunk_exec[st] || M.chunk_k[st] != k)) {
       if (M.chunk_exec[st]) (void)hipGraphExecDestroy(M.chunk_exec[st]);
       M.chunk_exec[st] = nullptr;
       TRY(capture(ctx, &M.chunk_exec[st], [&]() { return launch_chunk<T>(ctx, M, k, st, nullptr, 0); }));
       M.chunk_k[st] = k;
     }
     for (int j = 0; j < m; j++) {
-      if (graphs && !compact && !sampled_group()) {  // every unsampled group replays the graph
+      if (graphs && !compact && !brief && !sampled_group()) {  // every unsampled group replays the graph
         HIPCHK(ctx, hipGraphLaunch(M.chunk_exec[st], s));
         if (S->sampling) S->sample_it += k;
         S->stat[9] += 1;
       } else {
-        TRY(launch_chunk<T>(ctx, compact ? PG : M, k, st, S->sampling ? S : nullptr, every));
+        TRY(launch_chunk<T>(ctx, compact ? PG : M, group_iters, st, S->sampling ? S : nullptr, brief ? 2 : every));
         S->stat[10] += 1;
       }
     }
@@ -1324,9 +1328,9 @@ int tick_impl(hobak_sched* S) {
     }
   }
   S->stat[8] += work_bytes;
-  const long long launches = std::max<long long>(nsolving ? (long long)m * k : 0, res_launches);
+  const long long launches = std::max<long long>(nsolving ? (long long)m * group_iters : 0, res_launches);
   if (ran) S->stat[7] += (double)launches;
-  if (S->sampling) S->sample_it += std::max(0, (int)res_launches - (sample_first ? k : 0));
+  if (S->sampling) S->sample_it += std::max(0, (int)res_launches - (sample_first ? group_iters : 0));
   const double now = clock_s(S);
   if (pro) {
     if (pro_split) {
