@@ -6,8 +6,8 @@
 // few hundred vertices, where nothing but the launches and their dependent loads is left.  The chip's
 // registers and LDS hold 168 MB, so here an instance's rows are dealt out to W workgroups of one
 // compute unit each, every workgroup loads its slots once, and an iteration moves only the
-// vector entries its rows couple to.  Measured per iteration: 10.6 us for the 40^3 lattice (FP64, 206
-// workgroups; FP32 10.1), 6.0 us for 10^3 (8 workgroups), 4.0 us for 4^3 (one).
+// vector entries its rows couple to.  Measured per iteration: 10.4 us for the 40^3 lattice (FP64, 206
+// workgroups; FP32 9.4), 5.2 us for 10^3 (8 workgroups of one die), 4.0 us for 4^3 (one).
 //
 // Arithmetic (all but BIG).  Every sum runs in the order of the two-kernel iteration: a row's blocks by the lane that
 // handles them there, p.t by SpMV workgroup (four slices), r.r and r.z by update workgroup (four
@@ -16,8 +16,9 @@
 // one to the other at any even iteration.
 //
 // Work split.  Workgroup w owns a contiguous range of update workgroups' rows [ua, ub) and computes the
-// slices that cover it, plus the rest of the SpMV workgroups (of four slices) that begin in it; the
-// few rows past the range are computed twice, which costs less than handing t across workgroups.
+// slices that cover it, plus, past kSplitMax and with 16-row slices, the rest of the SpMV workgroups (of four
+// slices) that begin in it; the few rows past the range are computed twice, which costs less than handing t
+// across workgroups.
 //   registers  the first kReg 64-slot steps of each wave (9 values and a 16-bit place per slot);
 //   LDS        the vector entries the slots couple to (FP64: p, which every workgroup keeps up to date
 //              itself from z; FP32: z), t, and as many further steps as fit, dealt so that the
@@ -26,7 +27,7 @@
 // BIG is the reduced-precision form for more rows than the update workgroups cover in one run each (86,016
 // with two row groups), where the two-kernel form is bound by reading 160 MB of matrix and 30 MB of vectors an
 // iteration: 46 us for 303,242 vertices.  It runs on every compute unit, which hold about half the
-// matrix and stream the rest: 30 us, of which 13 for the streamed half (9 TB/s) and 5 for the update's
+// matrix and stream the rest: 29 us, of which 13 for the product (90 MB streamed, 7 TB/s) and 5 for the update's
 // vectors.  Its rows are dealt in single chunks of 21 R, and each workgroup publishes one word per sum; the
 // sums are so added in another order than the two-kernel form's (the same in every launch).  They
 // are FP64 sums behind FP32 step lengths, which that has not changed in any run.  FP64 solves keep the
