@@ -77,6 +77,7 @@ struct hobak_ctx {
   int cus = 0;                         // compute units of the device
   bool dies = true;                    // small batches of the resident PCG run on one die each
   int* tickets = nullptr;              // resident PCG launches of this context's stream
+  int64_t res_stat[HOBAK_RESIDENT_STATS] = {};  // see hobak_ctx_resident_stats
   hipStream_t stream = nullptr;
   size_t budget = 0;
   size_t in_use = 0;
@@ -471,6 +472,7 @@ struct hobak_inst {
   // Ctl::res_abort held at the last status poll, refinement sweeps of the last solve
   int res_pack = 0;
   int abort_seen = 0;
+  unsigned runs_seen = 0;  // likewise Ctl::res_runs
   int sweeps_seen = 0;
 };
 
@@ -1318,6 +1320,11 @@ int tick_impl(hobak_sched* S) {
     const bool stuck = die_wgs && w == I->work_seen && M.status_host[i].phase == PHASE_SOLVING &&
                        std::find(resident.begin(), resident.end(), I) != resident.end();
     I->work_seen = w;
+    const unsigned runs = M.status_host[i].res_runs - I->runs_seen;
+    I->runs_seen += runs;
+    ctx->res_stat[I->res_pack == kResBig ? HOBAK_RESIDENT_BIG : die_wgs ? HOBAK_RESIDENT_DIE : HOBAK_RESIDENT_DEVICE] +=
+        runs;
+    ctx->res_stat[HOBAK_RESIDENT_ABORTED] += M.status_host[i].res_abort - I->abort_seen;
     if (die_wgs && (stuck || M.status_host[i].res_abort != I->abort_seen)) {
       ctx->dies = false;
       I->abort_seen = M.status_host[i].res_abort;
@@ -1670,6 +1677,12 @@ void hobak_ctx_destroy(hobak_ctx* ctx) {
 }
 
 const char* hobak_last_error(hobak_ctx* ctx) { return ctx ? ctx->err.c_str() : "no context"; }
+
+int hobak_ctx_resident_stats(hobak_ctx* ctx, int64_t* out) {
+  if (!ctx || !out) return HOBAK_E_INVALID;
+  std::copy(ctx->res_stat, ctx->res_stat + HOBAK_RESIDENT_STATS, out);
+  return HOBAK_OK;
+}
 
 size_t hobak_ctx_bytes_in_use(hobak_ctx* ctx) { return ctx ? ctx->in_use : 0; }
 

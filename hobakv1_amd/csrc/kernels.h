@@ -115,10 +115,10 @@ struct Ctl {
   double ac_inv[3];  // coarse correction: 1 / (P^T A P), diagonal (see InstDev::coarse)
   unsigned spmv_work;  // SpMV launches that streamed this instance's matrix (wraps; a count)
   // the resident PCG (resident.hip): tag of the last published partial sums, the meeting point of an
-  // instance's workgroups, and the launches that left the instance untouched
+  // instance's workgroups, and the launches that left the instance untouched and that solved it
   unsigned res_epoch;
   int res_arrive, res_exit, res_abort;
-  int pad4;
+  unsigned res_runs;
 };
 
 // What the host reads back after a group of PCG iterations, one per instance of a batch.
@@ -135,6 +135,7 @@ struct InstStatus {
   double maxR;      // |S b|^2
   unsigned spmv_work;  // Ctl::spmv_work
   int res_abort;       // Ctl::res_abort
+  unsigned res_runs;   // Ctl::res_runs
 };
 
 // Read-only per-instance record.  Pointers typed void* hold the solve's real type T.

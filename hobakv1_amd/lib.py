@@ -120,6 +120,7 @@ SIGNATURES = {
     "hobak_kernel_stats": (ctypes.c_int, [_vp, _dp, ctypes.POINTER(ctypes.c_int64), _dp]),
     "hobak_copy_probe": (ctypes.c_int, [_vp, ctypes.c_size_t, ctypes.c_int32, _dp]),
     "hobak_ctx_set_tuning": (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.c_int32]),
+    "hobak_ctx_resident_stats": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int64)]),
     "hobak_sched_create": (ctypes.c_int, [_vp, ctypes.POINTER(_vp)]),
     "hobak_sched_destroy": (None, [_vp]),
     "hobak_sched_submit": (ctypes.c_int, [_vp, _vp, ctypes.c_uint64]),
@@ -260,6 +261,12 @@ class Context:
                          (TUNE_COARSE, coarse), (TUNE_AGG, agg), (TUNE_RESIDENT, resident)):
             if val is not None:
                 self.check(self.lib.hobak_ctx_set_tuning(self.h, key, int(val)), "set_tuning")
+
+    def resident_stats(self):
+        """Instance launches of the resident PCG by form, and those that left an instance untouched."""
+        out = (ctypes.c_int64 * 4)()
+        self.check(self.lib.hobak_ctx_resident_stats(self.h, out), "resident_stats")
+        return dict(zip(("device", "die", "big", "aborted"), out))
 
     def copy_probe(self, nbytes, reps=20):
         ms = ctypes.c_double(0)

@@ -322,6 +322,17 @@ int hobak_kernel_stats(hobak_inst* inst, double* spmv_avg_ms, int64_t* spmv_coun
 #define HOBAK_TUNE_RESIDENT 15
 int hobak_ctx_set_tuning(hobak_ctx* ctx, int32_t key, int32_t value);
 
+/* Counters since the context was created, HOBAK_RESIDENT_STATS int64: for each instance of each launch
+ * of the resident PCG (HOBAK_TUNE_RESIDENT), which form advanced it - over the whole device, on one die,
+ * or on every compute unit (FP32_REFINE instances of more rows than the update workgroups cover) - or
+ * that the launch left it untouched, for the two-kernel form to solve. */
+#define HOBAK_RESIDENT_DEVICE 0
+#define HOBAK_RESIDENT_DIE 1
+#define HOBAK_RESIDENT_BIG 2
+#define HOBAK_RESIDENT_ABORTED 3
+#define HOBAK_RESIDENT_STATS 4
+int hobak_ctx_resident_stats(hobak_ctx* ctx, int64_t* out);
+
 /* Continuous-batching scheduler (no counterpart in the reference, whose callers step one scene
  * at a time through SIMULATION_SCENE::stepSimulation, SIMULATION_SCENE.h:120-126).
  * A request advances one instance by one step.  Submitting attaches the instance to the
