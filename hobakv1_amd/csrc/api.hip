@@ -54,7 +54,31 @@ constexpr double kEps = 2.220446049250313e-16;  // Eigen's default CG tolerance 
 constexpr int kMaxPlans = 32;
 constexpr int kMaxSamples = 512;
 constexpr int kResBig = 1 << 20;      // hobak_inst::res_pack of an instance on every compute unit
-constexpr int kResidentIters = 2048;  // a solve of more iterations goes on in a second launch, after the whole batch
+// A solve of more iterations goes on in another launch, after the whole batch.  This also is the most that the
+// tuning key allows: 2,048 iterations of up to 40 us stay well below the time that the workgroups of an instance behind
+// them wait for each other.
+constexpr int kResidentIters = 2048;
+// How long an instance's workgroups wait for each other: they are dispatched together, so they meet within
+// microseconds unless other work holds compute units.  A launch of another context ends within tens of
+// milliseconds; past that something does not give its compute units back.
+constexpr int kJoinUs = 200000;
+// Launches in a row whose workgroups did not meet after which an instance on every compute unit solves in the two-kernel
+// form: its sums round differently there, so that is the last resort.
+constexpr int kBigTries = 4;
+
+// A form of the resident PCG whose workgroups did not meet is left out for a number of ticks, twice as many each
+// time it happens again, so that the waits cost little however long the other work stays; half as many each
+// time the form has run.
+struct Hold {
+  int first, left = 0, next;
+  explicit Hold(int first_) : first(first_), next(first_) {}
+  bool pass() { return left == 0 || left-- == 0; }  // whether this tick may take the form
+  void late() {
+    left = next;
+    next = std::min(2 * next, 1 << 20);
+  }
+  void met() { next = std::max(first, next / 2); }
+};
 }  // namespace
 
 struct hobak_ctx {
@@ -75,7 +99,7 @@ struct hobak_ctx {
   int agg = 0;                         // reduced-precision form: spatial order and local aggregates (2: also with the coarse correction)
   int resident = kResidentIters;       // resident PCG: iterations per launch, 0 off
   int cus = 0;                         // compute units of the device
-  bool dies = true;                    // small batches of the resident PCG run on one die each
+  Hold device_hold{64}, die_hold{16};  // the resident PCG over the device, and on one die each
   int* tickets = nullptr;              // resident PCG launches of this context's stream
   int64_t res_stat[HOBAK_RESIDENT_STATS] = {};  // see hobak_ctx_resident_stats
   hipStream_t stream = nullptr;
@@ -468,10 +492,14 @@ struct hobak_inst {
   double spmv_ms_sum = 0.0, spmv_bytes_sum = 0.0;
   long long spmv_count = 0;
   unsigned work_seen = 0;           // Ctl::spmv_work at the last status poll
-  // resident PCG: most update workgroups' rows one workgroup takes (0: never resident), what
-  // Ctl::res_abort held at the last status poll, refinement sweeps of the last solve
+  // resident PCG: most update workgroups' rows one workgroup takes (0: never resident), whether its columns fit
+  // the workgroups of one die, what Ctl::res_abort and res_late held at the last status poll, launches in a row
+  // whose workgroups did not meet and the hold that follows (kResBig), refinement sweeps of the last solve
   int res_pack = 0;
-  int abort_seen = 0;
+  bool die_fit = true;
+  int abort_seen = 0, late_seen = 0;
+  int late_row = 0;
+  Hold big_hold{64};
   unsigned runs_seen = 0;  // likewise Ctl::res_runs
   int sweeps_seen = 0;
 };
@@ -944,13 +972,14 @@ bool stream_matrix(const hobak_ctx* ctx, double solving_bytes) {
 // 1.77 ms on one die and 1.10, 1.31 and 1.65 ms over all of them; 30, 39 and 56 in FP64 1.04, 1.39 and
 // 1.48 ms, and 1.21, 1.38 and 1.57.
 int die_workgroups(const hobak_inst* I) {
+  if (!I->die_fit) return 0;
   const int nu = I->h.nb[K_UPD], per = (nu + kResDieWgs - 1) / kResDieWgs;
   return I->res_pack != kResBig && per <= std::min(I->res_pack, 2) ? (nu + per - 1) / per : 0;
 }
 // Whether the instances run on one die each, and if so the most workgroups of any: at most as many as there are
 // dies, each within one.
 int resident_per_die(const hobak_ctx* ctx, const std::vector<hobak_inst*>& m) {
-  if (!ctx->dies || ctx->cus != kResDies * kResDieWgs || (int)m.size() > kResDies) return 0;
+  if (ctx->cus != kResDies * kResDieWgs || (int)m.size() > kResDies) return 0;
   int most = 0;
   for (auto* I : m) {
     const int w = die_workgroups(I);
@@ -958,6 +987,13 @@ int resident_per_die(const hobak_ctx* ctx, const std::vector<hobak_inst*>& m) {
     most = std::max(most, w);
   }
   return most > 1 ? most : 0;  // (a workgroup by itself exchanges nothing)
+}
+
+// How long the workgroups of an instance wait for each other in the launches that follow.
+int set_join(hobak_ctx* ctx, int us) {
+  HIPCHK(ctx, hipMemcpyAsync(ctx->tickets + kResJoin, &us, sizeof(us), hipMemcpyHostToDevice, ctx->stream));
+  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  return HOBAK_OK;
 }
 
 // The resident PCG's launch tables in the arena: the instances, largest first (their solves take the
@@ -1222,20 +1258,28 @@ int tick_impl(hobak_sched* S) {
   // instances that fit on chip run the resident PCG; a tick whose next group is sampled first runs
   // that group over every solving instance in the two-kernel form, which the samples time
   const bool may_reside = ctx->resident > 0 && ctx->grid_cap == 0;
-  for (auto& r : S->active)
-    if (r.stage == 1 && may_reside && r.I->res_pack > 0) {
-      resident.push_back(r.I);
-      if (r.I->res_pack == kResBig) resident_big.push_back(r.I);
-    }
+  bool candidates = false;
+  for (auto& r : S->active) candidates |= r.stage == 1 && r.I->res_pack > 0 && r.I->res_pack != kResBig;
+  const bool over_device = may_reside && candidates && ctx->device_hold.pass();
+  std::vector<char> resides(S->active.size(), 0);
+  for (size_t i = 0; i < S->active.size(); i++) {
+    auto& r = S->active[i];
+    if (r.stage != 1 || !may_reside || r.I->res_pack == 0) continue;
+    if (r.I->res_pack == kResBig ? !r.I->big_hold.pass() : !over_device) continue;
+    resides[i] = 1;
+    resident.push_back(r.I);
+    if (r.I->res_pack == kResBig) resident_big.push_back(r.I);
+  }
   // (a step of resident instances whose samples would all fall inside its one launch has its second
   // iteration sampled instead)
   const bool brief = !resident.empty() && S->ephemeral && every > 0 && S->samples.empty() && !sampled_group();
   const bool sample_first = !resident.empty() && (brief || sampled_group());
   const int group_iters = brief ? 2 : k;
   int sweeps = 1, die_wgs = 0;
-  for (auto& r : S->active) {
+  for (size_t i = 0; i < S->active.size(); i++) {
+    auto& r = S->active[i];
     if (r.stage != 1) continue;
-    const bool res = may_reside && r.I->res_pack > 0;
+    const bool res = resides[i] != 0;
     if (res && r.I->h.refine) sweeps = std::max(sweeps, r.I->sweeps_seen > 0 ? r.I->sweeps_seen : 2);
     if (res && !sample_first) continue;
     nsolving++;
@@ -1279,17 +1323,19 @@ int tick_impl(hobak_sched* S) {
     for (auto* I : resident)
       if (I->res_pack != kResBig) rest.push_back(I);
     if (!rest.empty()) die_wgs = resident_per_die(ctx, rest);
+    if (die_wgs && !ctx->die_hold.pass()) die_wgs = 0;
     if (!rest.empty()) TRY(resident_tables(ctx, rest, die_wgs, rb));
     if (!resident_big.empty()) TRY(resident_tables(ctx, resident_big, 0, rbig));
     Plan PR;
     const bool all = (int)resident.size() == M.n;
     if (!all) TRY(plan_transient(ctx, resident, PR));
+    const int iters = std::min(ctx->resident, kResidentIters);
     for (int j = 0; j < sweeps; j++) {
       if (die_wgs)
-        HIPCHK(ctx, launch_cg_resident_die<T>(rb, M.shift, M.groups, die_wgs, ctx->tickets, ctx->resident, s));
+        HIPCHK(ctx, launch_cg_resident_die<T>(rb, M.shift, M.groups, die_wgs, ctx->tickets, iters, s));
       else
-        HIPCHK(ctx, launch_cg_resident<T>(rb, M.shift, M.groups, false, ctx->tickets, ctx->resident, s));
-      if (rbig.n) HIPCHK(ctx, launch_cg_resident<T>(rbig, M.shift, M.groups, true, ctx->tickets, ctx->resident, s));
+        HIPCHK(ctx, launch_cg_resident<T>(rb, M.shift, M.groups, false, ctx->tickets, iters, s));
+      if (rbig.n) HIPCHK(ctx, launch_cg_resident<T>(rbig, M.shift, M.groups, true, ctx->tickets, iters, s));
       TRY(launch_solve_ends<T>(ctx, all ? M : PR));
     }
     S->stat[1] += sweeps;
@@ -1311,6 +1357,7 @@ int tick_impl(hobak_sched* S) {
   // the resident PCG counts the products a solve formed; its launches are the most any instance did
   double work_bytes = 0.0;
   unsigned res_launches = 0;
+  bool ran_rest = false, late_rest = false;  // of the instances that are not on every compute unit
   for (int i = 0; i < M.n; i++) {
     hobak_inst* I = M.members[i];
     const unsigned w = M.status_host[i].spmv_work;
@@ -1324,16 +1371,38 @@ int tick_impl(hobak_sched* S) {
     I->runs_seen += runs;
     ctx->res_stat[I->res_pack == kResBig ? HOBAK_RESIDENT_BIG : die_wgs ? HOBAK_RESIDENT_DIE : HOBAK_RESIDENT_DEVICE] +=
         runs;
-    ctx->res_stat[HOBAK_RESIDENT_ABORTED] += M.status_host[i].res_abort - I->abort_seen;
-    if (die_wgs && (stuck || M.status_host[i].res_abort != I->abort_seen)) {
-      ctx->dies = false;
-      I->abort_seen = M.status_host[i].res_abort;
-    } else if (M.status_host[i].res_abort != I->abort_seen) {  // did not fit, or could not run at once
-      I->abort_seen = M.status_host[i].res_abort;
-      I->res_pack = I->res_pack == kResBig ? 0 : I->res_pack / 2;  // more workgroups, each with fewer rows, while the device has that many
+    const int aborts = M.status_host[i].res_abort - I->abort_seen, late = M.status_host[i].res_late - I->late_seen;
+    I->abort_seen += aborts;
+    I->late_seen += late;
+    ctx->res_stat[HOBAK_RESIDENT_ABORTED] += aborts;
+    ctx->res_stat[HOBAK_RESIDENT_LATE] += late;
+    // columns that do not fit never will: more workgroups, each with fewer rows, while the device has that many, and
+    // over the device instead of on one die.  Workgroups that did not meet may do so later.
+    const bool misfit = aborts > late;
+    if (I->res_pack == kResBig) {
+      if (runs) I->big_hold.met();
+      I->late_row = runs ? 0 : I->late_row + late;
+      if (I->late_row >= kBigTries) {
+        I->big_hold.late();
+        I->late_row = 0;
+      }
+      if (misfit) I->res_pack = 0;
+      continue;
+    }
+    ran_rest |= runs > 0;
+    late_rest |= late > 0 || (stuck && aborts == 0);
+    if (misfit && die_wgs) {
+      I->die_fit = false;
+    } else if (misfit) {
+      I->res_pack /= 2;
       if (I->res_pack > 0 && (I->h.nb[K_UPD] + I->res_pack - 1) / I->res_pack > ctx->cus) I->res_pack = 0;
     }
   }
+  Hold& hold = die_wgs ? ctx->die_hold : ctx->device_hold;
+  if (late_rest)
+    hold.late();
+  else if (ran_rest)
+    hold.met();
   S->stat[8] += work_bytes;
   const long long launches = std::max<long long>(nsolving ? (long long)m * group_iters : 0, res_launches);
   if (ran) S->stat[7] += (double)launches;
@@ -1644,8 +1713,9 @@ int hobak_ctx_create(int device, size_t hbm_budget_bytes, hobak_ctx** out) {
   }
   bool ok = true;
   for (auto& e : ctx->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
-  ok = ok && hipMalloc((void**)&ctx->tickets, (1 + kResDies) * sizeof(int)) == hipSuccess &&
-       hipMemsetAsync(ctx->tickets, 0, (1 + kResDies) * sizeof(int), ctx->stream) == hipSuccess;
+  ok = ok && hipMalloc((void**)&ctx->tickets, kResTickets * sizeof(int)) == hipSuccess &&
+       hipMemsetAsync(ctx->tickets, 0, kResTickets * sizeof(int), ctx->stream) == hipSuccess &&
+       set_join(ctx, kJoinUs) == HOBAK_OK;
   if (!ok || arena_ensure(ctx, 1 << 20) != HOBAK_OK || scratch_of_device(device, &ctx->scratch) != HOBAK_OK) {
     hobak_ctx_destroy(ctx);
     return HOBAK_E_HIP;
@@ -2462,6 +2532,10 @@ int hobak_ctx_set_tuning(hobak_ctx* ctx, int32_t key, int32_t value) {
       if (value < 0 || value > 65536) return fail(ctx, HOBAK_E_INVALID, "resident iterations out of range");
       ctx->resident = (value + 1) & ~1;
       return HOBAK_OK;
+    case HOBAK_TUNE_RESIDENT_JOIN:
+      if (value < 0 || value > 10000000) return fail(ctx, HOBAK_E_INVALID, "resident join time out of range");
+      HIPCHK(ctx, hipSetDevice(ctx->device));
+      return set_join(ctx, value);
     case HOBAK_TUNE_UPDATE_WGS:
       if (value < 1 || value > 65536) return fail(ctx, HOBAK_E_INVALID, "update workgroups out of range");
       ctx->update_cap = value;

@@ -115,9 +115,10 @@ struct Ctl {
   double ac_inv[3];  // coarse correction: 1 / (P^T A P), diagonal (see InstDev::coarse)
   unsigned spmv_work;  // SpMV launches that streamed this instance's matrix (wraps; a count)
   // the resident PCG (resident.hip): tag of the last published partial sums, the meeting point of an
-  // instance's workgroups, and the launches that left the instance untouched and that solved it
+  // instance's workgroups, the launches that left the instance untouched (res_late of them because its
+  // workgroups did not meet in time, the others because its columns do not fit) and those that advanced it
   unsigned res_epoch;
-  int res_arrive, res_exit, res_abort;
+  int res_arrive, res_exit, res_abort, res_late;
   unsigned res_runs;
 };
 
@@ -134,7 +135,7 @@ struct InstStatus {
   double err;       // sqrt(res^2 / b^2) of the finished solve
   double maxR;      // |S b|^2
   unsigned spmv_work;  // Ctl::spmv_work
-  int res_abort;       // Ctl::res_abort
+  int res_abort, res_late;  // Ctl's
   unsigned res_runs;   // Ctl::res_runs
 };
 
@@ -359,12 +360,17 @@ hipError_t launch_cg_spmv_p(const Batch& b, int shift, int pad, int stream, int 
 // Up to `iters` PCG iterations (from scalar set 0, which holds the current set again at the end) with
 // the matrices held on chip (resident.hip); b's prefix table counts each instance's workgroups, at
 // least 1 and at most nb[K_UPD], all of which must fit on the device at once; needs every update
-// workgroup to hold one run of rows (nb[K_UPD] below the cap).  tickets: 1 + kResDies zero ints.
+// workgroup to hold one run of rows (nb[K_UPD] below the cap), but for `big`, which every instance then takes
+// (resident_layout_big).  tickets: kResTickets ints, zero but for tickets[kResJoin], the microseconds that an
+// instance's workgroups wait for each other before they leave it untouched (0: those of an instance of several never
+// meet).  (As an argument of the kernel it would be kept in scalar registers that the loop needs: 40^3 FP64 step 4.90
+// instead of 4.80 ms.)
+constexpr int kResDies = 8, kResDieWgs = 32;
+constexpr int kResJoin = 1 + kResDies, kResTickets = kResJoin + 1;
 template <typename T>
 hipError_t launch_cg_resident(const Batch& b, int shift, int groups, bool big, int* tickets, int iters, hipStream_t s);
 // The same for at most kResDies instances, each on the workgroups of one die (at most `wgs`, the most any takes),
 // which exchange through its L2.  An instance whose die gets no workgroups is left untouched.
-constexpr int kResDies = 8, kResDieWgs = 32;
 template <typename T>
 hipError_t launch_cg_resident_die(const Batch& b, int shift, int groups, int wgs, int* tickets, int iters, hipStream_t s);
 // Whether the resident PCG has a variant for this slice height, update layout and row count.

@@ -67,7 +67,8 @@
 // whose workgroups have begun is incomplete and every other one makes progress.  Before a workgroup
 // changes anything it announces itself and waits for the others of its instance; if they do not appear in
 // time (another program holds the compute units) or one of them cannot hold its columns, the
-// instance is left untouched and counted in Ctl::res_abort, and the host runs the two-kernel form.
+// instance is left untouched and counted in Ctl::res_abort, and in Ctl::res_late where only time ran out: the
+// host then takes another form for good, or for a while.
 #include "kernels.h"
 #include "pcg_device.h"
 
@@ -91,13 +92,16 @@ constexpr int kResMaxUpd = 512;               // update workgroups of an instanc
 // the rest of its last group's rows a second time, up to 255 rows past its own 168 to 336 with 64-row slices.  A
 // lane then polls up to four words, so the rule ends where lanes would have more than one group each.
 constexpr int kSplitMax = 255;
-constexpr int kAbort = 1 << 30;
-constexpr u64 kJoinTicks = 20000000ull;       // 0.2 s of the 100 MHz wall clock
+constexpr int kMisfit = 1 << 30, kLate = 1 << 29, kAbort = kMisfit | kLate;  // of Ctl::res_arrive
 constexpr unsigned kWaitTicks = 500000000u;   // 5 s; every peer is running, so this is never reached
 constexpr int kAgentScope = 16;               // cache policy of a buffer access: coherent over the device's L2s
 constexpr int kDieScope = 0;                  // of a store: to this die's L2, where loads of the other policy find it
 constexpr int kArrived = 1023;                // Ctl::res_arrive: workgroups here; from kDieBit on, their dies as bits
 constexpr int kDieBit = 16;
+// How long the workgroups of an instance on one die wait for each other at most (Ctl::res_arrive; otherwise
+// tickets[kResJoin] us): another context's large instance may leave too few of that die's compute units while others
+// are free, and then the instance rather runs over the whole device soon.
+constexpr int kDieJoinUs = 1000;
 
 // 64-slot steps of a wave held in registers: 162 or 144 registers of values and 5 or 8 of places, of the
 // 256 a wave may use at two waves per SIMD.
@@ -247,7 +251,7 @@ __device__ __forceinline__ int al16(int x) { return (x + 15) & ~15; }
 
 template <typename T, int R, int H, bool BIG, bool ONE>
 __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __restrict__ I, int lb, int W,
-                                               int iters, char* lds) {
+                                               int iters, const int* join, char* lds) {
   constexpr bool kF32 = sizeof(T) < sizeof(double);
   constexpr int NR = kReg<T>, ND = kAhead<BIG>;
   constexpr unsigned ts = sizeof(T);
@@ -442,7 +446,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
       if (ONE) __hip_atomic_fetch_or(arr, 1 << (kDieBit + die_of_wave()), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_fetch_add(arr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     } else
-      __hip_atomic_fetch_or(arr, kAbort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_fetch_or(arr, kMisfit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (fits) {
     int* const clist = (int*)(lds + off_cl);
@@ -569,11 +573,13 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
       }
     // wait for the instance's other workgroups
     if (tid == 0) {
+      const unsigned join_us = ONE ? min(*gbl(join), kDieJoinUs) : *gbl(join);
       const u64 t0 = wall_clock64();
       int v = __hip_atomic_load(arr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      while (!(v & kAbort) && (v & kArrived) < W) {
-        if (wall_clock64() - t0 > kJoinTicks)
-          __hip_atomic_compare_exchange_strong(arr, &v, v | kAbort, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+      const bool never = join_us == 0 && W > 1;
+      while (!(v & kAbort) && (never || (v & kArrived) < W)) {
+        if (never || wall_clock64() - t0 > 100ull * join_us)
+          __hip_atomic_compare_exchange_strong(arr, &v, v | kLate, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT);
         else
           __builtin_amdgcn_s_sleep(1);
@@ -581,7 +587,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
       }
       // (every workgroup's die is in before it is counted, so all of them see the same ones here)
       if (ONE && !(v & kAbort) && __popc(v >> kDieBit) != 1)
-        v = __hip_atomic_fetch_or(arr, kAbort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) | kAbort;
+        v = __hip_atomic_fetch_or(arr, kLate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) | kLate;
       sh_flag = (v & kAbort) ? 0 : 1;
     }
     __syncthreads();
@@ -1166,7 +1172,9 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   if (tid == 0) {
     auto ex = (HOBAK_GLOBAL int*)&ctl->res_exit;
     if (__hip_atomic_fetch_add(ex, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == W - 1) {
-      if (__hip_atomic_load(arr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kAbort) ctl->res_abort += 1;
+      const int v = __hip_atomic_load(arr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (v & kAbort) ctl->res_abort += 1;
+      if ((v & kAbort) == kLate) ctl->res_late += 1;
       __hip_atomic_store(arr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(ex, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -1186,7 +1194,7 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 
   int lb, W;
   const HOBAK_GLOBAL InstDev* I =
       uptr((const InstDev*)seg_find(b, __builtin_amdgcn_readfirstlane(sh_ticket), lb, W));
-  resident_solve<T, R, H, BIG, false>(I, uniform_i(lb), uniform_i(W), iters, lds);
+  resident_solve<T, R, H, BIG, false>(I, uniform_i(lb), uniform_i(W), iters, tickets + kResJoin, lds);
   if (threadIdx.x == 0 &&
       __hip_atomic_fetch_add(tickets + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == b.total - 1) {
     __hip_atomic_store(tickets, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1211,7 +1219,7 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 
     const int lb = uniform_i(sh_ticket);
     if (lb < W) {
       const HOBAK_GLOBAL InstDev* I = uptr(b.n == 1 ? b.one : gbl(b.inst)[i]);
-      resident_solve<T, R, H, false, true>(I, lb, W, iters, lds);
+      resident_solve<T, R, H, false, true>(I, lb, W, iters, tickets + kResJoin, lds);
     }
   }
   if (threadIdx.x == 0 &&

@@ -1976,6 +1976,7 @@ __global__ __launch_bounds__(kBlock) void status_kernel(Batch b, InstStatus* out
     o.first_iters = I->refine ? c->rs.first_iters : s->iters;
     o.spmv_work = c->spmv_work;
     o.res_abort = c->res_abort;
+    o.res_late = c->res_late;
     o.res_runs = c->res_runs;
     if (I->refine) {
       o.err = c->rs.b2 > 0 ? sqrt(c->rs.res2 / c->rs.b2) : 0.0;

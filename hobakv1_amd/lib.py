@@ -148,6 +148,7 @@ TUNE_P_FORM = 12
 TUNE_COARSE = 13
 TUNE_AGG = 14
 TUNE_RESIDENT = 15
+TUNE_RESIDENT_JOIN = 16
 
 _lib = None
 
@@ -250,7 +251,7 @@ class Context:
     def set_tuning(self, slice_rows=None, poll_chunk=None, max_chunks=None, graphs=None,
                    grid_cap=None, update_wgs=None, spmv_pad=None, spmv_stream_mb=None,
                    row_sort=None, compact_pct=None, update_groups=None, p_form=None, coarse=None,
-                   agg=None, resident=None):
+                   agg=None, resident=None, resident_join=None):
         """Kernel and engine tuning (see hobak_ctx_set_tuning)."""
         for key, val in ((TUNE_SLICE_ROWS, slice_rows), (TUNE_POLL_CHUNK, poll_chunk),
                          (TUNE_MAX_CHUNKS, max_chunks), (TUNE_GRAPHS, graphs),
@@ -258,15 +259,17 @@ class Context:
                          (TUNE_SPMV_PAD, spmv_pad), (TUNE_SPMV_STREAM_MB, spmv_stream_mb),
                          (TUNE_ROW_SORT, row_sort), (TUNE_COMPACT_PCT, compact_pct),
                          (TUNE_UPDATE_GROUPS, update_groups), (TUNE_P_FORM, p_form),
-                         (TUNE_COARSE, coarse), (TUNE_AGG, agg), (TUNE_RESIDENT, resident)):
+                         (TUNE_COARSE, coarse), (TUNE_AGG, agg), (TUNE_RESIDENT, resident),
+                         (TUNE_RESIDENT_JOIN, resident_join)):
             if val is not None:
                 self.check(self.lib.hobak_ctx_set_tuning(self.h, key, int(val)), "set_tuning")
 
     def resident_stats(self):
-        """Instance launches of the resident PCG by form, and those that left an instance untouched."""
-        out = (ctypes.c_int64 * 4)()
+        """Instance launches of the resident PCG by form, and those that left an instance untouched
+        (`late` of them because its workgroups did not meet in time)."""
+        out = (ctypes.c_int64 * 5)()
         self.check(self.lib.hobak_ctx_resident_stats(self.h, out), "resident_stats")
-        return dict(zip(("device", "die", "big", "aborted"), out))
+        return dict(zip(("device", "die", "big", "aborted", "late"), out))
 
     def copy_probe(self, nbytes, reps=20):
         ms = ctypes.c_double(0)

@@ -304,7 +304,15 @@ int hobak_kernel_stats(hobak_inst* inst, double* spmv_avg_ms, int64_t* spmv_coun
  *                          two-kernel form, as does everything while GRID_CAP is set.  Results do not
  *                          depend on it, but for FP32_REFINE instances of more rows than the update
  *                          workgroups cover in one run each (86,016 by default), whose sums of products
- *                          round in another order than the two-kernel form's.  Default 2048; 0 never */
+ *                          round in another order than the two-kernel form's.  Default 2048, which values
+                          above it count as; 0 never
+ *   HOBAK_TUNE_RESIDENT_JOIN  microseconds that the workgroups of an instance of the resident form, which run
+                          at the same time, wait for each other (at most 1000 where the instance is on one
+                          die).  Where other work holds the compute units for longer, the instance is left
+                          untouched, solves in the two-kernel form (from one die: over the device), and
+                          tries again some ticks later, twice as many each time.  FP32_REFINE instances
+                          whose sums would round differently there take the two-kernel form only
+                          after four waits in a row.  Default 200000; 0: they never meet */
 #define HOBAK_TUNE_SLICE_ROWS 0
 #define HOBAK_TUNE_POLL_CHUNK 2
 #define HOBAK_TUNE_MAX_CHUNKS 3
@@ -320,17 +328,20 @@ int hobak_kernel_stats(hobak_inst* inst, double* spmv_avg_ms, int64_t* spmv_coun
 #define HOBAK_TUNE_COARSE 13
 #define HOBAK_TUNE_AGG 14
 #define HOBAK_TUNE_RESIDENT 15
+#define HOBAK_TUNE_RESIDENT_JOIN 16
 int hobak_ctx_set_tuning(hobak_ctx* ctx, int32_t key, int32_t value);
 
 /* Counters since the context was created, HOBAK_RESIDENT_STATS int64: for each instance of each launch
  * of the resident PCG (HOBAK_TUNE_RESIDENT), which form advanced it - over the whole device, on one die,
  * or on every compute unit (FP32_REFINE instances of more rows than the update workgroups cover) - or
- * that the launch left it untouched, for the two-kernel form to solve. */
+ * that the launch left it untouched, for another form to solve: all of those, and the ones among them whose
+ * workgroups did not meet in time (HOBAK_TUNE_RESIDENT_JOIN; the others' columns do not fit). */
 #define HOBAK_RESIDENT_DEVICE 0
 #define HOBAK_RESIDENT_DIE 1
 #define HOBAK_RESIDENT_BIG 2
 #define HOBAK_RESIDENT_ABORTED 3
-#define HOBAK_RESIDENT_STATS 4
+#define HOBAK_RESIDENT_LATE 4
+#define HOBAK_RESIDENT_STATS 5
 int hobak_ctx_resident_stats(hobak_ctx* ctx, int64_t* out);
 
 /* Continuous-batching scheduler (no counterpart in the reference, whose callers step one scene

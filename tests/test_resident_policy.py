@@ -1,0 +1,103 @@
+"""Which PCG form the engine takes after a resident launch left an instance untouched, on the CPU (host_engine)."""
+import pytest
+
+import host_engine
+from host_engine import LATE, MISFIT, RUNS
+from hobakv1_amd import lib, scenes
+
+F64, F32 = lib.PRECISION_FP64, lib.PRECISION_FP32_REFINE
+
+
+@pytest.fixture
+def engine(monkeypatch):
+    monkeypatch.setattr(lib, "_lib", host_engine.load())
+    made = []
+
+    def make(**tuning):
+        made.append(host_engine.Engine(**tuning))
+        return made[-1]
+
+    yield make
+    for e in made:
+        e.ctx.close()
+
+
+def _inst(e, dims, precision=F64, **script):
+    inst = lib.Instance(e.ctx, scenes.lattice_scene(dims, seed=1), precision=precision)
+    e.script(inst, **script)
+    e.log()
+    return inst
+
+
+def _step(e, inst):
+    inst.step(True)
+    return e.forms()
+
+
+def test_workgroups_that_did_not_meet_meet_later(engine):
+    """40^3: 411 update workgroups; a stall once sends a step to the two-kernel form, for a while and not for good."""
+    e = engine()
+    inst = _inst(e, (40, 40, 40))
+    assert _step(e, inst) == ["device"]
+    e.script(inst, device=LATE)
+    assert _step(e, inst) == ["device", "spmv"]
+    e.script(inst)
+    later = [_step(e, inst) for _ in range(200)]
+    assert later[0] == ["spmv"] and later[-1] == ["device"]
+    assert e.ctx.resident_stats()["late"] == 1
+
+
+def test_stalls_that_go_on_cost_ever_fewer_waits(engine):
+    e = engine()
+    inst = _inst(e, (40, 40, 40), device=LATE)
+    waits = sum(_step(e, inst)[0] == "device" for _ in range(2000))
+    assert 2 <= waits <= 8
+    assert e.ctx.resident_stats() == {"device": 0, "die": 0, "big": 0, "aborted": waits, "late": waits}
+
+
+def test_columns_that_do_not_fit_take_more_workgroups_and_then_the_two_kernel_form(engine):
+    e = engine()
+    inst = _inst(e, (40, 40, 40), device=MISFIT)
+    for _ in range(4):
+        _step(e, inst)
+    assert _step(e, inst) == ["spmv"]
+    e.script(inst)
+    assert all(_step(e, inst) == ["spmv"] for _ in range(200))
+
+
+def test_a_die_without_room_leaves_the_device_to_the_instance(engine):
+    """Another context's large instance holds most of every die: the step goes on over the device, at once."""
+    e = engine()
+    inst = _inst(e, (10, 10, 10))
+    assert _step(e, inst) == ["die"]
+    e.script(inst, die=LATE)
+    assert _step(e, inst) == ["die", "device"]
+    assert _step(e, inst) == ["device"]
+    e.script(inst)
+    assert [_step(e, inst) for _ in range(60)][-1] == ["die"]
+
+
+def test_columns_that_do_not_fit_a_die_keep_only_their_instance_off_it(engine):
+    e = engine()
+    a, b = _inst(e, (10, 10, 10)), _inst(e, (10, 10, 12), die=MISFIT)
+    assert _step(e, b) == ["die", "device"]
+    assert _step(e, b) == ["device"]
+    assert _step(e, a) == ["die"]
+
+
+def test_an_instance_on_every_compute_unit_keeps_its_form_through_a_stall(engine):
+    """Its sums round differently in the two-kernel form, so that is taken only after several waits in a row."""
+    e = engine(update_wgs=256)
+    inst = _inst(e, (35, 37, 35), precision=F32, big=LATE)
+    e.ctx.set_tuning(max_chunks=1, poll_chunk=2)
+    forms = _step(e, inst)
+    assert forms[:2] == ["big", "spmv"] and e.ctx.resident_stats()["late"] == 4
+    e.script(inst)
+    assert [_step(e, inst) for _ in range(200)][-1] == ["big"]
+
+
+def test_a_launch_ends_before_the_wait_of_those_behind_it(engine):
+    e = engine(resident=65536)
+    inst = _inst(e, (10, 10, 10), iters=5000)
+    inst.step(True)
+    assert [int(w[3]) for w in e.log() if w[0] == "die"] == [2048] * 3
