@@ -99,6 +99,7 @@ struct hobak_ctx {
   int agg = 0;                         // reduced-precision form: spatial order and local aggregates (2: also with the coarse correction)
   int resident = kResidentIters;       // resident PCG: iterations per launch, 0 off
   int cus = 0;                         // compute units of the device
+  int join_us = kJoinUs;               // resident PCG: how long workgroups wait for each other
   Hold device_hold{64}, die_hold{16};  // the resident PCG over the device, and on one die each
   int* tickets = nullptr;              // resident PCG launches of this context's stream
   int64_t res_stat[HOBAK_RESIDENT_STATS] = {};  // see hobak_ctx_resident_stats
@@ -993,6 +994,7 @@ int resident_per_die(const hobak_ctx* ctx, const std::vector<hobak_inst*>& m) {
 int set_join(hobak_ctx* ctx, int us) {
   HIPCHK(ctx, hipMemcpyAsync(ctx->tickets + kResJoin, &us, sizeof(us), hipMemcpyHostToDevice, ctx->stream));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  ctx->join_us = us;
   return HOBAK_OK;
 }
 
@@ -1330,9 +1332,11 @@ int tick_impl(hobak_sched* S) {
     const bool all = (int)resident.size() == M.n;
     if (!all) TRY(plan_transient(ctx, resident, PR));
     const int iters = std::min(ctx->resident, kResidentIters);
+    // (workgroups that never meet: on a die, some are not there either)
+    const int wgs = ctx->join_us == 0 ? std::max(1, die_wgs - 1) : die_wgs;
     for (int j = 0; j < sweeps; j++) {
       if (die_wgs)
-        HIPCHK(ctx, launch_cg_resident_die<T>(rb, M.shift, M.groups, die_wgs, ctx->tickets, iters, s));
+        HIPCHK(ctx, launch_cg_resident_die<T>(rb, M.shift, M.groups, wgs, ctx->tickets, iters, s));
       else
         HIPCHK(ctx, launch_cg_resident<T>(rb, M.shift, M.groups, false, ctx->tickets, iters, s));
       if (rbig.n) HIPCHK(ctx, launch_cg_resident<T>(rbig, M.shift, M.groups, true, ctx->tickets, iters, s));
@@ -1363,9 +1367,6 @@ int tick_impl(hobak_sched* S) {
     const unsigned w = M.status_host[i].spmv_work;
     work_bytes += (double)(unsigned)(w - I->work_seen) * spmv_bytes_of(I);
     if (!resident.empty()) res_launches = std::max(res_launches, w - I->work_seen);
-    // (an instance still solving that did not advance: its die had no compute units for it)
-    const bool stuck = die_wgs && w == I->work_seen && M.status_host[i].phase == PHASE_SOLVING &&
-                       std::find(resident.begin(), resident.end(), I) != resident.end();
     I->work_seen = w;
     const unsigned runs = M.status_host[i].res_runs - I->runs_seen;
     I->runs_seen += runs;
@@ -1390,7 +1391,7 @@ int tick_impl(hobak_sched* S) {
       continue;
     }
     ran_rest |= runs > 0;
-    late_rest |= late > 0 || (stuck && aborts == 0);
+    late_rest |= late > 0;
     if (misfit && die_wgs) {
       I->die_fit = false;
     } else if (misfit) {

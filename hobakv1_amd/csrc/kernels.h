@@ -370,7 +370,7 @@ constexpr int kResJoin = 1 + kResDies, kResTickets = kResJoin + 1;
 template <typename T>
 hipError_t launch_cg_resident(const Batch& b, int shift, int groups, bool big, int* tickets, int iters, hipStream_t s);
 // The same for at most kResDies instances, each on the workgroups of one die (at most `wgs`, the most any takes),
-// which exchange through its L2.  An instance whose die gets no workgroups is left untouched.
+// which exchange through its L2.  An instance whose die gets too few of them is left untouched.
 template <typename T>
 hipError_t launch_cg_resident_die(const Batch& b, int shift, int groups, int wgs, int* tickets, int iters, hipStream_t s);
 // Whether the resident PCG has a variant for this slice height, update layout and row count.

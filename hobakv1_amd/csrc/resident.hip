@@ -59,8 +59,8 @@
 // words go to the die's own L2 by ordinary stores: both waits then take about 1000 cycles less of an
 // iteration's 13,000 (10^3 FP64 step 783 -> 686 us, 17x9x23 BDF 2.37 -> 2.03 ms).  The loads are the same, past the
 // compute unit's cache (a load of workgroup scope may be served from that cache and never see the
-// word).  Workgroups learn their die from the hardware; an instance whose workgroups turn out to be on several, or
-// whose die gets none, is left untouched, and the context uses the general form from then on.
+// word).  Workgroups learn their die from the hardware and take its tickets; an instance whose die gets too few
+// workgroups is left untouched.
 //
 // Residency.  An instance's workgroups wait for each other, so all of them must run at once.
 // Workgroups take tickets, and tickets are dealt to instances in order, so at most the last instance
@@ -96,8 +96,7 @@ constexpr int kMisfit = 1 << 30, kLate = 1 << 29, kAbort = kMisfit | kLate;  // 
 constexpr unsigned kWaitTicks = 500000000u;   // 5 s; every peer is running, so this is never reached
 constexpr int kAgentScope = 16;               // cache policy of a buffer access: coherent over the device's L2s
 constexpr int kDieScope = 0;                  // of a store: to this die's L2, where loads of the other policy find it
-constexpr int kArrived = 1023;                // Ctl::res_arrive: workgroups here; from kDieBit on, their dies as bits
-constexpr int kDieBit = 16;
+constexpr int kArrived = 1023;                // Ctl::res_arrive: workgroups here
 // How long the workgroups of an instance on one die wait for each other at most (Ctl::res_arrive; otherwise
 // tickets[kResJoin] us): another context's large instance may leave too few of that die's compute units while others
 // are free, and then the instance rather runs over the whole device soon.
@@ -442,10 +441,9 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   // announce this workgroup (or that its instance cannot run here)
   auto arr = (HOBAK_GLOBAL int*)&ctl->res_arrive;
   if (tid == 0) {
-    if (fits) {
-      if (ONE) __hip_atomic_fetch_or(arr, 1 << (kDieBit + die_of_wave()), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (fits)
       __hip_atomic_fetch_add(arr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else
+    else
       __hip_atomic_fetch_or(arr, kMisfit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (fits) {
@@ -585,9 +583,6 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           __builtin_amdgcn_s_sleep(1);
         v = __hip_atomic_load(arr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
-      // (every workgroup's die is in before it is counted, so all of them see the same ones here)
-      if (ONE && !(v & kAbort) && __popc(v >> kDieBit) != 1)
-        v = __hip_atomic_fetch_or(arr, kLate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) | kLate;
       sh_flag = (v & kAbort) ? 0 : 1;
     }
     __syncthreads();
@@ -1167,7 +1162,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
       }
     }
   }
-  // the last workgroup to leave clears the instance's meeting point
+  // the last workgroup to leave clears the instance's meeting point (ONE: if all W of them came; see the kernel)
   __syncthreads();
   if (tid == 0) {
     auto ex = (HOBAK_GLOBAL int*)&ctl->res_exit;
@@ -1222,10 +1217,22 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 
       resident_solve<T, R, H, false, true>(I, lb, W, iters, tickets + kResJoin, lds);
     }
   }
-  if (threadIdx.x == 0 &&
-      __hip_atomic_fetch_add(tickets, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1)
-    for (int k = 0; k <= kResDies; k++)
-      __hip_atomic_store(tickets + k, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x != 0) return;
+  __builtin_amdgcn_s_waitcnt(0);  // what this workgroup did to its meeting point is done
+  if (__hip_atomic_fetch_add(tickets, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (int)gridDim.x - 1) return;
+  // the grid's last workgroup: an instance whose die got too few workgroups is untouched, and its meeting point
+  // holds what those that came left there
+  for (int k = 0; k < b.n; k++) {
+    const int W = b.n == 1 ? b.total : gbl(b.boff)[k + 1] - gbl(b.boff)[k];
+    if (__hip_atomic_load(tickets + 1 + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= W) continue;
+    auto ctl = ctl_of(uptr(b.n == 1 ? b.one : gbl(b.inst)[k]));
+    if (ctl->sc[0].done) continue;
+    ctl->res_abort += 1;
+    ctl->res_late += 1;
+    __hip_atomic_store((HOBAK_GLOBAL int*)&ctl->res_arrive, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store((HOBAK_GLOBAL int*)&ctl->res_exit, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  for (int k = 0; k <= kResDies; k++) __hip_atomic_store(tickets + k, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <typename T, int R, int H, bool BIG>

@@ -312,7 +312,8 @@ int hobak_kernel_stats(hobak_inst* inst, double* spmv_avg_ms, int64_t* spmv_coun
                           untouched, solves in the two-kernel form (from one die: over the device), and
                           tries again some ticks later, twice as many each time.  FP32_REFINE instances
                           whose sums would round differently there take the two-kernel form only
-                          after four waits in a row.  Default 200000; 0: they never meet */
+                          after four waits in a row.  Default 200000; 0: they never meet, and a launch
+                          on single dies brings one workgroup too few to each */
 #define HOBAK_TUNE_SLICE_ROWS 0
 #define HOBAK_TUNE_POLL_CHUNK 2
 #define HOBAK_TUNE_MAX_CHUNKS 3

@@ -56,3 +56,17 @@ def test_every_compute_unit():
     got, stats = _run(scs, F32, [0], update_wgs=256, max_chunks=1)
     assert stats[0]["late"] >= 4 and stats[0]["big"] == 0
     assert np.linalg.norm(got[0][0] - want[0][0]) <= 1e-9 * np.linalg.norm(scs[0].rest.ravel() + want[0][0])
+
+
+@pytest.mark.parametrize("precision", [F64, F32])
+def test_a_die_that_gets_too_few_workgroups(precision):
+    """(With the wait at 0 a launch brings one workgroup too few to each die.)  Nothing of the launch stays behind:
+    the next ones on a die, and over the device, run."""
+    scs = [_lattice((10, 10, 10)), _lattice((17, 9, 23))]
+    joins = [0] + [200000] * 70
+    want, _ = _run(scs, precision, joins, resident=0)
+    got, stats = _run(scs, precision, joins)
+    for (u, v), (uw, vw) in zip(got, want):
+        assert np.array_equal(u, uw) and np.array_equal(v, vw)
+    assert stats[0]["late"] >= 2 and stats[0]["die"] == stats[0]["device"] == 0
+    assert stats[-1]["late"] == stats[0]["late"] and stats[-1]["die"] > 0
