@@ -58,10 +58,6 @@ constexpr int kResBig = 1 << 20;      // hobak_inst::res_pack of an instance on 
 // tuning key allows: 2,048 iterations of up to 40 us stay well below the time that the workgroups of an instance behind
 // them wait for each other.
 constexpr int kResidentIters = 2048;
-// How long an instance's workgroups wait for each other: they are dispatched together, so they meet within
-// microseconds unless other work holds compute units.  A launch of another context ends within tens of
-// milliseconds; past that something does not give its compute units back.
-constexpr int kJoinUs = 200000;
 // Launches in a row whose workgroups did not meet after which an instance on every compute unit solves in the two-kernel
 // form: its sums round differently there, so that is the last resort.
 constexpr int kBigTries = 4;
@@ -99,7 +95,7 @@ struct hobak_ctx {
   int agg = 0;                         // reduced-precision form: spatial order and local aggregates (2: also with the coarse correction)
   int resident = kResidentIters;       // resident PCG: iterations per launch, 0 off
   int cus = 0;                         // compute units of the device
-  int join_us = kJoinUs;               // resident PCG: how long workgroups wait for each other
+  int join = 1;                        // resident PCG: 0 marks every instance as one whose workgroups did not meet
   Hold device_hold{64}, die_hold{16};  // the resident PCG over the device, and on one die each
   int* tickets = nullptr;              // resident PCG launches of this context's stream
   int64_t res_stat[HOBAK_RESIDENT_STATS] = {};  // see hobak_ctx_resident_stats
@@ -990,14 +986,6 @@ int resident_per_die(const hobak_ctx* ctx, const std::vector<hobak_inst*>& m) {
   return most > 1 ? most : 0;  // (a workgroup by itself exchanges nothing)
 }
 
-// How long the workgroups of an instance wait for each other in the launches that follow.
-int set_join(hobak_ctx* ctx, int us) {
-  HIPCHK(ctx, hipMemcpyAsync(ctx->tickets + kResJoin, &us, sizeof(us), hipMemcpyHostToDevice, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  ctx->join_us = us;
-  return HOBAK_OK;
-}
-
 // The resident PCG's launch tables in the arena: the instances, largest first (their solves take the
 // most iterations, and what runs last should be short), and the workgroups of each.  An instance takes
 // as few workgroups as hold its matrix on chip (res_pack) when the batch fills the device's
@@ -1332,9 +1320,11 @@ int tick_impl(hobak_sched* S) {
     const bool all = (int)resident.size() == M.n;
     if (!all) TRY(plan_transient(ctx, resident, PR));
     const int iters = std::min(ctx->resident, kResidentIters);
-    // (workgroups that never meet: on a die, some are not there either)
-    const int wgs = ctx->join_us == 0 ? std::max(1, die_wgs - 1) : die_wgs;
+    const int wgs = ctx->join ? die_wgs : std::max(1, die_wgs - 1);
     for (int j = 0; j < sweeps; j++) {
+      if (!ctx->join)
+        for (auto* I : resident)
+          HIPCHK(ctx, hipMemcpyAsync(&I->h.ctl->res_arrive, &kResLate, sizeof(int), hipMemcpyHostToDevice, s));
       if (die_wgs)
         HIPCHK(ctx, launch_cg_resident_die<T>(rb, M.shift, M.groups, wgs, ctx->tickets, iters, s));
       else
@@ -1715,8 +1705,7 @@ int hobak_ctx_create(int device, size_t hbm_budget_bytes, hobak_ctx** out) {
   bool ok = true;
   for (auto& e : ctx->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
   ok = ok && hipMalloc((void**)&ctx->tickets, kResTickets * sizeof(int)) == hipSuccess &&
-       hipMemsetAsync(ctx->tickets, 0, kResTickets * sizeof(int), ctx->stream) == hipSuccess &&
-       set_join(ctx, kJoinUs) == HOBAK_OK;
+       hipMemsetAsync(ctx->tickets, 0, kResTickets * sizeof(int), ctx->stream) == hipSuccess;
   if (!ok || arena_ensure(ctx, 1 << 20) != HOBAK_OK || scratch_of_device(device, &ctx->scratch) != HOBAK_OK) {
     hobak_ctx_destroy(ctx);
     return HOBAK_E_HIP;
@@ -2534,9 +2523,8 @@ int hobak_ctx_set_tuning(hobak_ctx* ctx, int32_t key, int32_t value) {
       ctx->resident = (value + 1) & ~1;
       return HOBAK_OK;
     case HOBAK_TUNE_RESIDENT_JOIN:
-      if (value < 0 || value > 10000000) return fail(ctx, HOBAK_E_INVALID, "resident join time out of range");
-      HIPCHK(ctx, hipSetDevice(ctx->device));
-      return set_join(ctx, value);
+      ctx->join = value != 0;
+      return HOBAK_OK;
     case HOBAK_TUNE_UPDATE_WGS:
       if (value < 1 || value > 65536) return fail(ctx, HOBAK_E_INVALID, "update workgroups out of range");
       ctx->update_cap = value;

@@ -361,12 +361,9 @@ hipError_t launch_cg_spmv_p(const Batch& b, int shift, int pad, int stream, int 
 // the matrices held on chip (resident.hip); b's prefix table counts each instance's workgroups, at
 // least 1 and at most nb[K_UPD], all of which must fit on the device at once; needs every update
 // workgroup to hold one run of rows (nb[K_UPD] below the cap), but for `big`, which every instance then takes
-// (resident_layout_big).  tickets: kResTickets ints, zero but for tickets[kResJoin], the microseconds that an
-// instance's workgroups wait for each other before they leave it untouched (0: those of an instance of several never
-// meet).  (As an argument of the kernel it would be kept in scalar registers that the loop needs: 40^3 FP64 step 4.90
-// instead of 4.80 ms.)
-constexpr int kResDies = 8, kResDieWgs = 32;
-constexpr int kResJoin = 1 + kResDies, kResTickets = kResJoin + 1;
+// (resident_layout_big).  tickets: kResTickets zero ints.
+constexpr int kResDies = 8, kResDieWgs = 32, kResTickets = 1 + kResDies;
+constexpr int kResLate = 1 << 29;  // of Ctl::res_arrive: the workgroups did not meet, and leave the instance untouched
 template <typename T>
 hipError_t launch_cg_resident(const Batch& b, int shift, int groups, bool big, int* tickets, int iters, hipStream_t s);
 // The same for at most kResDies instances, each on the workgroups of one die (at most `wgs`, the most any takes),

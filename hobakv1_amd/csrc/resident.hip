@@ -92,15 +92,17 @@ constexpr int kResMaxUpd = 512;               // update workgroups of an instanc
 // the rest of its last group's rows a second time, up to 255 rows past its own 168 to 336 with 64-row slices.  A
 // lane then polls up to four words, so the rule ends where lanes would have more than one group each.
 constexpr int kSplitMax = 255;
-constexpr int kMisfit = 1 << 30, kLate = 1 << 29, kAbort = kMisfit | kLate;  // of Ctl::res_arrive
+constexpr int kMisfit = 1 << 30, kLate = kResLate, kAbort = kMisfit | kLate;  // of Ctl::res_arrive
+// How long an instance's workgroups wait for each other, in ticks of the 100 MHz wall clock: they are dispatched
+// together, so they meet within microseconds unless other work holds compute units.  A launch of another context
+// ends within tens of milliseconds; past 0.2 s something does not give its compute units back.  On one die, of
+// which a large instance of another context may leave too few compute units although others are free: 1 ms, after which
+// the instance rather runs over the whole device.
+constexpr u64 kJoinTicks = 20000000ull, kDieJoinTicks = 100000ull;
 constexpr unsigned kWaitTicks = 500000000u;   // 5 s; every peer is running, so this is never reached
 constexpr int kAgentScope = 16;               // cache policy of a buffer access: coherent over the device's L2s
 constexpr int kDieScope = 0;                  // of a store: to this die's L2, where loads of the other policy find it
 constexpr int kArrived = 1023;                // Ctl::res_arrive: workgroups here
-// How long the workgroups of an instance on one die wait for each other at most (Ctl::res_arrive; otherwise
-// tickets[kResJoin] us): another context's large instance may leave too few of that die's compute units while others
-// are free, and then the instance rather runs over the whole device soon.
-constexpr int kDieJoinUs = 1000;
 
 // 64-slot steps of a wave held in registers: 162 or 144 registers of values and 5 or 8 of places, of the
 // 256 a wave may use at two waves per SIMD.
@@ -250,7 +252,7 @@ __device__ __forceinline__ int al16(int x) { return (x + 15) & ~15; }
 
 template <typename T, int R, int H, bool BIG, bool ONE>
 __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __restrict__ I, int lb, int W,
-                                               int iters, const int* join, char* lds) {
+                                               int iters, char* lds) {
   constexpr bool kF32 = sizeof(T) < sizeof(double);
   constexpr int NR = kReg<T>, ND = kAhead<BIG>;
   constexpr unsigned ts = sizeof(T);
@@ -571,12 +573,10 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
       }
     // wait for the instance's other workgroups
     if (tid == 0) {
-      const unsigned join_us = ONE ? min(*gbl(join), kDieJoinUs) : *gbl(join);
       const u64 t0 = wall_clock64();
       int v = __hip_atomic_load(arr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const bool never = join_us == 0 && W > 1;
-      while (!(v & kAbort) && (never || (v & kArrived) < W)) {
-        if (never || wall_clock64() - t0 > 100ull * join_us)
+      while (!(v & kAbort) && (v & kArrived) < W) {
+        if (wall_clock64() - t0 > (ONE ? kDieJoinTicks : kJoinTicks))
           __hip_atomic_compare_exchange_strong(arr, &v, v | kLate, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT);
         else
@@ -1189,12 +1189,24 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 
   int lb, W;
   const HOBAK_GLOBAL InstDev* I =
       uptr((const InstDev*)seg_find(b, __builtin_amdgcn_readfirstlane(sh_ticket), lb, W));
-  resident_solve<T, R, H, BIG, false>(I, uniform_i(lb), uniform_i(W), iters, tickets + kResJoin, lds);
+  resident_solve<T, R, H, BIG, false>(I, uniform_i(lb), uniform_i(W), iters, lds);
   if (threadIdx.x == 0 &&
       __hip_atomic_fetch_add(tickets + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == b.total - 1) {
     __hip_atomic_store(tickets, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(tickets + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+}
+
+// The arguments of cg_resident_die_kernel, read anew from the argument segment: what its end needs is not held in
+// scalar registers through the solve.
+struct DieArgs {
+  Batch b;
+  int* tickets;
+};
+__device__ __forceinline__ const __attribute__((address_space(4))) DieArgs* late_args() {
+  auto a = (const __attribute__((address_space(4))) DieArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  return a;
 }
 
 // The same for up to eight instances, instance i on die i alone: the grid holds as many workgroups for each die as
@@ -1214,25 +1226,28 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 
     const int lb = uniform_i(sh_ticket);
     if (lb < W) {
       const HOBAK_GLOBAL InstDev* I = uptr(b.n == 1 ? b.one : gbl(b.inst)[i]);
-      resident_solve<T, R, H, false, true>(I, lb, W, iters, tickets + kResJoin, lds);
+      resident_solve<T, R, H, false, true>(I, lb, W, iters, lds);
     }
   }
   if (threadIdx.x != 0) return;
   __builtin_amdgcn_s_waitcnt(0);  // what this workgroup did to its meeting point is done
-  if (__hip_atomic_fetch_add(tickets, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (int)gridDim.x - 1) return;
+  const auto args = late_args();
+  const auto t = gbl(args->tickets);
+  if (__hip_atomic_fetch_add(t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (int)gridDim.x - 1) return;
   // the grid's last workgroup: an instance whose die got too few workgroups is untouched, and its meeting point
   // holds what those that came left there
-  for (int k = 0; k < b.n; k++) {
-    const int W = b.n == 1 ? b.total : gbl(b.boff)[k + 1] - gbl(b.boff)[k];
-    if (__hip_atomic_load(tickets + 1 + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= W) continue;
-    auto ctl = ctl_of(uptr(b.n == 1 ? b.one : gbl(b.inst)[k]));
+  const int n = args->b.n;
+  for (int k = 0; k < n; k++) {
+    const int W = n == 1 ? args->b.total : gbl(args->b.boff)[k + 1] - gbl(args->b.boff)[k];
+    if (__hip_atomic_load(t + 1 + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= W) continue;
+    auto ctl = ctl_of(gbl(n == 1 ? args->b.one : gbl(args->b.inst)[k]));
     if (ctl->sc[0].done) continue;
     ctl->res_abort += 1;
     ctl->res_late += 1;
     __hip_atomic_store((HOBAK_GLOBAL int*)&ctl->res_arrive, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store((HOBAK_GLOBAL int*)&ctl->res_exit, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  for (int k = 0; k <= kResDies; k++) __hip_atomic_store(tickets + k, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int k = 0; k <= kResDies; k++) __hip_atomic_store(t + k, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <typename T, int R, int H, bool BIG>

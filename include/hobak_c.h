@@ -306,14 +306,14 @@ int hobak_kernel_stats(hobak_inst* inst, double* spmv_avg_ms, int64_t* spmv_coun
  *                          workgroups cover in one run each (86,016 by default), whose sums of products
  *                          round in another order than the two-kernel form's.  Default 2048, which values
                           above it count as; 0 never
- *   HOBAK_TUNE_RESIDENT_JOIN  microseconds that the workgroups of an instance of the resident form, which run
-                          at the same time, wait for each other (at most 1000 where the instance is on one
-                          die).  Where other work holds the compute units for longer, the instance is left
-                          untouched, solves in the two-kernel form (from one die: over the device), and
-                          tries again some ticks later, twice as many each time.  FP32_REFINE instances
-                          whose sums would round differently there take the two-kernel form only
-                          after four waits in a row.  Default 200000; 0: they never meet, and a launch
-                          on single dies brings one workgroup too few to each */
+ *   HOBAK_TUNE_RESIDENT_JOIN  the workgroups of an instance of the resident form run at the same time, and wait
+ *                          for each other before they start (0.2 s, or 1 ms where the instance is on one
+ *                          die).  Where other work holds the compute units for longer, the instance is left
+ *                          untouched, solves in the two-kernel form (from one die: over the device), and
+ *                          tries again some ticks later, twice as many each time.  FP32_REFINE instances
+ *                          whose sums would round differently there take the two-kernel form only
+ *                          after four waits in a row.  Default 1; 0, for tests of that path: they never
+ *                          meet, and a launch on single dies brings one workgroup too few to each */
 #define HOBAK_TUNE_SLICE_ROWS 0
 #define HOBAK_TUNE_POLL_CHUNK 2
 #define HOBAK_TUNE_MAX_CHUNKS 3

@@ -37,7 +37,7 @@ def _run(scs, precision, joins, resident=512, **tuning):
                                        ([(5 + k, 8, 7) for k in range(12)], "device")])
 def test_left_untouched_and_taken_up_again(dims, form, precision):
     scs = [_lattice(d, seed=k) for k, d in enumerate(dims)]
-    joins = [200000, 0] + [200000] * 70
+    joins = [1, 0] + [1] * 70
     print(f"  {dims} precision {precision}", flush=True)
     want, _ = _run(scs, precision, joins, resident=0)
     got, stats = _run(scs, precision, joins)
@@ -52,7 +52,7 @@ def test_left_untouched_and_taken_up_again(dims, form, precision):
 
 def test_every_compute_unit():
     scs = [_lattice((35, 37, 35))]
-    want, _ = _run(scs, F32, [200000], resident=0, update_wgs=256)
+    want, _ = _run(scs, F32, [1], resident=0, update_wgs=256)
     got, stats = _run(scs, F32, [0], update_wgs=256, max_chunks=1)
     assert stats[0]["late"] >= 4 and stats[0]["big"] == 0
     assert np.linalg.norm(got[0][0] - want[0][0]) <= 1e-9 * np.linalg.norm(scs[0].rest.ravel() + want[0][0])
@@ -60,10 +60,10 @@ def test_every_compute_unit():
 
 @pytest.mark.parametrize("precision", [F64, F32])
 def test_a_die_that_gets_too_few_workgroups(precision):
-    """(With the wait at 0 a launch brings one workgroup too few to each die.)  Nothing of the launch stays behind:
+    """(With HOBAK_TUNE_RESIDENT_JOIN 0 a launch brings one workgroup too few to each die.)  Nothing of the launch stays behind:
     the next ones on a die, and over the device, run."""
     scs = [_lattice((10, 10, 10)), _lattice((17, 9, 23))]
-    joins = [0] + [200000] * 70
+    joins = [0] + [1] * 70
     want, _ = _run(scs, precision, joins, resident=0)
     got, stats = _run(scs, precision, joins)
     for (u, v), (uw, vw) in zip(got, want):
