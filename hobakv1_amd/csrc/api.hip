@@ -488,7 +488,7 @@ struct hobak_inst {
   int first_iters = 0;              // iterations of the last step's first (inner) solve
   double spmv_ms_sum = 0.0, spmv_bytes_sum = 0.0;
   long long spmv_count = 0;
-  unsigned work_seen = 0;           // Ctl::spmv_work at the last status poll
+  unsigned work_seen = 0, res_seen = 0;  // Ctl::spmv_work and res_work at the last status poll
   // resident PCG: most update workgroups' rows one workgroup takes (0: never resident), whether its columns fit
   // the workgroups of one die, what Ctl::res_abort and res_late held at the last status poll, launches in a row
   // whose workgroups did not meet and the hold that follows (kResBig), refinement sweeps of the last solve
@@ -531,6 +531,8 @@ struct hobak_sched {
   // sampled SpMV launches of the current batch: (iteration index since the batch's prologue, slot)
   std::vector<std::pair<int, int>> samples;
   int sample_it = 0;
+  int res_it = 0;  // resident PCG iterations since the last sample
+  bool whole = false;  // a private scheduler's one sample is that of all members' first launch
   bool sampling = false;
   // a long-lived scheduler's own sampling (hobak_sched_set_kernel_sampling): every spmv_every-th
   // SpMV launch is timed and credited with the matrix bytes of the instances solving in its tick
@@ -1045,6 +1047,23 @@ int launch_solve_ends(hobak_ctx* ctx, const Plan& P) {
   return HOBAK_OK;
 }
 
+// The SpMV of an iteration of parity `j`, with timing events if a and b are.
+// FP64 groups whose matrices stream from HBM form p_new once per entry and gather it alone
+// (three kernels per iteration, bitwise the same results); the extra launch does not pay for
+// a working set that stays in the caches.
+template <typename T>
+int launch_spmv(hobak_ctx* ctx, const Plan& P, int stream, int j, hipEvent_t a = nullptr, hipEvent_t b = nullptr) {
+  hipStream_t s = ctx->stream;
+  const int cap = ctx->grid_cap;
+  if (sizeof(T) == 8 && (ctx->p_form == 2 || (ctx->p_form == 1 && stream))) {
+    HIPCHK(ctx, launch_cg_p(P.b[K_UPD], j & 1, cap, s));
+    HIPCHK(ctx, launch_cg_spmv_p(P.b[K_SPMV], P.shift, ctx->spmv_pad, stream, j & 1, cap, s, a, b));
+  } else {
+    HIPCHK(ctx, launch_cg_spmv<T>(P.b[K_SPMV], P.shift, ctx->spmv_pad, stream, P.coarse, j & 1, cap, s, a, b));
+  }
+  return HOBAK_OK;
+}
+
 // k PCG iterations over the batch (k even, so the current scalar set is set 0 again at the end),
 // then the gated end-of-solve kernels: the refinement residual, check and re-seed, or the plain
 // form's finish flag.  With a sampling scheduler, some SpMV launches carry timing events.
@@ -1052,10 +1071,6 @@ template <typename T>
 int launch_chunk(hobak_ctx* ctx, const Plan& P, int k, int stream, hobak_sched* S, int every) {
   hipStream_t s = ctx->stream;
   const int cap = ctx->grid_cap;
-  // FP64 groups whose matrices stream from HBM form p_new once per entry and gather it alone
-  // (three kernels per iteration, bitwise the same results); the extra launch does not pay for
-  // a working set that stays in the caches
-  const bool pform = sizeof(T) == 8 && (ctx->p_form == 2 || (ctx->p_form == 1 && stream));
   for (int j = 0; j < k; j++) {
     hipEvent_t a = nullptr, b = nullptr;
     if (S) {
@@ -1067,12 +1082,7 @@ int launch_chunk(hobak_ctx* ctx, const Plan& P, int k, int stream, hobak_sched* 
         S->samples.emplace_back(g, slot);
       }
     }
-    if (pform) {
-      HIPCHK(ctx, launch_cg_p(P.b[K_UPD], j & 1, cap, s));
-      HIPCHK(ctx, launch_cg_spmv_p(P.b[K_SPMV], P.shift, ctx->spmv_pad, stream, j & 1, cap, s, a, b));
-    } else {
-      HIPCHK(ctx, launch_cg_spmv<T>(P.b[K_SPMV], P.shift, ctx->spmv_pad, stream, P.coarse, j & 1, cap, s, a, b));
-    }
+    TRY(launch_spmv<T>(ctx, P, stream, j, a, b));
     HIPCHK(ctx, launch_cg_update<T>(P.b[K_UPD], P.groups, P.coarse | (P.agg << 1), j & 1, cap, s));
   }
   return launch_solve_ends<T>(ctx, P);
@@ -1108,7 +1118,7 @@ template <typename T>
 int tick_impl(hobak_sched* S) {
   hobak_ctx* ctx = S->ctx;
   hipStream_t s = ctx->stream;
-  TRY(arena_ensure(ctx, 7 * plan_bytes(S->members.size() + 1)));
+  TRY(arena_ensure(ctx, 9 * plan_bytes(S->members.size() + 1)));
   ctx->arena_off = 0;
   TRY(plan_get(ctx, S->members, &S->mplan));
   if (S->dirty) {
@@ -1183,6 +1193,7 @@ int tick_impl(hobak_sched* S) {
       if (r.begin) starters.push_back(r.I);
     }
   const bool pro = !join.empty();
+  const bool all_start = (int)starters.size() == M.n;
   bool pro_split = false;
   if (pro) {
     const Range r_pro("hobak prologue");
@@ -1245,8 +1256,7 @@ int tick_impl(hobak_sched* S) {
     return every > 0 && (int)S->samples.size() < kMaxSamples &&
            (S->sample_it / every) * every + every - 1 < S->sample_it + k;
   };
-  // instances that fit on chip run the resident PCG; a tick whose next group is sampled first runs
-  // that group over every solving instance in the two-kernel form, which the samples time
+  // instances that fit on chip run the resident PCG
   const bool may_reside = ctx->resident > 0 && ctx->grid_cap == 0;
   bool candidates = false;
   for (auto& r : S->active) candidates |= r.stage == 1 && r.I->res_pack > 0 && r.I->res_pack != kResBig;
@@ -1260,18 +1270,13 @@ int tick_impl(hobak_sched* S) {
     resident.push_back(r.I);
     if (r.I->res_pack == kResBig) resident_big.push_back(r.I);
   }
-  // (a step of resident instances whose samples would all fall inside its one launch has its second
-  // iteration sampled instead)
-  const bool brief = !resident.empty() && S->ephemeral && every > 0 && S->samples.empty() && !sampled_group();
-  const bool sample_first = !resident.empty() && (brief || sampled_group());
-  const int group_iters = brief ? 2 : k;
   int sweeps = 1, die_wgs = 0;
   for (size_t i = 0; i < S->active.size(); i++) {
     auto& r = S->active[i];
     if (r.stage != 1) continue;
     const bool res = resides[i] != 0;
     if (res && r.I->h.refine) sweeps = std::max(sweeps, r.I->sweeps_seen > 0 ? r.I->sweeps_seen : 2);
-    if (res && !sample_first) continue;
+    if (res) continue;
     nsolving++;
     solving_bytes += spmv_bytes_of(r.I);
     solving_wgs += r.I->h.nb[K_SPMV];
@@ -1280,27 +1285,57 @@ int tick_impl(hobak_sched* S) {
     const int q = p > 0 ? (p - r.done_iters) / k : 0;
     m = std::min(m, std::max(1, q));
   }
-  if (sample_first) m = 1;
   if (nsolving || !resident.empty()) HIPCHK(ctx, hipEventRecord(ctx->ev[4], s));
+  // The resident PCG has no SpMV launches, so where a sample is due, solves that start in it first have one
+  // SpMV launch of the two-kernel form timed.  What that writes, the first iteration of either form forms again from
+  // the same inputs, so results do not depend on sampling.  A private scheduler credits its samples with the whole
+  // batch: it times all of its members' first launch, and with resident members nothing else.
+  S->whole |= S->ephemeral && !resident.empty();
+  const bool group_samples = S->sampling && !S->whole;
+  int probed = 0;
+  double probe_bytes = 0.0;
+  if (every > 0 && !resident.empty() && (int)S->samples.size() < kMaxSamples &&
+      (S->ephemeral ? all_start : S->res_it >= every || S->spmv_n == 0)) {
+    std::vector<hobak_inst*> fresh;
+    double fresh_bytes = 0.0;
+    for (size_t i = 0; i < S->active.size(); i++) {
+      auto& r = S->active[i];
+      if (r.stage != 1 || std::find(join.begin(), join.end(), r.I) == join.end()) continue;
+      if (!S->ephemeral && !resides[i]) continue;
+      fresh.push_back(r.I);
+      fresh_bytes += spmv_bytes_of(r.I);
+    }
+    if (!fresh.empty()) {
+      Plan PF;
+      TRY(plan_transient(ctx, fresh, PF));
+      const int slot = (int)S->samples.size();
+      TRY(launch_spmv<T>(ctx, PF, stream_matrix(ctx, fresh_bytes) ? 1 : 0, 0, ctx->sample_ev[2 * slot],
+                         ctx->sample_ev[2 * slot + 1]));
+      S->samples.emplace_back(0, slot);
+      S->res_it = 0;
+      probed = 1;
+      probe_bytes = fresh_bytes;
+    }
+  }
   if (nsolving) {
     const Range r_pcg("hobak pcg groups");
     const int st = stream_matrix(ctx, solving_bytes) ? 1 : 0;
     const bool compact = nsolving < M.n && solving_wgs * 100 <= (long)ctx->compact_pct * M.b[K_SPMV].total;
     Plan PG;
     if (compact) TRY(plan_transient(ctx, solving, PG));
-    if (graphs && !compact && !brief && (!M.chunk_exec[st] || M.chunk_k[st] != k)) {
+    if (graphs && !compact && (!M.chunk_exec[st] || M.chunk_k[st] != k)) {
       if (M.chunk_exec[st]) (void)hipGraphExecDestroy(M.chunk_exec[st]);
       M.chunk_exec[st] = nullptr;
       TRY(capture(ctx, &M.chunk_exec[st], [&]() { return launch_chunk<T>(ctx, M, k, st, nullptr, 0); }));
       M.chunk_k[st] = k;
     }
     for (int j = 0; j < m; j++) {
-      if (graphs && !compact && !brief && !sampled_group()) {  // every unsampled group replays the graph
+      if (graphs && !compact && !(group_samples && sampled_group())) {  // every unsampled group replays the graph
         HIPCHK(ctx, hipGraphLaunch(M.chunk_exec[st], s));
-        if (S->sampling) S->sample_it += k;
+        if (group_samples) S->sample_it += k;
         S->stat[9] += 1;
       } else {
-        TRY(launch_chunk<T>(ctx, compact ? PG : M, group_iters, st, S->sampling ? S : nullptr, brief ? 2 : every));
+        TRY(launch_chunk<T>(ctx, compact ? PG : M, k, st, group_samples ? S : nullptr, every));
         S->stat[10] += 1;
       }
     }
@@ -1349,15 +1384,17 @@ int tick_impl(hobak_sched* S) {
   // algorithmic SpMV bytes of this tick: each member's matrix and vectors once per launch that
   // streamed them (counted on the device; launches after a member's solve ended read nothing)
   // the resident PCG counts the products a solve formed; its launches are the most any instance did
-  double work_bytes = 0.0;
+  double work_bytes = 0.0, launch_bytes = 0.0;  // all products; those of the SpMV's own launches
   unsigned res_launches = 0;
   bool ran_rest = false, late_rest = false;  // of the instances that are not on every compute unit
   for (int i = 0; i < M.n; i++) {
     hobak_inst* I = M.members[i];
-    const unsigned w = M.status_host[i].spmv_work;
-    work_bytes += (double)(unsigned)(w - I->work_seen) * spmv_bytes_of(I);
-    if (!resident.empty()) res_launches = std::max(res_launches, w - I->work_seen);
-    I->work_seen = w;
+    const unsigned work = M.status_host[i].spmv_work - I->work_seen, res_work = M.status_host[i].res_work - I->res_seen;
+    I->work_seen += work;
+    I->res_seen += res_work;
+    launch_bytes += (double)work * spmv_bytes_of(I);
+    work_bytes += (double)(work + res_work) * spmv_bytes_of(I);
+    res_launches = std::max(res_launches, res_work);
     const unsigned runs = M.status_host[i].res_runs - I->runs_seen;
     I->runs_seen += runs;
     ctx->res_stat[I->res_pack == kResBig ? HOBAK_RESIDENT_BIG : die_wgs ? HOBAK_RESIDENT_DIE : HOBAK_RESIDENT_DEVICE] +=
@@ -1395,9 +1432,9 @@ int tick_impl(hobak_sched* S) {
   else if (ran_rest)
     hold.met();
   S->stat[8] += work_bytes;
-  const long long launches = std::max<long long>(nsolving ? (long long)m * group_iters : 0, res_launches);
-  if (ran) S->stat[7] += (double)launches;
-  if (S->sampling) S->sample_it += std::max(0, (int)res_launches - (sample_first ? group_iters : 0));
+  const long long group_launches = nsolving ? (long long)m * k : 0;
+  if (ran) S->stat[7] += (double)(std::max<long long>(group_launches, res_launches) + probed);
+  S->res_it += (int)res_launches;
   const double now = clock_s(S);
   if (pro) {
     if (pro_split) {
@@ -1412,9 +1449,10 @@ int tick_impl(hobak_sched* S) {
   if (epi) S->ms[4] += elapsed(ctx, 6, 7);
   if (!S->ephemeral && S->sampling) {
     // the window's algorithmic bytes and launches; the sampled launches (every `every`-th one)
-    // give the average launch time, so bytes / (launches * average) is the window's rate
-    S->spmv_bytes += work_bytes;
-    if (ran) S->spmv_launches += launches;
+    // give the average launch time, so bytes / (launches * average) is the window's rate.  A launch ahead of
+    // resident solves stands for `every` of theirs.
+    S->spmv_bytes += launch_bytes + (probed ? (double)(every - 1) * probe_bytes : 0.0);
+    S->spmv_launches += group_launches + (probed ? every : 0);
   }
   if (!S->ephemeral && S->sampling && !S->samples.empty()) {
     for (auto& sm : S->samples) {
@@ -2623,6 +2661,7 @@ int hobak_sched_set_kernel_sampling(hobak_sched* S, int32_t every) {
   S->spmv_every = every;
   S->sampling = every > 0;
   S->sample_it = 0;
+  S->res_it = 0;
   S->samples.clear();
   S->spmv_ms = S->spmv_bytes = 0.0;
   S->spmv_n = S->spmv_launches = 0;

@@ -120,6 +120,7 @@ struct Ctl {
   unsigned res_epoch;
   int res_arrive, res_exit, res_abort, res_late;
   unsigned res_runs;
+  unsigned res_work;  // products the resident PCG formed with this instance's matrix (wraps, as spmv_work)
 };
 
 // What the host reads back after a group of PCG iterations, one per instance of a batch.
@@ -134,7 +135,7 @@ struct InstStatus {
   int first_iters;  // iterations of the first (refinement: first sweep's) inner solve
   double err;       // sqrt(res^2 / b^2) of the finished solve
   double maxR;      // |S b|^2
-  unsigned spmv_work;  // Ctl::spmv_work
+  unsigned spmv_work, res_work;  // Ctl's
   int res_abort, res_late;  // Ctl's
   unsigned res_runs;   // Ctl::res_runs
 };

@@ -1156,7 +1156,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
           N->status = status;
           N->first = first ? 1 : 0;
         }
-        ctl->spmv_work += (unsigned)it;
+        ctl->res_work += (unsigned)it;
         ctl->res_runs += 1u;
         ctl->res_epoch = epoch + 2u + (unsigned)it;
       }

@@ -1975,6 +1975,7 @@ __global__ __launch_bounds__(kBlock) void status_kernel(Batch b, InstStatus* out
     o.ref_done = c->rs.done;
     o.first_iters = I->refine ? c->rs.first_iters : s->iters;
     o.spmv_work = c->spmv_work;
+    o.res_work = c->res_work;
     o.res_abort = c->res_abort;
     o.res_late = c->res_late;
     o.res_runs = c->res_runs;

@@ -223,7 +223,9 @@ int hobak_last_step_timing(hobak_inst* inst, double* out_ms);
  * hobak_set_kernel_sampling: every `every`-th PCG iteration of the following steps brackets its
  * SpMV launch with HIP events on the instance's stream (0 turns sampling off and clears the
  * accumulators).  A group of PCG iterations that holds a sampled launch runs uncaptured; the
- * other groups replay their graph.  hobak_kernel_stats: average duration (ms) and count of the sampled SpMV
+ * other groups replay their graph.  The resident form (HOBAK_TUNE_RESIDENT) has no such launches: a step or
+ * batch step with instances in it times one SpMV launch over all of its instances, ahead of their first
+ * solve, and results do not depend on it.  hobak_kernel_stats: average duration (ms) and count of the sampled SpMV
  * launches that did work, and the SpMV's algorithmic bytes per launch
  * nnzb * (9 s + 4) + 4 (nv + 1) + 2 * 3 s * nv  (s = bytes per real). */
 int hobak_set_kernel_sampling(hobak_inst* inst, int32_t every);
@@ -393,7 +395,9 @@ int hobak_sched_stats(hobak_sched* sched, double* out);
  * sampling was set (an instance's matrix and vectors count in the launches that streamed them,
  * as counted on the device; the workgroups of an instance whose solve has ended return at once).
  * Bytes over the average time is then the rate over all launches of the window, the samples
- * being spread evenly over them. */
+ * being spread evenly over them.  For solves in the resident form (HOBAK_TUNE_RESIDENT), which has no SpMV launches,
+ * one over the solves that start in a tick is timed ahead of them after every `every` of their iterations, and
+ * counts as `every` launches; results do not depend on it. */
 int hobak_sched_set_kernel_sampling(hobak_sched* sched, int32_t every);
 int hobak_sched_kernel_stats(hobak_sched* sched, double* spmv_avg_ms, int64_t* spmv_count,
                              double* spmv_bytes);

@@ -72,7 +72,7 @@ void resident(const Batch& b, int form, int iters) {
     c->sc[0].iters += k;
     c->sc[0].first = 0;
     if (c->sc[0].iters >= s.iters) c->sc[0].done = 1;
-    c->spmv_work += (unsigned)k;
+    c->res_work += (unsigned)k;
     c->res_runs += 1;
   }
 }
@@ -153,6 +153,7 @@ std::function<void()> stand_in(const std::string& name, void** a) {
         o.ref_done = c->rs.done;
         o.first_iters = inst(b, i)->refine ? c->rs.first_iters : c->sc[0].iters;
         o.spmv_work = c->spmv_work;
+        o.res_work = c->res_work;
         o.res_abort = c->res_abort;
         o.res_late = c->res_late;
         o.res_runs = c->res_runs;

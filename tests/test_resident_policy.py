@@ -101,3 +101,57 @@ def test_a_launch_ends_before_the_wait_of_those_behind_it(engine):
     inst = _inst(e, (10, 10, 10), iters=5000)
     inst.step(True)
     assert [int(w[3]) for w in e.log() if w[0] == "die"] == [2048] * 3
+
+
+def _two_kernel_launches(e):
+    log = e.log()
+    return [w[0] for w in log].count("sample"), [w for w in log if w[0] == "spmv"]
+
+
+@pytest.mark.parametrize("dims,precision,form", [((10, 10, 10), F64, "die"), ((40, 40, 40), F64, "device"),
+                                                 ((35, 37, 35), F32, "big")])
+def test_sampling_times_one_launch_and_leaves_the_solve_in_its_form(engine, dims, precision, form):
+    """No iterations of the two-kernel form, whose sums may round differently (every compute unit)."""
+    e = engine(update_wgs=256 if form == "big" else 512)
+    inst = _inst(e, dims, precision=precision, iters=100)
+    for every in (1, 2, 64):
+        inst.set_kernel_sampling(every)
+        inst.step(True)
+        sampled, launches = _two_kernel_launches(e)
+        assert sampled == 1 and launches == [["spmv", "1"]]
+        assert inst.kernel_stats()["spmv_count"] == 1
+        inst.set_kernel_sampling(0)
+
+
+def test_a_batch_of_both_forms_samples_the_whole_batch(engine):
+    """A sample is credited with every member's bytes, so it has to be a launch over all of them."""
+    e = engine(row_sort=0)
+    a, b = _inst(e, (10, 10, 10), iters=100), _inst(e, (26, 26, 26), iters=100, device=MISFIT, die=MISFIT)
+    for _ in range(4):
+        lib.step_batch(e.ctx, [a, b], True)  # b is in the two-kernel form from here on
+    for i in (a, b):
+        i.set_kernel_sampling(2)
+    e.log()
+    lib.step_batch(e.ctx, [a, b], True)
+    log = e.log()
+    at = [k for k, w in enumerate(log) if w[0] == "sample"]
+    assert len(at) == 1 and log[at[0] + 1] == ["spmv", "2"]
+
+
+def test_a_scheduler_samples_solves_that_start(engine):
+    e = engine()
+    insts = [_inst(e, (10, 10, 10), iters=40), _inst(e, (10, 10, 12), iters=40)]
+    sch = lib.Scheduler(e.ctx)
+    sch.set_kernel_sampling(100)
+    for k in range(10):
+        for i in insts:
+            sch.submit(i, k)
+    left = 1
+    while left:
+        _, left = sch.tick()
+    sampled, launches = _two_kernel_launches(e)
+    assert sampled == 4 and launches == [["spmv", "2"]] * 4  # after 0, 120, 240 and 360 of 400 iterations
+    row = [int(i.bsr_pattern()[0][-1]) for i in insts]
+    expect = sum(n * 76 + 4 * (i.nv + 1) + 48 * i.nv for n, i in zip(row, insts))
+    assert sch.kernel_stats()["spmv_bytes"] == expect
+    sch.close()
