@@ -1320,7 +1320,10 @@ int tick_impl(hobak_sched* S) {
   if (nsolving) {
     const Range r_pcg("hobak pcg groups");
     const int st = stream_matrix(ctx, solving_bytes) ? 1 : 0;
-    const bool compact = nsolving < M.n && solving_wgs * 100 <= (long)ctx->compact_pct * M.b[K_SPMV].total;
+    // (beside resident instances always: those on every compute unit round differently in a group, so it is not for
+    // the rest of the batch to give them one)
+    const bool compact = nsolving < M.n && (!resident.empty() ||
+                                            solving_wgs * 100 <= (long)ctx->compact_pct * M.b[K_SPMV].total);
     Plan PG;
     if (compact) TRY(plan_transient(ctx, solving, PG));
     if (graphs && !compact && (!M.chunk_exec[st] || M.chunk_k[st] != k)) {

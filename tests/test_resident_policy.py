@@ -155,3 +155,18 @@ def test_a_scheduler_samples_solves_that_start(engine):
     expect = sum(n * 76 + 4 * (i.nv + 1) + 48 * i.nv for n, i in zip(row, insts))
     assert sch.kernel_stats()["spmv_bytes"] == expect
     sch.close()
+
+
+@pytest.mark.parametrize("compact_pct", [0, 100])
+def test_groups_of_the_two_kernel_form_leave_resident_members_out(engine, compact_pct):
+    """An instance on every compute unit beside one in the two-kernel form: its sums keep their order."""
+    e = engine(update_wgs=256, compact_pct=compact_pct)
+    big = _inst(e, (35, 37, 35), precision=F32, iters=100)
+    other = _inst(e, (30, 30, 30), precision=F32, iters=100, device=MISFIT)
+    for _ in range(4):
+        lib.step_batch(e.ctx, [big, other], True)
+    e.log()
+    lib.step_batch(e.ctx, [big, other], True)
+    log = e.log()
+    before = log[:[w[0] for w in log].index("big")]  # (afterwards its solve has ended)
+    assert ["spmv", "1"] in before and ["spmv", "2"] not in before
