@@ -2296,6 +2296,7 @@ int hobak_inst_compute_fdots(hobak_inst* I, const double* velocity) {
 int hobak_inst_set_state(hobak_inst* I, const double* u, const double* v) {
   if (!I) return HOBAK_E_INVALID;
   if (I->requests) return fail(I->ctx, HOBAK_E_INVALID, "instance has a step in flight");
+  (void)hipSetDevice(I->ctx->device);
   const size_t bytes = sizeof(double) * I->dofs;
   double* stage = (double*)stage_get(I->ctx, 2 * bytes);
   if (stage) {
@@ -2321,6 +2322,7 @@ int hobak_inst_set_state(hobak_inst* I, const double* u, const double* v) {
 int hobak_inst_get_state(hobak_inst* I, double* u, double* v) {
   if (!I) return HOBAK_E_INVALID;
   hipStream_t s = I->ctx->stream;
+  (void)hipSetDevice(I->ctx->device);
   const size_t bytes = sizeof(double) * I->dofs;
   double* stage = (double*)stage_get(I->ctx, 2 * bytes);
   if (stage) {
