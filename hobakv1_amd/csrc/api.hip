@@ -1120,7 +1120,8 @@ int worse(int a, int b) {
   return b;
 }
 
-// One tick of the engine (see the file comment).  Requires an idle stream on entry; leaves it idle.
+// One tick of the engine (see the file comment).  On entry the stream holds no work that reads the arena or a plan's
+// tables, which the tick writes anew (a state on its way in may be queued: it reads neither); leaves it idle.
 template <typename T>
 int tick_impl(hobak_sched* S) {
   hobak_ctx* ctx = S->ctx;
@@ -2316,9 +2317,12 @@ int hobak_inst_set_state(hobak_inst* I, const double* u, const double* v) {
     }
     HIPCHK(I->ctx, hipStreamSynchronize(I->ctx->stream));
   }
+  // what the last step took says nothing about a new state
   for (auto& p : I->pred) p = -1;
+  I->sweeps_seen = 0;
   return HOBAK_OK;
 }
+
 int hobak_inst_get_state(hobak_inst* I, double* u, double* v) {
   if (!I) return HOBAK_E_INVALID;
   hipStream_t s = I->ctx->stream;

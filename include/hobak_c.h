@@ -171,7 +171,9 @@ int hobak_inst_set_damping(hobak_inst* inst, int32_t model, double mu);
  * velocity gradients Fdot = [v1 - v0, v2 - v0, v3 - v0] DmInv from a DOF-length host velocity,
  * or from the instance's current velocity when velocity is NULL.  Needs HOBAK_DAMPING_GREEN. */
 int hobak_inst_compute_fdots(hobak_inst* inst, const double* velocity);
-/* position() = u and velocity() = v, DOF-length host arrays; NULL leaves that vector unchanged. */
+/* position() = u and velocity() = v, DOF-length host arrays; NULL leaves that vector unchanged.
+ * hobak_inst_set_state has read the arrays when it returns, but the state may then still be on its way to the
+ * device, ahead of whatever the context does next (a device error in it is reported there). */
 int hobak_inst_set_state(hobak_inst* inst, const double* u, const double* v);
 int hobak_inst_get_state(hobak_inst* inst, double* u, double* v);
 

@@ -211,3 +211,18 @@ def test_small_sessions_do_not_wait_for_a_large_resident_one(engine):
     for run in (lambda: _serve(e, [large], 4)[0][0], lambda: (lib.step_batch(e.ctx, [large] + small, True), e.log())[1]):
         log = run()
         assert {int(w[3]) for w in log if w[0] == "device"} == {2048}
+
+
+def test_a_new_state_forgets_how_many_sweeps_the_last_step_took(engine):
+    e = engine()
+    inst = _inst(e, (10, 10, 10), precision=F32, sweeps=5)
+
+    def first_tick():
+        inst.step(True)
+        log = [w[0] for w in e.log()]
+        return log[:log.index("status")].count("die")
+
+    assert [first_tick(), first_tick()] == [2, 5]
+    inst.set_state(inst.scene.initial_u(), inst.scene.initial_v())
+    e.log()
+    assert first_tick() == 2
