@@ -678,6 +678,9 @@ size_t estimate_bytes(int nv, int nt, int nslots_est, int precision) {
   b += (size_t)nv * (9 + 18) * ts;              // minv + PCG vectors
   b += (size_t)nt * (4 * 4 + 8 + 4) + (size_t)nv * 16;  // vertex lists, element vertex lists, misc
   b += 64 * 1024;                               // records, control block, partial sums
+  // resident PCG: published words (at most this many SpMV and update workgroups); the relabelling
+  const int nq = nv / 64 + 1, nu = std::min(nv / 84 + 1, kUpdateCap);
+  b += 8 * resident_words(nq, nu) + (size_t)nv * 4;
   if (precision != HOBAK_PRECISION_FP64)        // coarse-correction partial sums, aggregate inverses
     b += ((size_t)6 * (nv / kBlock + 1) + (size_t)3 * kUpdateCap) * 8 + 2 * 256 + (size_t)9 * (nv / 21 + 1) * ts;
   return b;
@@ -1817,9 +1820,10 @@ int hobak_check_offsets(int64_t nv, int64_t nslots, int32_t precision) {
 }
 
 size_t hobak_inst_bytes_estimate(int32_t nv, int32_t nt, int32_t precision) {
-  // a Kuhn lattice has ~15 blocks per row; padding of the slices adds a few percent
+  // a Kuhn lattice has ~15 blocks per row; padding of the slices adds a few percent, and the last slice's rows
+  // (at most 64) may be all but one padding
   const size_t nnzb = (size_t)nv * 16;
-  return estimate_bytes(nv, nt, (int)(nnzb * 1.15), precision);
+  return estimate_bytes(nv, nt, (int)(nnzb * 1.15) + 64 * 16, precision);
 }
 
 int hobak_inst_create(hobak_ctx* ctx, const double* rest_xyz, int32_t nv, const int32_t* tets,
