@@ -45,6 +45,7 @@
 
 #include "../../include/hobak_c.h"
 #include "kernels.h"
+#include "share.h"
 
 using namespace hobak;
 
@@ -65,6 +66,10 @@ constexpr int kResidentIters = 2048;
 // of 5.9, and at a least of 64 or 96 iterations 3.3 or 3.6.  Not where workgroups queue for compute units: their time is
 // what a tick then takes, and launches that end early leave some idle (24 served sessions 17.8 instead of 16.5 ms).
 constexpr int kShareIters = 32;
+// What an iteration of the resident PCG takes, roughly (one die, over the device, on every compute unit; see
+// resident.hip), and the fewest iterations of a launch that ends early for another context's (share.h).
+constexpr double kDieIterUs = 5.5, kDeviceIterUs = 10.0, kBigIterUs = 29.0;
+constexpr int kTurnIters = 32;
 // Launches in a row whose workgroups did not meet after which an instance on every compute unit solves in the two-kernel
 // form: its sums round differently there, so that is the last resort.
 constexpr int kBigTries = 4;
@@ -102,6 +107,7 @@ struct hobak_ctx {
   int agg = 0;                         // reduced-precision form: spatial order and local aggregates (2: also with the coarse correction)
   int resident = kResidentIters;       // resident PCG: iterations per launch, 0 off
   int cus = 0;                         // compute units of the device
+  Claim claim;                         // this context's part of them (share_of(device))
   int join = 1;                        // resident PCG: 0 marks every instance as one whose workgroups did not meet
   Hold device_hold{64}, die_hold{16};  // the resident PCG over the device, and on one die each
   int* tickets = nullptr;              // resident PCG launches of this context's stream
@@ -155,6 +161,23 @@ int scratch_of_device(int device, void** out) {
 }  // namespace
 
 namespace {
+
+static_assert(kShareDies == kResDies, "a claim counts compute units by die");
+Share& share_of(int device) {
+  static Share* const shares = new Share[kMaxDevices];  // (never destroyed: contexts may outlive static objects)
+  return shares[device];
+}
+
+// Gives a claim back at the end of the tick that made it, whose wait its launches have passed.
+struct ClaimGuard {
+  hobak_ctx* ctx;
+  ~ClaimGuard() { release(); }
+  void release() {
+    if (!ctx->claim.live) return;
+    std::lock_guard<std::mutex> lock(share_of(ctx->device).mu);
+    ctx->claim.live = false;
+  }
+};
 
 struct Pattern {
   int nv = 0, nt = 0, nslices = 0, nslots = 0, nrows_pad = 0, nnzb = 0;
@@ -506,6 +529,7 @@ struct hobak_inst {
   Hold big_hold{64};
   unsigned runs_seen = 0;  // likewise Ctl::res_runs
   int sweeps_seen = 0;
+  int sweep_iters = 100;  // iterations of the last solve's longest sweep, roughly (only how long launches take goes by it)
 };
 
 struct hobak_sched {
@@ -1003,8 +1027,8 @@ int resident_per_die(const hobak_ctx* ctx, const std::vector<hobak_inst*>& m) {
 // as few workgroups as hold its matrix on chip (res_pack) when the batch fills the device's
 // compute units that way, and up to one per update workgroup's rows while compute units are left.
 // `die_wgs`: 0, or the most workgroups of any instance where each instance runs on one die (see
-// resident_per_die), which gives them their number.
-int resident_tables(hobak_ctx* ctx, const std::vector<hobak_inst*>& m, int die_wgs, Batch& b) {
+// resident_per_die), which gives them their number.  wgs: the workgroups of each, in the table's order.
+int resident_tables(hobak_ctx* ctx, const std::vector<hobak_inst*>& m, int die_wgs, Batch& b, std::vector<int>& wgs) {
   const int n = (int)m.size();
   long packed = 0;
   const bool big = m[0]->res_pack == kResBig;
@@ -1018,8 +1042,10 @@ int resident_tables(hobak_ctx* ctx, const std::vector<hobak_inst*>& m, int die_w
     const int per = (int)((nu + w - 1) / w);
     return (nu + per - 1) / per;  // no more than it takes at that many each
   };
+  wgs.clear();
   if (n == 1) {
-    b = Batch{nullptr, nullptr, m[0]->dev, 1, workgroups(m[0])};
+    wgs.push_back(workgroups(m[0]));
+    b = Batch{nullptr, nullptr, m[0]->dev, 1, wgs[0]};
     return HOBAK_OK;
   }
   std::vector<hobak_inst*> order = m;
@@ -1034,7 +1060,8 @@ int resident_tables(hobak_ctx* ctx, const std::vector<hobak_inst*>& m, int die_w
   bo[0] = 0;
   for (int i = 0; i < n; i++) {
     hp[i] = order[i]->dev;
-    bo[i + 1] = bo[i] + workgroups(order[i]);
+    wgs.push_back(workgroups(order[i]));
+    bo[i + 1] = bo[i] + wgs[i];
   }
   b = Batch{(const InstDev* const*)dev, (const int*)(dev + tab), nullptr, n, bo[n]};
   HIPCHK(ctx, hipMemcpyAsync(dev, host, need, hipMemcpyHostToDevice, ctx->stream));
@@ -1249,6 +1276,7 @@ int tick_impl(hobak_sched* S) {
   //    workgroups; below that, over a table of the solving instances only, launched directly, so
   //    that the workgroups of finished instances are not dispatched just to return.
   bool ran = false;
+  ClaimGuard claimed{ctx};
   int m = ctx->max_chunks;
   int nsolving = 0;
   double solving_bytes = 0.0;
@@ -1371,8 +1399,39 @@ int tick_impl(hobak_sched* S) {
       if (I->res_pack != kResBig) rest.push_back(I);
     if (!rest.empty()) die_wgs = resident_per_die(ctx, rest);
     if (die_wgs && !ctx->die_hold.pass()) die_wgs = 0;
-    if (!rest.empty()) TRY(resident_tables(ctx, rest, die_wgs, rb));
-    if (!resident_big.empty()) TRY(resident_tables(ctx, resident_big, 0, rbig));
+    std::vector<int> each;
+    if (!resident_big.empty()) TRY(resident_tables(ctx, resident_big, 0, rbig, each));
+    if (!rest.empty()) TRY(resident_tables(ctx, rest, die_wgs, rb, each));
+    // this context's part of the device (share.h): on the emptiest dies, else over the device if that has room,
+    // else on what it would take alone, after the others
+    Share& share = share_of(ctx->device);
+    const int per_die = std::max(1, ctx->cus / kResDies);
+    const std::lock_guard<std::mutex> lock(share.mu);
+    int use[kResDies] = {}, first_die = 0;
+    auto over_all = [&](int total) {
+      for (auto& u : use) u = std::max(u, std::min(per_die, (total + kResDies - 1) / kResDies));
+    };
+    if (die_wgs) {
+      first_die = share.first_die(&ctx->claim, each.data(), (int)each.size(), per_die);
+      if (first_die < 0) {
+        Batch over{};
+        std::vector<int> each_over;
+        TRY(resident_tables(ctx, rest, 0, over, each_over));
+        over_all(over.total);
+        if (share.fits(&ctx->claim, use, per_die)) {
+          rb = over;
+          die_wgs = 0;
+        } else {
+          first_die = 0;
+        }
+        std::fill(std::begin(use), std::end(use), 0);
+      }
+    }
+    if (die_wgs)
+      for (size_t i = 0; i < each.size(); i++) use[(first_die + i) % kResDies] += each[i];
+    else
+      over_all(rb.total);
+    if (rbig.n) over_all(ctx->cus);
     Plan PR;
     const bool all = (int)resident.size() == M.n;
     if (!all) TRY(plan_transient(ctx, resident, PR));
@@ -1381,13 +1440,29 @@ int tick_impl(hobak_sched* S) {
       const int share = std::max(kShareIters, (shortest / sweeps * 5 / 4 + 9) & ~1);
       if (longest / sweeps > 2 * share) iters = std::min(iters, share);
     }
+    const double now_s = std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
+    const double iter_us = rbig.n ? kBigIterUs : die_wgs ? kDieIterUs : kDeviceIterUs * (1 + rb.total / ctx->cus);
+    int sweep_iters = 0;
+    for (auto* I : resident) sweep_iters = std::max(sweep_iters, I->sweep_iters);
+    const double turn_ms = share.turn_ms(&ctx->claim, use, per_die, now_s);
+    ctx->claim.ms = 1e-3 * iter_us * sweeps * std::min(iters, sweep_iters);
+    if (turn_ms > 0.0 && ctx->claim.ms > 1.25 * turn_ms) {
+      iters = std::min(iters, std::max(kTurnIters, (int)(1e3 * turn_ms / iter_us) & ~1));
+      if (sweep_iters > iters) sweeps = 1;
+    }
+    if (!share.fits(&ctx->claim, use, per_die))
+      for (const Claim* c : share.claims)
+        if (c != &ctx->claim && c->live) HIPCHK(ctx, hipStreamWaitEvent(s, (hipEvent_t)c->done, 0));
+    std::copy(use, use + kResDies, ctx->claim.use);
+    ctx->claim.last_s = now_s;
+    ctx->claim.live = true;
     const int wgs = ctx->join ? die_wgs : std::max(1, die_wgs - 1);
     for (int j = 0; j < sweeps; j++) {
       if (!ctx->join)
         for (auto* I : resident)
           HIPCHK(ctx, hipMemcpyAsync(&I->h.ctl->res_arrive, &kResLate, sizeof(int), hipMemcpyHostToDevice, s));
       if (die_wgs)
-        HIPCHK(ctx, launch_cg_resident_die<T>(rb, M.shift, M.groups, wgs, ctx->tickets, iters, s));
+        HIPCHK(ctx, launch_cg_resident_die<T>(rb, M.shift, M.groups, first_die, wgs, ctx->tickets, iters, s));
       else
         HIPCHK(ctx, launch_cg_resident<T>(rb, M.shift, M.groups, false, ctx->tickets, iters, s));
       if (rbig.n) HIPCHK(ctx, launch_cg_resident<T>(rbig, M.shift, M.groups, true, ctx->tickets, iters, s));
@@ -1395,9 +1470,11 @@ int tick_impl(hobak_sched* S) {
     }
     S->stat[1] += sweeps;
     S->stat[10] += sweeps;
-    ran = true;
+    HIPCHK(ctx, hipEventRecord(ctx->ev[5], s));
+  } else if (ran) {
+    HIPCHK(ctx, hipEventRecord(ctx->ev[5], s));
   }
-  if (ran) HIPCHK(ctx, hipEventRecord(ctx->ev[5], s));
+  ran |= !resident.empty();
 
   S->stat[1] += nsolving ? m : 0;
   // 5. statuses
@@ -1406,6 +1483,7 @@ int tick_impl(hobak_sched* S) {
     HIPCHK(ctx, launch_status(M.b[K_ONE], M.status_dev, s));
     HIPCHK(ctx, hipMemcpyAsync(M.status_host, M.status_dev, sizeof(InstStatus) * M.n, hipMemcpyDeviceToHost, s));
     HIPCHK(ctx, hipStreamSynchronize(s));
+    claimed.release();
   }
   // algorithmic SpMV bytes of this tick: each member's matrix and vectors once per launch that
   // streamed them (counted on the device; launches after a member's solve ended read nothing)
@@ -1540,6 +1618,7 @@ int tick_impl(hobak_sched* S) {
       r.st.status = worse(r.st.status, code);
       r.I->pred[nk] = iters;
       r.I->sweeps_seen = refine ? q.sweeps : 0;
+      r.I->sweep_iters = refine ? q.first_iters : iters;
       if (nk == 0) r.I->first_iters = q.first_iters;
       r.stage = 2;
       S->stat[6] += 1;
@@ -1752,7 +1831,8 @@ int hobak_ctx_create(int device, size_t hbm_budget_bytes, hobak_ctx** out) {
   if (!out) return HOBAK_E_INVALID;
   *out = nullptr;
   int n = 0;
-  if (hipGetDeviceCount(&n) != hipSuccess || n <= device || device < 0) return HOBAK_E_NODEVICE;
+  if (hipGetDeviceCount(&n) != hipSuccess || n <= device || device < 0 || device >= kMaxDevices)
+    return HOBAK_E_NODEVICE;
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, device) != hipSuccess) return HOBAK_E_NODEVICE;
   if (std::strncmp(prop.gcnArchName, "gfx950", 6) != 0) return HOBAK_E_NODEVICE;
@@ -1768,11 +1848,16 @@ int hobak_ctx_create(int device, size_t hbm_budget_bytes, hobak_ctx** out) {
   }
   bool ok = true;
   for (auto& e : ctx->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
+  ctx->claim.done = ctx->ev[5];
   ok = ok && hipMalloc((void**)&ctx->tickets, kResTickets * sizeof(int)) == hipSuccess &&
        hipMemsetAsync(ctx->tickets, 0, kResTickets * sizeof(int), ctx->stream) == hipSuccess;
   if (!ok || arena_ensure(ctx, 1 << 20) != HOBAK_OK || scratch_of_device(device, &ctx->scratch) != HOBAK_OK) {
     hobak_ctx_destroy(ctx);
     return HOBAK_E_HIP;
+  }
+  {
+    std::lock_guard<std::mutex> lock(share_of(device).mu);
+    share_of(device).claims.push_back(&ctx->claim);
   }
   *out = ctx;
   return HOBAK_OK;
@@ -1786,6 +1871,11 @@ void hobak_ctx_destroy(hobak_ctx* ctx) {
   for (auto* S : ss) hobak_sched_destroy(S);
   std::vector<hobak_inst*> all(ctx->insts.begin(), ctx->insts.end());
   for (auto* I : all) hobak_inst_destroy(I);
+  {
+    Share& share = share_of(ctx->device);
+    std::lock_guard<std::mutex> lock(share.mu);
+    share.claims.erase(std::remove(share.claims.begin(), share.claims.end(), &ctx->claim), share.claims.end());
+  }
   for (auto* P : ctx->plans) plan_free(P);
   ctx->plans.clear();
   if (ctx->arena_dev) (void)hipFree(ctx->arena_dev);

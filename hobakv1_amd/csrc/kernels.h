@@ -367,10 +367,12 @@ constexpr int kResDies = 8, kResDieWgs = 32, kResTickets = 1 + kResDies;
 constexpr int kResLate = 1 << 29;  // of Ctl::res_arrive: the workgroups did not meet, and leave the instance untouched
 template <typename T>
 hipError_t launch_cg_resident(const Batch& b, int shift, int groups, bool big, int* tickets, int iters, hipStream_t s);
-// The same for at most kResDies instances, each on the workgroups of one die (at most `wgs`, the most any takes),
+// The same for at most kResDies instances, instance i on the workgroups of die `first` + i mod kResDies (at most `wgs`,
+// the most any takes),
 // which exchange through its L2.  An instance whose die gets too few of them is left untouched.
 template <typename T>
-hipError_t launch_cg_resident_die(const Batch& b, int shift, int groups, int wgs, int* tickets, int iters, hipStream_t s);
+hipError_t launch_cg_resident_die(const Batch& b, int shift, int groups, int first, int wgs, int* tickets, int iters,
+                                  hipStream_t s);
 // Whether the resident PCG has a variant for this slice height, update layout and row count.
 bool resident_layout(int shift, int groups, int nb_upd);
 // The same of the form for more rows than the update workgroups cover in one run each, on `wgs` workgroups.

@@ -1209,15 +1209,15 @@ __device__ __forceinline__ const __attribute__((address_space(4))) DieArgs* late
   return a;
 }
 
-// The same for up to eight instances, instance i on die i alone: the grid holds as many workgroups for each die as
+// The same for up to eight instances, instance i on die `first` + i (mod 8) alone: the grid holds as many workgroups for each die as
 // the largest instance takes, and those past an instance's, or of a die without one, leave at once.
 // tickets: [0] workgroups done, [1 + i] instance i's next ticket; all zero between launches.
 template <typename T, int R, int H>
 __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void cg_resident_die_kernel(
-    Batch b, int* tickets, int iters) {
+    Batch b, int* tickets, int iters, int first) {
   extern __shared__ __align__(16) char lds[];
   __shared__ int sh_ticket;
-  const int i = __builtin_amdgcn_readfirstlane(die_of_wave());
+  const int i = __builtin_amdgcn_readfirstlane((die_of_wave() - first) & (kResDies - 1));
   if (i < b.n) {
     const int W = uniform_i(b.n == 1 ? b.total : gbl(b.boff)[i + 1] - gbl(b.boff)[i]);
     if (threadIdx.x == 0)
@@ -1260,20 +1260,20 @@ hipError_t resident_rh(const Batch& b, int* tickets, int iters, hipStream_t s) {
   return hipGetLastError();
 }
 template <typename T, int R, int H>
-hipError_t resident_die(const Batch& b, int wgs, int* tickets, int iters, hipStream_t s) {
+hipError_t resident_die(const Batch& b, int first, int wgs, int* tickets, int iters, hipStream_t s) {
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&cg_resident_die_kernel<T, R, H>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, kResLds);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((cg_resident_die_kernel<T, R, H>), dim3(kResDies * wgs), dim3(kResThreads), kResLds, s, b, tickets,
-                     iters);
+                     iters, first);
   return hipGetLastError();
 }
 template <typename T, int R>
-hipError_t resident_die_r(const Batch& b, int shift, int wgs, int* tickets, int iters, hipStream_t s) {
+hipError_t resident_die_r(const Batch& b, int shift, int first, int wgs, int* tickets, int iters, hipStream_t s) {
   switch (shift) {
-    case 4: return resident_die<T, R, 16>(b, wgs, tickets, iters, s);
-    case 5: return resident_die<T, R, 32>(b, wgs, tickets, iters, s);
-    case 6: return resident_die<T, R, 64>(b, wgs, tickets, iters, s);
+    case 4: return resident_die<T, R, 16>(b, first, wgs, tickets, iters, s);
+    case 5: return resident_die<T, R, 32>(b, first, wgs, tickets, iters, s);
+    case 6: return resident_die<T, R, 64>(b, first, wgs, tickets, iters, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1315,16 +1315,17 @@ hipError_t launch_cg_resident(const Batch& b, int shift, int groups, bool big, i
   }
 }
 template <typename T>
-hipError_t launch_cg_resident_die(const Batch& b, int shift, int groups, int wgs, int* tickets, int iters, hipStream_t s) {
+hipError_t launch_cg_resident_die(const Batch& b, int shift, int groups, int first, int wgs, int* tickets, int iters,
+                                  hipStream_t s) {
   if (b.n < 1 || b.n > kResDies || wgs < 1) return hipErrorInvalidValue;
   switch (groups) {
-    case 2: return resident_die_r<T, 2>(b, shift, wgs, tickets, iters, s);
-    case 4: return resident_die_r<T, 4>(b, shift, wgs, tickets, iters, s);
+    case 2: return resident_die_r<T, 2>(b, shift, first, wgs, tickets, iters, s);
+    case 4: return resident_die_r<T, 4>(b, shift, first, wgs, tickets, iters, s);
     default: return hipErrorInvalidValue;
   }
 }
-template hipError_t launch_cg_resident_die<double>(const Batch&, int, int, int, int*, int, hipStream_t);
-template hipError_t launch_cg_resident_die<float>(const Batch&, int, int, int, int*, int, hipStream_t);
+template hipError_t launch_cg_resident_die<double>(const Batch&, int, int, int, int, int*, int, hipStream_t);
+template hipError_t launch_cg_resident_die<float>(const Batch&, int, int, int, int, int*, int, hipStream_t);
 template hipError_t launch_cg_resident<double>(const Batch&, int, int, bool, int*, int, hipStream_t);
 template hipError_t launch_cg_resident<float>(const Batch&, int, int, bool, int*, int, hipStream_t);
 

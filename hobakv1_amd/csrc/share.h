@@ -1,0 +1,82 @@
+// How the contexts of one process share a device's compute units in the resident PCG.
+//
+// The workgroups of a resident launch wait for each other, so two launches that each hold part of the compute units they
+// need would both wait until they give up (0.2 s each time; four contexts of 303,242, 68,921, 9,261 and 1,331
+// vertices stepping in four threads took up to 1.4 s for a step).  A context therefore claims the compute units of
+// its launches, by die, while they are queued or running.  Where they do not fit beside those of others its
+// stream first waits for those: claims are made one at a time, so a launch only ever waits for earlier ones.
+//
+// A launch holds its compute units for a whole solve, which a context with a small instance would wait for each
+// time.  Where contexts that were here lately do not fit together, one whose launches take longer than another's
+// therefore takes turns of about the other's length.
+#pragma once
+#include <algorithm>
+#include <mutex>
+#include <vector>
+
+namespace hobak {
+
+constexpr int kShareDies = 8;
+
+// One context's part of a device.
+struct Claim {
+  void* done = nullptr;      // the event behind its last launch
+  int use[kShareDies] = {};  // compute units on each die
+  double ms = 0.0;           // what its launches take, roughly
+  double last_s = -1e9;      // when it was made
+  bool live = false;         // its launches are queued or running
+};
+
+constexpr double kShareLatelyS = 0.05;  // a context that claimed within this time is expected again
+constexpr double kShareTurnMs = 2.0;    // the shortest turn: a launch's set-up and the host's part take 0.1 ms
+
+struct Share {
+  std::mutex mu;               // held while a claim is made and its launches are queued
+  std::vector<Claim*> claims;  // of every context on the device
+
+  // Whether `use` fits beside the live claims of others (on `per_die` compute units a die).
+  bool fits(const Claim* mine, const int (&use)[kShareDies], int per_die) const { return room(mine, use, per_die, -1.0); }
+  // The longest a turn of `mine` should take, given contexts that were here lately: no limit (0) where it fits beside
+  // them, else as long as the shortest of theirs.
+  double turn_ms(const Claim* mine, const int (&use)[kShareDies], int per_die, double now_s) const {
+    if (room(mine, use, per_die, now_s)) return 0.0;
+    double ms = 1e30;
+    for (const Claim* c : claims)
+      if (c != mine && lately(*c, now_s)) ms = std::min(ms, c->ms);
+    return std::max(ms, kShareTurnMs);
+  }
+  // The die on which to put the first of `n` instances that take wgs[i] compute units of successive dies: where
+  // the fullest die is emptiest; -1 if they fit on none.
+  int first_die(const Claim* mine, const int* wgs, int n, int per_die) const {
+    int best = -1, least = per_die + 1;
+    for (int first = 0; first < kShareDies; first++) {
+      int use[kShareDies] = {};
+      for (int i = 0; i < n; i++) use[(first + i) % kShareDies] += wgs[i];
+      int full = 0;
+      for (int d = 0; d < kShareDies; d++) {
+        for (const Claim* c : claims)
+          if (c != mine && c->live) use[d] += c->use[d];
+        full = std::max(full, use[d]);
+      }
+      if (full < least) {
+        least = full;
+        best = first;
+      }
+    }
+    return best;
+  }
+
+ private:
+  static bool lately(const Claim& c, double now_s) { return c.live || now_s - c.last_s < kShareLatelyS; }
+  bool room(const Claim* mine, const int (&use)[kShareDies], int per_die, double now_s) const {
+    for (int d = 0; d < kShareDies; d++) {
+      int sum = use[d];
+      for (const Claim* c : claims)
+        if (c != mine && (now_s < 0.0 ? c->live : lately(*c, now_s))) sum += c->use[d];
+      if (sum > per_die) return false;
+    }
+    return true;
+  }
+};
+
+}  // namespace hobak

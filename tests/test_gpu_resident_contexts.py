@@ -1,0 +1,55 @@
+"""Contexts of one process stepping in threads of their own, whose resident launches together need more compute units than
+the device has: none of them waits in vain, and each ends bitwise where it ends alone."""
+import threading
+
+import numpy as np
+import pytest
+
+from hobakv1_amd import lib, scenes
+
+pytestmark = pytest.mark.gpu
+
+F64, F32 = lib.PRECISION_FP64, lib.PRECISION_FP32_REFINE
+
+
+class _Program:
+    def __init__(self, dims, precision, steps, **tuning):
+        self.ctx = lib.Context(0, precision="fp64" if precision == F64 else "fp32")
+        self.ctx.set_tuning(**tuning)
+        self.scene = scenes.lattice_scene(dims, seed=3, stretch_velocity=True)
+        self.inst = lib.Instance(self.ctx, self.scene, precision=precision)
+        self.steps = steps
+
+    def run(self):
+        self.inst.set_state(self.scene.initial_u(), self.scene.initial_v())
+        for _ in range(self.steps):
+            self.inst.step(True)
+        self.end = self.inst.state()
+
+    def close(self):
+        self.inst.close()
+        self.ctx.close()
+
+
+@pytest.mark.parametrize("programs", [
+    [((35, 37, 35), F32, 30, dict(update_wgs=256)), ((30, 30, 30), F64, 40, {}), ((20, 20, 20), F64, 100, {}),
+     ((10, 10, 10), F32, 200, {})],
+    [((36, 36, 36), F64, 40, {}), ((36, 36, 35), F64, 40, {}), ((35, 36, 36), F32, 40, {})],
+    [((20, 20, 20), F64, 60, {})] * 2 + [((10, 10, 10), F64, 150, {})] * 4])
+def test_contexts_in_threads(programs):
+    print(f"  {programs}", flush=True)
+    ps = [_Program(d, prec, n, **t) for d, prec, n, t in programs]
+    for p in ps:
+        p.run()
+    alone = [p.end for p in ps]
+    threads = [threading.Thread(target=p.run) for p in ps]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    stats = [p.ctx.resident_stats() for p in ps]
+    for p, (u, v) in zip(ps, alone):
+        assert np.array_equal(p.end[0], u) and np.array_equal(p.end[1], v)
+    for p in ps:
+        p.close()
+    assert all(s["late"] == 0 and s["aborted"] == 0 for s in stats), stats

@@ -1,0 +1,59 @@
+"""How contexts share a device's compute units in the resident PCG (csrc/share.h), on the CPU."""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SOURCE = r"""
+#include "share.h"
+#include <cstdio>
+#include <cstdlib>
+using namespace hobak;
+#define CHECK(c) do { if (!(c)) { std::printf("line %d: %s\n", __LINE__, #c); std::exit(1); } } while (0)
+struct Use { int u[kShareDies]; };
+Use all(int n) { Use x; for (int& v : x.u) v = n; return x; }
+Use one(int d, int n) { Use x = all(0); x.u[d] = n; return x; }
+void hold(Claim& c, Use x, double ms, double at) { std::copy(x.u, x.u + kShareDies, c.use); c.ms = ms; c.last_s = at; c.live = true; }
+int main() {
+  Share s;
+  Claim a, b, c;
+  s.claims = {&a, &b, &c};
+  // nobody here: room for everything, no turns
+  CHECK(s.fits(&a, all(32).u, 32) && !s.fits(&a, all(33).u, 32));
+  CHECK(s.turn_ms(&a, all(32).u, 32, 10.0) == 0.0);
+  int w[2] = {28, 8};
+  CHECK(s.first_die(&a, w, 2, 32) == 0);
+  // b holds 26 compute units of each die: 6 are left
+  hold(b, all(26), 4.7, 10.0);
+  CHECK(s.fits(&a, all(6).u, 32) && !s.fits(&a, one(3, 7).u, 32));
+  CHECK(s.first_die(&a, w, 2, 32) == -1);
+  // its own claim is not in a context's way
+  CHECK(s.fits(&b, all(32).u, 32));
+  // no turns where both fit, turns of the other's length where not, of 2 ms at least
+  CHECK(s.turn_ms(&a, all(6).u, 32, 10.0) == 0.0);
+  CHECK(s.turn_ms(&a, all(32).u, 32, 10.0) == 4.7);
+  hold(c, one(0, 8), 0.5, 10.0);
+  CHECK(s.turn_ms(&a, all(32).u, 32, 10.0) == kShareTurnMs);
+  // a claim given back leaves room at once, and its context is expected again for a while
+  b.live = c.live = false;
+  CHECK(s.fits(&a, all(32).u, 32));
+  CHECK(s.turn_ms(&a, all(32).u, 32, 10.01) == kShareTurnMs && s.turn_ms(&a, all(32).u, 32, 11.0) == 0.0);
+  // the emptiest dies
+  hold(b, one(0, 28), 1.0, 12.0);
+  CHECK(s.first_die(&a, w, 1, 32) == 1);
+  hold(c, one(1, 28), 1.0, 12.0);
+  CHECK(s.first_die(&a, w, 2, 32) == 2);
+  int v[8] = {4, 4, 4, 4, 4, 4, 4, 4}, x[8] = {5, 5, 5, 5, 5, 5, 5, 5};
+  CHECK(s.first_die(&a, v, 8, 32) == 0 && s.first_die(&a, x, 8, 32) == -1);
+  return 0;
+}
+"""
+
+
+def test_claims(tmp_path):
+    src, exe = tmp_path / "share.cpp", tmp_path / "share"
+    src.write_text(SOURCE)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", os.path.join(ROOT, "hobakv1_amd", "csrc"), str(src),
+                    "-o", str(exe), "-pthread"], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout
