@@ -1444,17 +1444,18 @@ int tick_impl(hobak_sched* S) {
     const double iter_us = rbig.n ? kBigIterUs : die_wgs ? kDieIterUs : kDeviceIterUs * (1 + rb.total / ctx->cus);
     int sweep_iters = 0;
     for (auto* I : resident) sweep_iters = std::max(sweep_iters, I->sweep_iters);
-    const double turn_ms = share.turn_ms(&ctx->claim, use, per_die, now_s);
+    const bool alone = share.fits(&ctx->claim, use, per_die);
+    if (!alone) share.meets(&ctx->claim, now_s);
+    const double turn_ms = share.turn_ms(&ctx->claim, now_s);
     ctx->claim.ms = 1e-3 * iter_us * sweeps * std::min(iters, sweep_iters);
     if (turn_ms > 0.0 && ctx->claim.ms > 1.25 * turn_ms) {
       iters = std::min(iters, std::max(kTurnIters, (int)(1e3 * turn_ms / iter_us) & ~1));
       if (sweep_iters > iters) sweeps = 1;
     }
-    if (!share.fits(&ctx->claim, use, per_die))
+    if (!alone)
       for (const Claim* c : share.claims)
         if (c != &ctx->claim && c->live) HIPCHK(ctx, hipStreamWaitEvent(s, (hipEvent_t)c->done, 0));
     std::copy(use, use + kResDies, ctx->claim.use);
-    ctx->claim.last_s = now_s;
     ctx->claim.live = true;
     const int wgs = ctx->join ? die_wgs : std::max(1, die_wgs - 1);
     for (int j = 0; j < sweeps; j++) {

@@ -7,8 +7,8 @@
 // stream first waits for those: claims are made one at a time, so a launch only ever waits for earlier ones.
 //
 // A launch holds its compute units for a whole solve, which a context with a small instance would wait for each
-// time.  Where contexts that were here lately do not fit together, one whose launches take longer than another's
-// therefore takes turns of about the other's length.
+// time.  Of contexts that were in each other's way lately, one whose launches take longer than another's therefore
+// takes turns of about the other's length.  (Contexts that one thread uses in turn never are.)
 #pragma once
 #include <algorithm>
 #include <mutex>
@@ -23,11 +23,11 @@ struct Claim {
   void* done = nullptr;      // the event behind its last launch
   int use[kShareDies] = {};  // compute units on each die
   double ms = 0.0;           // what its launches take, roughly
-  double last_s = -1e9;      // when it was made
+  double met_s = -1e9;       // when it last did not fit beside another, or another beside it
   bool live = false;         // its launches are queued or running
 };
 
-constexpr double kShareLatelyS = 0.05;  // a context that claimed within this time is expected again
+constexpr double kShareLatelyS = 0.05;  // contexts that were in each other's way within this time are expected to be again
 constexpr double kShareTurnMs = 2.0;    // the shortest turn: a launch's set-up and the host's part take 0.1 ms
 
 struct Share {
@@ -35,15 +35,27 @@ struct Share {
   std::vector<Claim*> claims;  // of every context on the device
 
   // Whether `use` fits beside the live claims of others (on `per_die` compute units a die).
-  bool fits(const Claim* mine, const int (&use)[kShareDies], int per_die) const { return room(mine, use, per_die, -1.0); }
-  // The longest a turn of `mine` should take, given contexts that were here lately: no limit (0) where it fits beside
-  // them, else as long as the shortest of theirs.
-  double turn_ms(const Claim* mine, const int (&use)[kShareDies], int per_die, double now_s) const {
-    if (room(mine, use, per_die, now_s)) return 0.0;
-    double ms = 1e30;
-    for (const Claim* c : claims)
-      if (c != mine && lately(*c, now_s)) ms = std::min(ms, c->ms);
-    return std::max(ms, kShareTurnMs);
+  bool fits(const Claim* mine, const int (&use)[kShareDies], int per_die) const {
+    for (int d = 0; d < kShareDies; d++) {
+      int sum = use[d];
+      for (const Claim* c : claims)
+        if (c != mine && c->live) sum += c->use[d];
+      if (sum > per_die) return false;
+    }
+    return true;
+  }
+  // `mine` does not fit beside the live claims of others.
+  void meets(Claim* mine, double now_s) {
+    for (Claim* c : claims)
+      if (c == mine || c->live) c->met_s = now_s;
+  }
+  // The longest a turn of `mine` should take: no limit (0), or as long as the shortest of the others it met.
+  double turn_ms(const Claim* mine, double now_s) const {
+    double ms = 0.0;
+    if (now_s - mine->met_s < kShareLatelyS)
+      for (const Claim* c : claims)
+        if (c != mine && now_s - c->met_s < kShareLatelyS) ms = ms > 0.0 ? std::min(ms, c->ms) : c->ms;
+    return ms > 0.0 ? std::max(ms, kShareTurnMs) : 0.0;
   }
   // The die on which to put the first of `n` instances that take wgs[i] compute units of successive dies: where
   // the fullest die is emptiest; -1 if they fit on none.
@@ -64,18 +76,6 @@ struct Share {
       }
     }
     return best;
-  }
-
- private:
-  static bool lately(const Claim& c, double now_s) { return c.live || now_s - c.last_s < kShareLatelyS; }
-  bool room(const Claim* mine, const int (&use)[kShareDies], int per_die, double now_s) const {
-    for (int d = 0; d < kShareDies; d++) {
-      int sum = use[d];
-      for (const Claim* c : claims)
-        if (c != mine && (now_s < 0.0 ? c->live : lately(*c, now_s))) sum += c->use[d];
-      if (sum > per_die) return false;
-    }
-    return true;
   }
 };
 

@@ -13,35 +13,41 @@ using namespace hobak;
 struct Use { int u[kShareDies]; };
 Use all(int n) { Use x; for (int& v : x.u) v = n; return x; }
 Use one(int d, int n) { Use x = all(0); x.u[d] = n; return x; }
-void hold(Claim& c, Use x, double ms, double at) { std::copy(x.u, x.u + kShareDies, c.use); c.ms = ms; c.last_s = at; c.live = true; }
+void hold(Claim& c, Use x, double ms) { std::copy(x.u, x.u + kShareDies, c.use); c.ms = ms; c.live = true; }
 int main() {
   Share s;
   Claim a, b, c;
   s.claims = {&a, &b, &c};
   // nobody here: room for everything, no turns
   CHECK(s.fits(&a, all(32).u, 32) && !s.fits(&a, all(33).u, 32));
-  CHECK(s.turn_ms(&a, all(32).u, 32, 10.0) == 0.0);
+  CHECK(s.turn_ms(&a, 10.0) == 0.0);
   int w[2] = {28, 8};
   CHECK(s.first_die(&a, w, 2, 32) == 0);
   // b holds 26 compute units of each die: 6 are left
-  hold(b, all(26), 4.7, 10.0);
+  hold(b, all(26), 4.7);
   CHECK(s.fits(&a, all(6).u, 32) && !s.fits(&a, one(3, 7).u, 32));
   CHECK(s.first_die(&a, w, 2, 32) == -1);
   // its own claim is not in a context's way
   CHECK(s.fits(&b, all(32).u, 32));
-  // no turns where both fit, turns of the other's length where not, of 2 ms at least
-  CHECK(s.turn_ms(&a, all(6).u, 32, 10.0) == 0.0);
-  CHECK(s.turn_ms(&a, all(32).u, 32, 10.0) == 4.7);
-  hold(c, one(0, 8), 0.5, 10.0);
-  CHECK(s.turn_ms(&a, all(32).u, 32, 10.0) == kShareTurnMs);
-  // a claim given back leaves room at once, and its context is expected again for a while
+  // contexts that met take turns of the other's length, for a while
+  CHECK(s.turn_ms(&a, 10.0) == 0.0);
+  a.ms = 14.0;
+  s.meets(&a, 10.0);
+  CHECK(s.turn_ms(&a, 10.0) == 4.7 && s.turn_ms(&b, 10.01) == 14.0 && s.turn_ms(&c, 10.0) == 0.0);
+  CHECK(s.turn_ms(&a, 11.0) == 0.0 && s.turn_ms(&b, 11.0) == 0.0);
+  // of 2 ms at least
+  hold(c, one(0, 8), 0.5);
+  s.meets(&a, 12.0);
+  CHECK(s.turn_ms(&a, 12.0) == kShareTurnMs && s.turn_ms(&b, 12.0) == kShareTurnMs && s.turn_ms(&c, 12.0) == 4.7);
+  // a claim given back leaves room at once; contexts used in turn do not meet
   b.live = c.live = false;
   CHECK(s.fits(&a, all(32).u, 32));
-  CHECK(s.turn_ms(&a, all(32).u, 32, 10.01) == kShareTurnMs && s.turn_ms(&a, all(32).u, 32, 11.0) == 0.0);
+  s.meets(&a, 20.0);
+  CHECK(s.turn_ms(&a, 20.0) == 0.0 && s.turn_ms(&b, 20.0) == 0.0);
   // the emptiest dies
-  hold(b, one(0, 28), 1.0, 12.0);
+  hold(b, one(0, 28), 1.0);
   CHECK(s.first_die(&a, w, 1, 32) == 1);
-  hold(c, one(1, 28), 1.0, 12.0);
+  hold(c, one(1, 28), 1.0);
   CHECK(s.first_die(&a, w, 2, 32) == 2);
   int v[8] = {4, 4, 4, 4, 4, 4, 4, 4}, x[8] = {5, 5, 5, 5, 5, 5, 5, 5};
   CHECK(s.first_die(&a, v, 8, 32) == 0 && s.first_die(&a, x, 8, 32) == -1);
