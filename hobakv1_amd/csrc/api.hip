@@ -59,13 +59,6 @@ constexpr int kResBig = 1 << 20;      // hobak_inst::res_pack of an instance on 
 // tuning key allows: 2,048 iterations of up to 40 us stay well below the time that the workgroups of an instance behind
 // them wait for each other.
 constexpr int kResidentIters = 2048;
-// A served session waits for the tick that others solve in, so a scheduler's launches end about when the solve closest to
-// finishing does (a quarter past its iterations in the last step), after this many iterations at least, where
-// others would go on for more than twice as long.  Each launch loads the matrices anew, 40 us: beside a 40^3
-// session (FP32, 480 iterations, 7.1 ms instead of 5.9 alone in its launches) eight of 6^3 take 2.6 ms a step instead
-// of 5.9, and at a least of 64 or 96 iterations 3.3 or 3.6.  Not where workgroups queue for compute units: their time is
-// what a tick then takes, and launches that end early leave some idle (24 served sessions 17.8 instead of 16.5 ms).
-constexpr int kShareIters = 32;
 // What an iteration of the resident PCG takes, roughly (one die, over the device, on every compute unit; see
 // resident.hip), and the fewest iterations of a launch that ends early for another context's (share.h).
 constexpr double kDieIterUs = 5.5, kDeviceIterUs = 10.0, kBigIterUs = 29.0;
@@ -1270,10 +1263,13 @@ int tick_impl(hobak_sched* S) {
   }
 
   // 4. groups of PCG iterations: as many as the solving instance closest to finishing is
-  //    predicted to need (from its last step), at least one; in a scheduler that requests go on arriving at, one that
-  //    completes in this tick counts too, as its next request would wait.  They run over the member set (one
-  //    captured graph) while the solving instances hold more than compact_pct percent of its SpMV
-  //    workgroups; below that, over a table of the solving instances only, launched directly, so
+  //    predicted to need (from its last step), at least one; in a scheduler that requests go on arriving at, resident
+  //    instances and one that completes in this tick count too, as their next requests would wait.  (Resident
+  //    solves go on to their end: ending a launch early for the shortest takes eight 6^3 sessions beside one of
+  //    40^3 from 5.9 to 2.6 ms a step, but 40^3 itself from 5.9 to 7.1, and 4 to 16 uneven sessions with three
+  //    requests each 6% to 25% longer in all.  HOBAK_TUNE_RESIDENT sets shorter launches where that is wanted.)
+  //    They run over the member set (one captured graph) while the solving instances hold more than compact_pct
+  //    percent of its SpMV workgroups; below that, over a table of the solving instances only, launched directly, so
   //    that the workgroups of finished instances are not dispatched just to return.
   bool ran = false;
   ClaimGuard claimed{ctx};
@@ -1310,21 +1306,14 @@ int tick_impl(hobak_sched* S) {
     resident.push_back(r.I);
     if (r.I->res_pack == kResBig) resident_big.push_back(r.I);
   }
-  int sweeps = 1, die_wgs = 0, shortest = INT32_MAX, longest = 0;
+  int sweeps = 1, die_wgs = 0;
   for (size_t i = 0; i < S->active.size(); i++) {
     auto& r = S->active[i];
     const bool res = resides[i] != 0;
     const int p = r.I->pred[r.newton_k], left = p > 0 ? std::max(p - r.done_iters, 0) : 0;
-    if (!S->ephemeral && r.stage == 3 && p > 0) {
-      shortest = std::min(shortest, p);
-      m = std::min(m, std::max(1, p / k));
-    }
+    if (!S->ephemeral && r.stage == 3 && p > 0) m = std::min(m, std::max(1, p / k));
     if (r.stage != 1) continue;
     if (res && r.I->h.refine) sweeps = std::max(sweeps, r.I->sweeps_seen > 0 ? r.I->sweeps_seen : 2);
-    if (p > 0) {
-      shortest = std::min(shortest, left);
-      longest = std::max(longest, left);
-    }
     if (!res || !S->ephemeral) m = std::min(m, std::max(1, left / k));
     if (res) continue;
     nsolving++;
@@ -1436,10 +1425,6 @@ int tick_impl(hobak_sched* S) {
     const bool all = (int)resident.size() == M.n;
     if (!all) TRY(plan_transient(ctx, resident, PR));
     int iters = std::min(ctx->resident, kResidentIters);
-    if (!S->ephemeral && rb.total + rbig.total <= ctx->cus) {
-      const int share = std::max(kShareIters, (shortest / sweeps * 5 / 4 + 9) & ~1);
-      if (longest / sweeps > 2 * share) iters = std::min(iters, share);
-    }
     const double now_s = std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
     const double iter_us = rbig.n ? kBigIterUs : die_wgs ? kDieIterUs : kDeviceIterUs * (1 + rb.total / ctx->cus);
     int sweep_iters = 0;

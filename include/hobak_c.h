@@ -309,7 +309,9 @@ int hobak_kernel_stats(hobak_inst* inst, double* spmv_avg_ms, int64_t* spmv_coun
  *                          depend on it, but for FP32_REFINE instances of more rows than the update
  *                          workgroups cover in one run each (86,016 by default), whose sums of products
  *                          round in another order than the two-kernel form's.  Default 2048, which values
-                          above it count as; 0 never
+ *                          above it count as; 0 never.  A scheduler's tick lasts as long as its
+ *                          resident solves, so where small sessions should not wait for a large
+ *                          one's, about 64 serves them better
  *   HOBAK_TUNE_RESIDENT_JOIN  the workgroups of an instance of the resident form run at the same time, and wait
  *                          for each other before they start (0.2 s, or 1 ms where the instance is on one
  *                          die).  Where other work holds the compute units for longer, the instance is left
