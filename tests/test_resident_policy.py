@@ -192,18 +192,3 @@ def test_small_sessions_do_not_wait_for_a_large_one_in_the_two_kernel_form(engin
     small = [_inst(e, (6, 6, 6 + k), precision=F32, iters=35, sweeps=2) for k in range(4)]
     ticks = _serve(e, [large] + small, 80)
     assert max(sum(w[0] == "spmv" for w in t) for t in ticks[20:]) <= 80  # a step of theirs
-
-
-def test_a_new_state_forgets_how_many_sweeps_the_last_step_took(engine):
-    e = engine()
-    inst = _inst(e, (10, 10, 10), precision=F32, sweeps=5)
-
-    def first_tick():
-        inst.step(True)
-        log = [w[0] for w in e.log()]
-        return log[:log.index("status")].count("die")
-
-    assert [first_tick(), first_tick()] == [2, 5]
-    inst.set_state(inst.scene.initial_u(), inst.scene.initial_v())
-    e.log()
-    assert first_tick() == 2
