@@ -556,7 +556,7 @@ struct hobak_sched {
   std::vector<std::pair<int, int>> samples;
   int sample_it = 0;
   int res_it = 0;  // resident PCG iterations since the last sample
-  bool whole = false;  // a private scheduler's one sample is that of all members' first launch
+  bool uneven = false;  // a resident launch has advanced some member: a group's launches are not over all of them
   bool sampling = false;
   // a long-lived scheduler's own sampling (hobak_sched_set_kernel_sampling): every spmv_every-th
   // SpMV launch is timed and credited with the matrix bytes of the instances solving in its tick
@@ -1326,8 +1326,7 @@ int tick_impl(hobak_sched* S) {
   // SpMV launch of the two-kernel form timed.  What that writes, the first iteration of either form forms again from
   // the same inputs, so results do not depend on sampling.  A private scheduler credits its samples with the whole
   // batch: it times all of its members' first launch, and with resident members nothing else.
-  S->whole |= S->ephemeral && !resident.empty();
-  const bool group_samples = S->sampling && !S->whole;
+  const bool group_samples = S->sampling && !S->uneven && !(S->ephemeral && !resident.empty());
   int probed = 0;
   double probe_bytes = 0.0;
   if (every > 0 && !resident.empty() && (int)S->samples.size() < kMaxSamples &&
@@ -1486,6 +1485,7 @@ int tick_impl(hobak_sched* S) {
     work_bytes += (double)(work + res_work) * spmv_bytes_of(I);
     res_launches = std::max(res_launches, res_work);
     const unsigned runs = M.status_host[i].res_runs - I->runs_seen;
+    S->uneven |= S->ephemeral && runs > 0;
     I->runs_seen += runs;
     ctx->res_stat[I->res_pack == kResBig ? HOBAK_RESIDENT_BIG : die_wgs ? HOBAK_RESIDENT_DIE : HOBAK_RESIDENT_DEVICE] +=
         runs;

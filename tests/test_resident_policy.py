@@ -123,6 +123,15 @@ def test_sampling_times_one_launch_and_leaves_the_solve_in_its_form(engine, dims
         inst.set_kernel_sampling(0)
 
 
+def test_an_instance_that_does_not_fit_is_sampled_as_ever(engine):
+    """Its first step tries the resident form, is left untouched and goes on in groups, whose launches are sampled."""
+    e = engine(update_wgs=256)
+    inst = _inst(e, (35, 37, 35), precision=F32, iters=100, big=MISFIT)
+    inst.set_kernel_sampling(1)
+    inst.step(True)
+    assert inst.kernel_stats()["spmv_count"] > 90
+
+
 def test_a_batch_of_both_forms_samples_the_whole_batch(engine):
     """A sample is credited with every member's bytes, so it has to be a launch over all of them."""
     e = engine(row_sort=0)
