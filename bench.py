@@ -13,11 +13,14 @@ first request) is outside the clock; the end-to-end rate that charges it is repo
 
 Output: one JSON line (see the field list in main()).
   value      serving tet-Newton-steps/s = sum over requests of nt / the stream's makespan
-  roofline   the dominant kernel of the serving stream, the PCG's BSR SpMV (FP32): algorithmic
-             bytes nnzb*(9*4+4) + 4*(nv+1) + 2*3*4*nv of the instances solving in a launch's tick,
+  roofline   the PCG's BSR SpMV (FP32) on the serving stream: algorithmic
+             bytes nnzb*(9*4+4) + 4*(nv+1) + 2*3*4*nv of the instances of a launch,
              over its duration, sampled live with HIP start/stop events that the SpMV's own
              dispatch carries (hipExtLaunchKernelGGL) on the library's stream; `traffic` is the
-             HBM bytes per launch from the committed rocprofv3 --pmc summary of this stream
+             HBM bytes per launch from the committed rocprofv3 --pmc summary of this stream.
+             Solves that run in the resident form read their matrix once per launch, so a
+             launch ahead of those that start is timed; `products_gbs` is what their kernel
+             gets through: the bytes of all products formed over the stream's PCG time
   cpu_baseline  the oracle's FP64 restatement (OpenMP) timed on a bounded sample of the same
              stream's sessions on this host's cores (the literal reference has no penalty
              ground); cpu_baseline_c2 times the literal reference (oracle/_ref) on the 40^3 scene
@@ -470,10 +473,11 @@ def serving_form(lib, scenes, args):
                            "bytes_per_launch": ks["spmv_bytes"], "avg_launch_ms": ks["spmv_avg_ms"],
                            "launches_sampled": ks["spmv_count"],
                            "stream_avg_bytes_per_launch": eng.get("spmv_bytes_per_launch"),
-                           "note": "average time of every n-th SpMV launch of the serving engine; "
-                                   "algorithmic bytes per launch averaged over all its launches, "
-                                   "each instance's matrix and vectors counted in the launches "
-                                   "that streamed them (counted on the device)"}
+                           "products_gbs": round(eng["spmv_bytes"] / eng["pcg_gpu_ms"] / 1e6, 1)
+                           if eng.get("pcg_gpu_ms") else None,
+                           "note": "average time and algorithmic bytes of the SpMV launches timed, "
+                                   "every n-th of the two-kernel form and, after every n iterations "
+                                   "of the resident form, one over the solves that start"}
     ca.close()
     if cb is not None:
         cb.close()

@@ -385,7 +385,8 @@ double hobak_sched_clock(hobak_sched* sched);
  * of PCG groups and of epilogues, host milliseconds inside hobak_sched_tick, solves finished,
  * SpMV launches queued, their algorithmic bytes summed (per launch: the matrices and vectors of
  * the instances whose solve was still running in it, nnzb (9 s + 4) + 4 (nv + 1) + 2 * 3 s nv
- * each; the SpMV counts those launches per instance on the device), PCG groups
+ * each; the SpMV counts those launches per instance on the device, and the resident form the
+ * products it formed with each matrix, which count the same), PCG groups
  * replayed from a captured graph, and PCG groups launched directly (over the still-solving
  * instances only, or holding a sampled launch).
  * The engine also marks its work with roctx ranges ("hobak_step", "hobak_step_batch",

@@ -45,8 +45,7 @@ Stream* on(hipStream_t s) {
 const InstDev* inst(const Batch& b, int i) { return b.n == 1 ? b.one : b.inst[i]; }
 bool has(const std::string& name, const char* kernel) { return name.find(kernel) != std::string::npos; }
 
-// one PCG iteration of every instance whose solve is running; `parity` as in the kernels (the current set is 0 again
-// after the odd one)
+// one PCG iteration of every instance whose solve is running
 void iterate(const Batch& b) {
   for (int i = 0; i < b.n; i++) {
     Ctl* c = ctl_of(inst(b, i));
