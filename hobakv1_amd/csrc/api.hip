@@ -56,8 +56,8 @@ constexpr int kMaxPlans = 32;
 constexpr int kMaxSamples = 512;
 constexpr int kResBig = 1 << 20;      // hobak_inst::res_pack of an instance on every compute unit
 // A solve of more iterations goes on in another launch, after the whole batch.  This also is the most that the
-// tuning key allows: 2,048 iterations of up to 40 us stay well below the time that the workgroups of an instance behind
-// them wait for each other.
+// tuning key allows: 2,048 iterations, most often of 4 to 20 us, stay below the time that the workgroups of an instance
+// behind them wait for each other.
 constexpr int kResidentIters = 2048;
 // What an iteration of the resident PCG takes, roughly (one die, over the device, on every compute unit; see
 // resident.hip), and the fewest iterations of a launch that ends early for another context's (share.h).
@@ -68,17 +68,21 @@ constexpr int kTurnIters = 32;
 constexpr int kBigTries = 4;
 
 // A form of the resident PCG whose workgroups did not meet is left out for a number of ticks, twice as many each
-// time it happens again, so that the waits cost little however long the other work stays; half as many each
-// time the form has run.
+// time it happens again, so that the waits cost little however long the other work stays; half as many after every
+// kHoldRuns ticks that the form has run.
+constexpr int kHoldRuns = 256;
 struct Hold {
-  int first, left = 0, next;
+  int first, left = 0, next, runs = 0;
   explicit Hold(int first_) : first(first_), next(first_) {}
   bool pass() { return left == 0 || left-- == 0; }  // whether this tick may take the form
   void late() {
     left = next;
     next = std::min(2 * next, 1 << 20);
+    runs = 0;
   }
-  void met() { next = std::max(first, next / 2); }
+  void met() {
+    if (++runs % kHoldRuns == 0) next = std::max(first, next / 2);
+  }
 };
 }  // namespace
 
@@ -101,7 +105,7 @@ struct hobak_ctx {
   int resident = kResidentIters;       // resident PCG: iterations per launch, 0 off
   int cus = 0;                         // compute units of the device
   Claim claim;                         // this context's part of them (share_of(device))
-  int join = 1;                        // resident PCG: 0 marks every instance as one whose workgroups did not meet
+  int join = 1;                        // resident PCG: 0 and 2 mark instances (HOBAK_TUNE_RESIDENT_JOIN)
   Hold device_hold{64}, die_hold{16};  // the resident PCG over the device, and on one die each
   int* tickets = nullptr;              // resident PCG launches of this context's stream
   int64_t res_stat[HOBAK_RESIDENT_STATS] = {};  // see hobak_ctx_resident_stats
@@ -1443,9 +1447,10 @@ int tick_impl(hobak_sched* S) {
     ctx->claim.live = true;
     const int wgs = ctx->join ? die_wgs : std::max(1, die_wgs - 1);
     for (int j = 0; j < sweeps; j++) {
-      if (!ctx->join)
+      if (ctx->join == 0 || (ctx->join == 2 && j == 0))  // (a lost solve's other launches do not run)
         for (auto* I : resident)
-          HIPCHK(ctx, hipMemcpyAsync(&I->h.ctl->res_arrive, &kResLate, sizeof(int), hipMemcpyHostToDevice, s));
+          HIPCHK(ctx, hipMemcpyAsync(&I->h.ctl->res_arrive, ctx->join ? &kResLost : &kResLate, sizeof(int),
+                                     hipMemcpyHostToDevice, s));
       if (die_wgs)
         HIPCHK(ctx, launch_cg_resident_die<T>(rb, M.shift, M.groups, first_die, wgs, ctx->tickets, iters, s));
       else
@@ -1497,9 +1502,12 @@ int tick_impl(hobak_sched* S) {
     // columns that do not fit never will: more workgroups, each with fewer rows, while the device has that many, and
     // over the device instead of on one die.  Workgroups that did not meet may do so later.
     const bool misfit = aborts > late;
+    // (a solve whose workgroups lost each other is started again below)
+    const int lost = runs > 0 && M.status_host[i].res_lost ? 1 : 0;
+    ctx->res_stat[HOBAK_RESIDENT_LOST] += lost;
     if (I->res_pack == kResBig) {
-      if (runs) I->big_hold.met();
-      I->late_row = runs ? 0 : I->late_row + late;
+      if (runs && !lost) I->big_hold.met();
+      I->late_row = runs && !lost ? 0 : I->late_row + late + lost;
       if (I->late_row >= kBigTries) {
         I->big_hold.late();
         I->late_row = 0;
@@ -1508,7 +1516,7 @@ int tick_impl(hobak_sched* S) {
       continue;
     }
     ran_rest |= runs > 0;
-    late_rest |= late > 0;
+    late_rest |= late + lost > 0;
     if (misfit && die_wgs) {
       I->die_fit = false;
     } else if (misfit) {
@@ -1585,7 +1593,11 @@ int tick_impl(hobak_sched* S) {
     if (r.stage != 1) continue;
     const InstStatus& q = M.status_host[S->index[r.I]];
     const bool refine = r.I->h.refine != 0;
-    if (q.phase == PHASE_FINISHED) {
+    if (q.res_lost) {  // its Newton iteration starts again, from the displacement it started from
+      r.stage = 0;
+      r.begin = 0;
+      r.done_iters = 0;
+    } else if (q.phase == PHASE_FINISHED) {
       const int nk = r.newton_k;
       const int iters = refine ? q.inner_total : q.iters;
       r.st.pcg_iters[nk] = iters;
@@ -2670,7 +2682,8 @@ int hobak_ctx_set_tuning(hobak_ctx* ctx, int32_t key, int32_t value) {
       ctx->resident = (value + 1) & ~1;
       return HOBAK_OK;
     case HOBAK_TUNE_RESIDENT_JOIN:
-      ctx->join = value != 0;
+      if (value < 0 || value > 2) return fail(ctx, HOBAK_E_INVALID, "resident join out of range");
+      ctx->join = value;
       return HOBAK_OK;
     case HOBAK_TUNE_UPDATE_WGS:
       if (value < 1 || value > 65536) return fail(ctx, HOBAK_E_INVALID, "update workgroups out of range");

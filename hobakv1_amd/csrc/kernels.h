@@ -120,6 +120,9 @@ struct Ctl {
   unsigned res_epoch;
   int res_arrive, res_exit, res_abort, res_late;
   unsigned res_runs;
+  // set where workgroups that had met stopped answering (see resident.hip): the solve's vectors are not to be used, and
+  // the solve starts again; cleared by its start
+  int res_lost;
   unsigned res_work;  // products the resident PCG formed with this instance's matrix (wraps, as spmv_work)
 };
 
@@ -136,7 +139,7 @@ struct InstStatus {
   double err;       // sqrt(res^2 / b^2) of the finished solve
   double maxR;      // |S b|^2
   unsigned spmv_work, res_work;  // Ctl's
-  int res_abort, res_late;  // Ctl's
+  int res_abort, res_late, res_lost;  // Ctl's
   unsigned res_runs;   // Ctl::res_runs
 };
 
@@ -364,7 +367,9 @@ hipError_t launch_cg_spmv_p(const Batch& b, int shift, int pad, int stream, int 
 // workgroup to hold one run of rows (nb[K_UPD] below the cap), but for `big`, which every instance then takes
 // (resident_layout_big).  tickets: kResTickets zero ints.
 constexpr int kResDies = 8, kResDieWgs = 32, kResTickets = 1 + kResDies;
-constexpr int kResLate = 1 << 29;  // of Ctl::res_arrive: the workgroups did not meet, and leave the instance untouched
+// of Ctl::res_arrive: the workgroups did not meet, and leave the instance untouched; a workgroup waited in vain for
+// others it had met
+constexpr int kResLate = 1 << 29, kResLost = 1 << 28;
 template <typename T>
 hipError_t launch_cg_resident(const Batch& b, int shift, int groups, bool big, int* tickets, int iters, hipStream_t s);
 // The same for at most kResDies instances, instance i on the workgroups of die `first` + i mod kResDies (at most `wgs`,

@@ -68,7 +68,11 @@
 // changes anything it announces itself and waits for the others of its instance; if they do not appear in
 // time (another program holds the compute units) or one of them cannot hold its columns, the
 // instance is left untouched and counted in Ctl::res_abort, and in Ctl::res_late where only time ran out: the
-// host then takes another form for good, or for a while.
+// host then takes another form for good, or for a while.  Workgroups that have met run until the launch ends, so the
+// waits of its iterations are short; but where several processes share the device, it takes queues off its compute
+// units and puts them back, and two launches that each got only part of theirs back wait in vain (four
+// processes on one device: once in some 10,000 launches).  A workgroup that waits too long marks the instance
+// (Ctl::res_lost) and leaves, as all others then do; the host starts that solve again from its right-hand side.
 #include "kernels.h"
 #include "pcg_device.h"
 
@@ -92,14 +96,18 @@ constexpr int kResMaxUpd = 512;               // update workgroups of an instanc
 // the rest of its last group's rows a second time, up to 255 rows past its own 168 to 336 with 64-row slices.  A
 // lane then polls up to four words, so the rule ends where lanes would have more than one group each.
 constexpr int kSplitMax = 255;
-constexpr int kMisfit = 1 << 30, kLate = kResLate, kAbort = kMisfit | kLate;  // of Ctl::res_arrive
+constexpr int kMisfit = 1 << 30, kLate = kResLate, kAbort = kMisfit | kLate, kLost = kResLost;  // of Ctl::res_arrive
 // How long an instance's workgroups wait for each other, in ticks of the 100 MHz wall clock: they are dispatched
-// together, so they meet within microseconds unless other work holds compute units.  A launch of another context
-// ends within tens of milliseconds; past 0.2 s something does not give its compute units back.  On one die, of
-// which a large instance of another context may leave too few compute units although others are free: 1 ms, after which
-// the instance rather runs over the whole device.
-constexpr u64 kJoinTicks = 20000000ull, kDieJoinTicks = 100000ull;
-constexpr unsigned kWaitTicks = 500000000u;   // 5 s; every peer is running, so this is never reached
+// together, so they meet within microseconds unless other work holds compute units: earlier instances of the
+// same launch, or another process's launch, which ends within milliseconds to tens of them, or whose workgroups wait
+// in vain too because this launch holds the compute units they lack.  On every compute unit, 20 ms, so that of such
+// two the other goes on (with 0.2 s for all, four processes that step 303,242, 68,921, 9,261 and 1,331 vertices took
+// 0.2 to 0.8 s for a step now and then); otherwise 50 ms; on one die, of which a large instance of another
+// process may leave too few compute units although others are free, 1 ms, after which the instance rather runs over the
+// whole device.
+template <bool BIG, bool ONE>
+constexpr u64 kJoinTicks = ONE ? 100000ull : BIG ? 2000000ull : 5000000ull;
+constexpr unsigned kWaitTicks = 10000000u;    // 0.1 s: the longest wait in an iteration (see Residency above)
 constexpr int kAgentScope = 16;               // cache policy of a buffer access: coherent over the device's L2s
 constexpr int kDieScope = 0;                  // of a store: to this die's L2, where loads of the other policy find it
 constexpr int kArrived = 1023;                // Ctl::res_arrive: workgroups here
@@ -576,7 +584,7 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
       const u64 t0 = wall_clock64();
       int v = __hip_atomic_load(arr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       while (!(v & kAbort) && (v & kArrived) < W) {
-        if (wall_clock64() - t0 > (ONE ? kDieJoinTicks : kJoinTicks))
+        if (wall_clock64() - t0 > kJoinTicks<BIG, ONE>)
           __hip_atomic_compare_exchange_strong(arr, &v, v | kLate, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT);
         else
@@ -1165,11 +1173,16 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
   // the last workgroup to leave clears the instance's meeting point (ONE: if all W of them came; see the kernel)
   __syncthreads();
   if (tid == 0) {
+    if (sh_failed) {
+      __hip_atomic_fetch_or(arr, kLost, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __builtin_amdgcn_s_waitcnt(0);  // before it counts as having left
+    }
     auto ex = (HOBAK_GLOBAL int*)&ctl->res_exit;
     if (__hip_atomic_fetch_add(ex, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == W - 1) {
       const int v = __hip_atomic_load(arr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (v & kAbort) ctl->res_abort += 1;
       if ((v & kAbort) == kLate) ctl->res_late += 1;
+      if (v & kLost) ctl->res_lost = 1;
       __hip_atomic_store(arr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(ex, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }

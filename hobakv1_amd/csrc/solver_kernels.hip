@@ -920,6 +920,7 @@ __global__ __launch_bounds__(kBlock) void cg_init_kernel(Batch b, int refine, in
     s->done = done;
     s->status = status;
     s->first = 1;
+    if (!gate) c->res_lost = 0;
     c->phase = PHASE_SOLVING;
   }
 }
@@ -1917,6 +1918,13 @@ __global__ __launch_bounds__(kBlock) void finish_check_kernel(Batch b, int refin
     int lb, lg;
     const HOBAK_GLOBAL InstDev* __restrict__ I = seg_find(b, vb, lb, lg);
     auto c = ctl_of(I);
+    if (c->res_lost && c->phase == PHASE_SOLVING) {  // the host starts it again
+      if (threadIdx.x == 0) {
+        c->sc[0].done = 1;
+        c->phase = PHASE_FINISHED;
+      }
+      continue;
+    }
     if (!solve_ended(c)) continue;
     if (!refine) {
       if (threadIdx.x == 0) c->phase = PHASE_FINISHED;
@@ -1978,6 +1986,7 @@ __global__ __launch_bounds__(kBlock) void status_kernel(Batch b, InstStatus* out
     o.res_work = c->res_work;
     o.res_abort = c->res_abort;
     o.res_late = c->res_late;
+    o.res_lost = c->res_lost;
     o.res_runs = c->res_runs;
     if (I->refine) {
       o.err = c->rs.b2 > 0 ? sqrt(c->rs.res2 / c->rs.b2) : 0.0;

@@ -267,9 +267,9 @@ class Context:
     def resident_stats(self):
         """Instance launches of the resident PCG by form, and those that left an instance untouched
         (`late` of them because its workgroups did not meet in time)."""
-        out = (ctypes.c_int64 * 5)()
+        out = (ctypes.c_int64 * 6)()
         self.check(self.lib.hobak_ctx_resident_stats(self.h, out), "resident_stats")
-        return dict(zip(("device", "die", "big", "aborted", "late"), out))
+        return dict(zip(("device", "die", "big", "aborted", "late", "lost"), out))
 
     def copy_probe(self, nbytes, reps=20):
         ms = ctypes.c_double(0)

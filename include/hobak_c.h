@@ -313,13 +313,16 @@ int hobak_kernel_stats(hobak_inst* inst, double* spmv_avg_ms, int64_t* spmv_coun
  *                          resident solves, so where small sessions should not wait for a large
  *                          one's, about 64 serves them better
  *   HOBAK_TUNE_RESIDENT_JOIN  the workgroups of an instance of the resident form run at the same time, and wait
- *                          for each other before they start (0.2 s, or 1 ms where the instance is on one
- *                          die).  Where other work holds the compute units for longer, the instance is left
+ *                          for each other before they start (50 ms, on every compute unit 20 ms, on one
+ *                          die 1 ms).  Where other work holds the compute units for longer, the instance is left
  *                          untouched, solves in the two-kernel form (from one die: over the device), and
  *                          tries again some ticks later, twice as many each time.  FP32_REFINE instances
  *                          whose sums would round differently there take the two-kernel form only
- *                          after four waits in a row.  Default 1; 0, for tests of that path: they never
- *                          meet, and a launch on single dies brings one workgroup too few to each */
+ *                          after four waits in a row.  Workgroups that have met and then wait in vain
+ *                          for 0.1 s, where several processes share the device, leave the solve to
+ *                          be started again.  Default 1; for tests of these paths 0: they never
+ *                          meet, and a launch on single dies brings one workgroup too few to each, and
+ *                          2: every launch counts as one whose workgroups lost each other */
 #define HOBAK_TUNE_SLICE_ROWS 0
 #define HOBAK_TUNE_POLL_CHUNK 2
 #define HOBAK_TUNE_MAX_CHUNKS 3
@@ -342,13 +345,15 @@ int hobak_ctx_set_tuning(hobak_ctx* ctx, int32_t key, int32_t value);
  * of the resident PCG (HOBAK_TUNE_RESIDENT), which form advanced it - over the whole device, on one die,
  * or on every compute unit (FP32_REFINE instances of more rows than the update workgroups cover) - or
  * that the launch left it untouched, for another form to solve: all of those, and the ones among them whose
- * workgroups did not meet in time (HOBAK_TUNE_RESIDENT_JOIN; the others' columns do not fit). */
+ * workgroups did not meet in time (HOBAK_TUNE_RESIDENT_JOIN; the others' columns do not fit); and how many solves
+ * were started again because workgroups that had met lost each other. */
 #define HOBAK_RESIDENT_DEVICE 0
 #define HOBAK_RESIDENT_DIE 1
 #define HOBAK_RESIDENT_BIG 2
 #define HOBAK_RESIDENT_ABORTED 3
 #define HOBAK_RESIDENT_LATE 4
-#define HOBAK_RESIDENT_STATS 5
+#define HOBAK_RESIDENT_LOST 5
+#define HOBAK_RESIDENT_STATS 6
 int hobak_ctx_resident_stats(hobak_ctx* ctx, int64_t* out);
 
 /* Continuous-batching scheduler (no counterpart in the reference, whose callers step one scene

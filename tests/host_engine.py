@@ -7,7 +7,7 @@ import tempfile
 
 from hobakv1_amd import build, lib
 
-RUNS, MISFIT, LATE = 0, 1, 2
+RUNS, MISFIT, LATE, LOST = 0, 1, 2, 3
 _fake = None
 
 

@@ -16,7 +16,7 @@
 using namespace hobak;
 
 namespace {
-enum Outcome { RUNS = 0, MISFIT = 1, LATE = 2 };
+enum Outcome { RUNS = 0, MISFIT = 1, LATE = 2, LOST = 3 };
 struct Script {
   int sweeps = 1, iters = 10;
   int outcome[3] = {RUNS, RUNS, RUNS};  // over the device, on one die, on every compute unit
@@ -62,6 +62,11 @@ void resident(const Batch& b, int form, int iters) {
     if (c->sc[0].done) continue;
     const Script& s = g_script[I->nv];
     const int what = s.outcome[form];
+    if (what == LOST) {
+      c->res_lost = 1;
+      c->res_runs += 1;
+      continue;
+    }
     if (what != RUNS) {
       c->res_abort += 1;
       if (what == LATE) c->res_late += 1;
@@ -95,6 +100,7 @@ std::function<void()> stand_in(const std::string& name, void** a) {
         if (!gate) c->rs = RefineState{};
         c->sc[0] = CgScalars{};
         c->sc[0].first = 1;
+        if (!gate) c->res_lost = 0;
         c->phase = PHASE_SOLVING;
       }
     };
@@ -127,6 +133,11 @@ std::function<void()> stand_in(const std::string& name, void** a) {
     return [=] {
       for (int i = 0; i < b.n; i++) {
         Ctl* c = ctl_of(inst(b, i));
+        if (c->phase == PHASE_SOLVING && c->res_lost) {
+          c->sc[0].done = 1;
+          c->phase = PHASE_FINISHED;
+          continue;
+        }
         if (!(c->phase == PHASE_SOLVING && c->sc[0].done)) continue;
         if (refine) {
           c->rs.inner_iters += c->sc[0].iters;
@@ -155,6 +166,7 @@ std::function<void()> stand_in(const std::string& name, void** a) {
         o.res_work = c->res_work;
         o.res_abort = c->res_abort;
         o.res_late = c->res_late;
+        o.res_lost = c->res_lost;
         o.res_runs = c->res_runs;
         out[i] = o;
       }

@@ -70,3 +70,39 @@ def test_a_die_that_gets_too_few_workgroups(precision):
         assert np.array_equal(u, uw) and np.array_equal(v, vw)
     assert stats[0]["late"] >= 2 and stats[0]["die"] == stats[0]["device"] == 0
     assert stats[-1]["late"] == stats[0]["late"] and stats[-1]["die"] > 0
+
+
+@pytest.mark.parametrize("dims,precision,tuning,form", [
+    ([(4, 4, 4)], F64, {}, "device"), ([(10, 10, 10)], F64, {}, "die"), ([(10, 10, 10)], F32, {}, "die"),
+    ([(22, 22, 22)], F64, {}, "device"), ([(22, 22, 22)], F32, {}, "device"),
+    ([(8, 7, 6), (9, 8, 7), (17, 9, 23)], F32, {}, "die"), ([(5 + k, 8, 7) for k in range(12)], F64, {}, "device")])
+def test_workgroups_that_lose_each_other(dims, precision, tuning, form):
+    """(HOBAK_TUNE_RESIDENT_JOIN 2: every launch counts as such.)  The solve starts again, with the same results."""
+    scs = [_lattice(d, seed=k) for k, d in enumerate(dims)]
+    joins = [1, 2, 2] + [1] * 140
+    want, _ = _run(scs, precision, joins, resident=0, **tuning)
+    got, stats = _run(scs, precision, joins, **tuning)
+    for (u, v), (uw, vw) in zip(got, want):
+        assert np.array_equal(u, uw) and np.array_equal(v, vw)
+    assert stats[0]["lost"] == 0 and stats[1]["lost"] >= len(dims) and stats[-1]["lost"] == stats[2]["lost"]
+    assert stats[-1][form] > stats[2][form] and stats[-1]["aborted"] == 0
+
+
+def test_workgroups_on_every_compute_unit_that_lose_each_other():
+    scs = [_lattice((35, 37, 35))]
+    want, _ = _run(scs, F32, [1, 1], resident=0, update_wgs=256)
+    got, stats = _run(scs, F32, [2, 1], update_wgs=256)
+    assert stats[0]["lost"] == 4 and np.isfinite(got[0][0]).all()
+    assert np.linalg.norm(got[0][0] - want[0][0]) <= 1e-9 * np.linalg.norm(scs[0].rest.ravel() + want[0][0])
+
+
+@pytest.mark.parametrize("precision", [F64, F32])
+def test_newton_iterations_and_plane_constraints_after_a_loss(precision):
+    sc = _lattice((9, 8, 7))
+    sc.newton_iters = 3
+    scs = [sc] + ([scenes.drop_scene((6, 6, 6))] if precision == F64 else [])
+    for s in scs:
+        want, _ = _run([s], precision, [1, 2, 1, 2], resident=0)
+        got, stats = _run([s], precision, [1, 2, 1, 2])
+        assert np.array_equal(got[0][0], want[0][0]) and np.array_equal(got[0][1], want[0][1])
+        assert stats[-1]["lost"] > 0

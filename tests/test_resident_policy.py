@@ -2,7 +2,7 @@
 import pytest
 
 import host_engine
-from host_engine import LATE, MISFIT, RUNS
+from host_engine import LATE, LOST, MISFIT
 from hobakv1_amd import lib, scenes
 
 F64, F32 = lib.PRECISION_FP64, lib.PRECISION_FP32_REFINE
@@ -52,7 +52,8 @@ def test_stalls_that_go_on_cost_ever_fewer_waits(engine):
     inst = _inst(e, (40, 40, 40), device=LATE)
     waits = sum(_step(e, inst)[0] == "device" for _ in range(2000))
     assert 2 <= waits <= 8
-    assert e.ctx.resident_stats() == {"device": 0, "die": 0, "big": 0, "aborted": waits, "late": waits}
+    assert e.ctx.resident_stats() == {"device": 0, "die": 0, "big": 0, "aborted": waits, "late": waits,
+                                       "lost": 0}
 
 
 def test_columns_that_do_not_fit_take_more_workgroups_and_then_the_two_kernel_form(engine):
@@ -94,6 +95,22 @@ def test_an_instance_on_every_compute_unit_keeps_its_form_through_a_stall(engine
     assert forms[:2] == ["big", "spmv"] and e.ctx.resident_stats()["late"] == 4
     e.script(inst)
     assert [_step(e, inst) for _ in range(200)][-1] == ["big"]
+
+
+@pytest.mark.parametrize("dims,precision,form", [((10, 10, 10), F64, "die"), ((40, 40, 40), F64, "device"),
+                                                 ((10, 10, 10), F32, "die")])
+def test_a_solve_whose_workgroups_lost_each_other_starts_again(engine, dims, precision, form):
+    e = engine()
+    inst = _inst(e, dims, precision=precision, iters=30, sweeps=2 if precision == F32 else 1, **{form: LOST})
+    e.ctx.set_tuning(max_chunks=1)
+    st = inst.step(True)
+    log = [w[0] for w in e.log()]
+    assert log.count("begin") == 1  # the step itself began once
+    assert st["status"] == 0 and st["total_pcg_iters"] == (60 if precision == F32 else 30)
+    assert e.ctx.resident_stats()["lost"] == 1
+    e.script(inst, iters=30)
+    assert _step(e, inst) == ["device" if form == "die" else "spmv"]
+    assert [_step(e, inst) for _ in range(200)][-1] == [form]
 
 
 def test_a_launch_ends_before_the_wait_of_those_behind_it(engine):
