@@ -105,6 +105,7 @@ struct hobak_ctx {
   int resident = kResidentIters;       // resident PCG: iterations per launch, 0 off
   int cus = 0;                         // compute units of the device
   Claim claim;                         // this context's part of them (share_of(device))
+  std::vector<hipEvent_t> group_ev;    // behind the groups of a tick
   int join = 1;                        // resident PCG: 0 and 2 mark instances (HOBAK_TUNE_RESIDENT_JOIN)
   Hold device_hold{64}, die_hold{16};  // the resident PCG over the device, and on one die each
   int* tickets = nullptr;              // resident PCG launches of this context's stream
@@ -165,14 +166,21 @@ Share& share_of(int device) {
   return shares[device];
 }
 
+double now_seconds() {
+  return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
+}
+
 // Gives a claim back at the end of the tick that made it, whose wait its launches have passed.
 struct ClaimGuard {
   hobak_ctx* ctx;
   ~ClaimGuard() { release(); }
   void release() {
-    if (!ctx->claim.live) return;
+    if (!ctx->claim.live && ctx->claim.groups.empty()) return;
     std::lock_guard<std::mutex> lock(share_of(ctx->device).mu);
     ctx->claim.live = false;
+    if (!ctx->claim.groups.empty()) ctx->claim.groups_s = now_seconds();
+    ctx->claim.groups.clear();
+    ctx->claim.passed = 0;
   }
 };
 
@@ -1019,6 +1027,24 @@ int resident_per_die(const hobak_ctx* ctx, const std::vector<hobak_inst*>& m) {
   return most > 1 ? most : 0;  // (a workgroup by itself exchanges nothing)
 }
 
+// The event behind the j-th group of a tick, for contexts that share the device (share.h).
+int publish_group(hobak_ctx* ctx, int j) {
+  Share& share = share_of(ctx->device);
+  {
+    std::lock_guard<std::mutex> lock(share.mu);
+    if (share.claims.size() < 2) return HOBAK_OK;
+  }
+  while ((int)ctx->group_ev.size() <= j) {
+    hipEvent_t e = nullptr;
+    HIPCHK(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    ctx->group_ev.push_back(e);
+  }
+  HIPCHK(ctx, hipEventRecord(ctx->group_ev[j], ctx->stream));
+  std::lock_guard<std::mutex> lock(share.mu);
+  ctx->claim.groups.push_back(ctx->group_ev[j]);
+  return HOBAK_OK;
+}
+
 // The resident PCG's launch tables in the arena: the instances, largest first (their solves take the
 // most iterations, and what runs last should be short), and the workgroups of each.  An instance takes
 // as few workgroups as hold its matrix on chip (res_pack) when the batch fills the device's
@@ -1380,6 +1406,7 @@ int tick_impl(hobak_sched* S) {
         TRY(launch_chunk<T>(ctx, compact ? PG : M, k, st, group_samples ? S : nullptr, every));
         S->stat[10] += 1;
       }
+      TRY(publish_group(ctx, j));
     }
     ran = true;
   }
@@ -1428,13 +1455,24 @@ int tick_impl(hobak_sched* S) {
     const bool all = (int)resident.size() == M.n;
     if (!all) TRY(plan_transient(ctx, resident, PR));
     int iters = std::min(ctx->resident, kResidentIters);
-    const double now_s = std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
+    const double now_s = now_seconds();
     const double iter_us = rbig.n ? kBigIterUs : die_wgs ? kDieIterUs : kDeviceIterUs * (1 + rb.total / ctx->cus);
     int sweep_iters = 0;
     for (auto* I : resident) sweep_iters = std::max(sweep_iters, I->sweep_iters);
     const bool alone = share.fits(&ctx->claim, use, per_die);
     if (!alone) share.meets(&ctx->claim, now_s);
-    const double turn_ms = share.turn_ms(&ctx->claim, now_s);
+    double turn_ms = share.turn_ms(&ctx->claim, now_s);
+    if (Share::large(use, per_die) && share.groups_lately(&ctx->claim, now_s)) {
+      turn_ms = kGroupsTurnMs;
+      for (Claim* c : share.claims) {
+        if (c == &ctx->claim || c->groups.empty()) continue;
+        while (c->passed < c->groups.size() && hipEventQuery((hipEvent_t)c->groups[c->passed]) == hipSuccess) c->passed++;
+        (void)hipGetLastError();  // (not ready is no error)
+        if (c->passed < c->groups.size())
+          HIPCHK(ctx, hipStreamWaitEvent(
+                          s, (hipEvent_t)c->groups[std::min(c->passed + kGroupsAhead, c->groups.size()) - 1], 0));
+      }
+    }
     ctx->claim.ms = 1e-3 * iter_us * sweeps * std::min(iters, sweep_iters);
     if (turn_ms > 0.0 && ctx->claim.ms > 1.25 * turn_ms) {
       iters = std::min(iters, std::max(kTurnIters, (int)(1e3 * turn_ms / iter_us) & ~1));
@@ -1884,6 +1922,7 @@ void hobak_ctx_destroy(hobak_ctx* ctx) {
     if (e) (void)hipEventDestroy(e);
   for (auto& e : ctx->sample_ev)
     if (e) (void)hipEventDestroy(e);
+  for (auto& e : ctx->group_ev) (void)hipEventDestroy(e);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
 }

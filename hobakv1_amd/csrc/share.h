@@ -9,6 +9,11 @@
 // A launch holds its compute units for a whole solve, which a context with a small instance would wait for each
 // time.  Of contexts that were in each other's way lately, one whose launches take longer than another's therefore
 // takes turns of about the other's length.  (Contexts that one thread uses in turn never are.)
+//
+// Groups of the two-kernel form wait for nobody, but their launches get only the compute units that resident ones leave,
+// between launches or beside them (57x64x50 in FP64 beside a 40^3 stepper: 200 ms a step, 60 before the resident PCG).
+// A context that queues groups therefore publishes an event behind each, and a launch that takes more than a
+// quarter of the device beside such a context first lets it run two groups, and takes a short turn.
 #pragma once
 #include <algorithm>
 #include <mutex>
@@ -25,10 +30,15 @@ struct Claim {
   double ms = 0.0;           // what its launches take, roughly
   double met_s = -1e9;       // when it last did not fit beside another, or another beside it
   bool live = false;         // its launches are queued or running
+  std::vector<void*> groups; // the events behind its groups of the two-kernel form in this tick ...
+  size_t passed = 0;         // ... of which this many are known to have run
+  double groups_s = -1e9;    // when it last had any
 };
 
 constexpr double kShareLatelyS = 0.05;  // contexts that were in each other's way within this time are expected to be again
-constexpr double kShareTurnMs = 2.0;    // the shortest turn: a launch's set-up and the host's part take 0.1 ms
+constexpr double kShareTurnMs = 2.0;    // the shortest turn: a launch's set-up and the host's part take 0.1 ms ...
+constexpr double kGroupsTurnMs = 1.0;   // ... and beside groups, of which two take 0.4 ms (40^3) to 2 ms (57x64x50)
+constexpr size_t kGroupsAhead = 2;
 
 struct Share {
   std::mutex mu;               // held while a claim is made and its launches are queued
@@ -56,6 +66,18 @@ struct Share {
       for (const Claim* c : claims)
         if (c != mine && now_s - c->met_s < kShareLatelyS) ms = ms > 0.0 ? std::min(ms, c->ms) : c->ms;
     return ms > 0.0 ? std::max(ms, kShareTurnMs) : 0.0;
+  }
+  // Whether `use` is so much of the device (of `per_die` compute units a die) that others' groups need turns.
+  static bool large(const int (&use)[kShareDies], int per_die) {
+    int sum = 0;
+    for (int u : use) sum += u;
+    return 4 * sum > kShareDies * per_die;
+  }
+  // Whether another context queues groups, or did lately.
+  bool groups_lately(const Claim* mine, double now_s) const {
+    for (const Claim* c : claims)
+      if (c != mine && (!c->groups.empty() || now_s - c->groups_s < kShareLatelyS)) return true;
+    return false;
   }
   // The die on which to put the first of `n` instances that take wgs[i] compute units of successive dies: where
   // the fullest die is emptiest; -1 if they fit on none.

@@ -1,6 +1,7 @@
 """Contexts of one process stepping in threads of their own, whose resident launches together need more compute units than
 the device has: none of them waits in vain, and each ends bitwise where it ends alone."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -53,3 +54,36 @@ def test_contexts_in_threads(programs):
     for p in ps:
         p.close()
     assert all(s["late"] == 0 and s["aborted"] == 0 for s in stats), stats
+
+
+@pytest.mark.parametrize("beside", [((40, 40, 40), F64, {}), ((35, 37, 35), F32, dict(update_wgs=256))])
+def test_groups_of_the_two_kernel_form_beside_a_resident_stepper(beside):
+    """A mesh beyond the resident form while another thread steps one that fills the device: its launches get compute
+    units of their own turns, and a step takes a few times what it takes alone, not as long as the other steps."""
+    large = _Program((40, 41, 42), F64, 3, update_wgs=256)
+    dims, precision, tuning = beside
+    other = _Program(dims, precision, 1, **tuning)
+    print(f"  {beside}", flush=True)
+    large.run()
+    t0 = time.perf_counter()
+    large.run()
+    alone, end = time.perf_counter() - t0, large.end
+    assert large.ctx.resident_stats()["device"] == 0
+    other.run()
+    stop = threading.Event()
+
+    def step():
+        while not stop.is_set():
+            other.run()
+
+    thread = threading.Thread(target=step)
+    thread.start()
+    t0 = time.perf_counter()
+    large.run()
+    took = time.perf_counter() - t0
+    stop.set()
+    thread.join()
+    assert np.array_equal(large.end[0], end[0]) and np.array_equal(large.end[1], end[1])
+    large.close()
+    other.close()
+    assert took < 5 * alone, (took, alone)

@@ -44,6 +44,15 @@ int main() {
   CHECK(s.fits(&a, all(32).u, 32));
   s.meets(&a, 20.0);
   CHECK(s.turn_ms(&a, 20.0) == 0.0 && s.turn_ms(&b, 20.0) == 0.0);
+  // groups of the two-kernel form: seen while they are queued and for a while after
+  CHECK(!Share::large(all(8).u, 32) && Share::large(all(9).u, 32) && !Share::large(one(0, 32).u, 32));
+  int event = 0;
+  CHECK(!s.groups_lately(&a, 20.0));
+  b.groups.push_back(&event);
+  CHECK(s.groups_lately(&a, 20.0) && !s.groups_lately(&b, 20.0));
+  b.groups.clear();
+  b.groups_s = 20.0;
+  CHECK(s.groups_lately(&a, 20.01) && !s.groups_lately(&a, 21.0));
   // the emptiest dies
   hold(b, one(0, 28), 1.0);
   CHECK(s.first_die(&a, w, 1, 32) == 1);
