@@ -184,6 +184,19 @@ struct ClaimGuard {
   }
 };
 
+// An entry point that launches only short kernels: its device is current, and launches of other contexts that fill
+// the device see it.  (Not the states', which are small enough to run beside a resident workgroup.)
+struct ShortCall {
+  hobak_ctx* ctx;
+  explicit ShortCall(hobak_ctx* c) : ctx(c) {
+    (void)hipSetDevice(c->device);
+    ctx->claim.calls.fetch_add(1, std::memory_order_relaxed);
+  }
+  ~ShortCall() { ctx->claim.calls.fetch_sub(1, std::memory_order_relaxed); }
+  ShortCall(const ShortCall&) = delete;
+  ShortCall& operator=(const ShortCall&) = delete;
+};
+
 struct Pattern {
   int nv = 0, nt = 0, nslices = 0, nslots = 0, nrows_pad = 0, nnzb = 0;
   int H = 16, shift = 4;  // rows per slice and its log2
@@ -1462,6 +1475,7 @@ int tick_impl(hobak_sched* S) {
     const bool alone = share.fits(&ctx->claim, use, per_die);
     if (!alone) share.meets(&ctx->claim, now_s);
     double turn_ms = share.turn_ms(&ctx->claim, now_s);
+    if (Share::fills(use, per_die) && share.calls_lately(&ctx->claim, now_s)) turn_ms = kGroupsTurnMs;
     if (Share::large(use, per_die) && share.groups_lately(&ctx->claim, now_s)) {
       turn_ms = kGroupsTurnMs;
       for (Claim* c : share.claims) {
@@ -2413,7 +2427,7 @@ int hobak_inst_compute_fdots(hobak_inst* I, const double* velocity) {
   hobak_ctx* ctx = I->ctx;
   if (I->requests) return fail(ctx, HOBAK_E_INVALID, "instance has a step in flight");
   if (!I->h.fdot) return fail(ctx, HOBAK_E_INVALID, "velocity gradients need energy damping (hobak_inst_set_damping)");
-  (void)hipSetDevice(ctx->device);
+  const ShortCall call(ctx);
   const double* vel = I->h.v;
   if (velocity) {
     std::vector<double> vbuf;
@@ -2533,7 +2547,7 @@ int hobak_get_bsr_pattern(hobak_inst* I, int32_t* nnzb, int32_t* row_ptr, int32_
 int hobak_eval_forces_hessian(hobak_inst* I, const double* u, double* forces, double* kvals) {
   if (!I || !u) return HOBAK_E_INVALID;
   if (I->requests) return fail(I->ctx, HOBAK_E_INVALID, "instance has a step in flight");
-  (void)hipSetDevice(I->ctx->device);
+  const ShortCall call(I->ctx);
   return I->tsize == 8 ? eval_forces_hessian<double>(I, u, forces, kvals)
                        : eval_forces_hessian<float>(I, u, forces, kvals);
 }
@@ -2553,7 +2567,7 @@ int hobak_eval_forces_noalloc(hobak_inst* I, const double* u_dev, double* forces
                     std::to_string((size_t)HOBAK_NOALLOC_SCRATCH_BYTES / (12 * (size_t)I->tsize)) + " tets)");
   if (I->requests) return fail(ctx, HOBAK_E_INVALID, "instance has a step in flight");
   if (!ctx->scratch) return fail(ctx, HOBAK_E_HIP, "no scratch address for this device");
-  (void)hipSetDevice(ctx->device);
+  const ShortCall call(ctx);
   hipStream_t s = ctx->stream;
   // a batch of one names its record directly: no device table is needed
   const Batch be{nullptr, nullptr, I->dev, 1, I->h.nb[K_ELEM]};
@@ -2573,7 +2587,7 @@ int hobak_eval_damping(hobak_inst* I, const double* u, double* forces, double* c
   if (!I || !u) return HOBAK_E_INVALID;
   if (I->requests) return fail(I->ctx, HOBAK_E_INVALID, "instance has a step in flight");
   if (!I->h.damping) return fail(I->ctx, HOBAK_E_INVALID, "the instance has no energy damping");
-  (void)hipSetDevice(I->ctx->device);
+  const ShortCall call(I->ctx);
   return I->tsize == 8 ? eval_damping<double>(I, u, forces, cvals) : eval_damping<float>(I, u, forces, cvals);
 }
 

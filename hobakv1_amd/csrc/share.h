@@ -13,9 +13,11 @@
 // Groups of the two-kernel form wait for nobody, but their launches get only the compute units that resident ones leave,
 // between launches or beside them (57x64x50 in FP64 beside a 40^3 stepper: 200 ms a step, 60 before the resident PCG).
 // A context that queues groups therefore publishes an event behind each, and a launch that takes more than a
-// quarter of the device beside such a context first lets it run two groups, and takes a short turn.
+// quarter of the device beside such a context first lets it run two groups, and takes a short turn.  So does, without the
+// wait, a launch that leaves no compute unit while another context is in a call of short kernels.
 #pragma once
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <vector>
 
@@ -33,6 +35,8 @@ struct Claim {
   std::vector<void*> groups; // the events behind its groups of the two-kernel form in this tick ...
   size_t passed = 0;         // ... of which this many are known to have run
   double groups_s = -1e9;    // when it last had any
+  std::atomic<int> calls{0}; // calls in progress that only launch short kernels (forces, stiffness)
+  double calls_s = -1e9;     // when a launch that filled the device last found any
 };
 
 constexpr double kShareLatelyS = 0.05;  // contexts that were in each other's way within this time are expected to be again
@@ -72,6 +76,19 @@ struct Share {
     int sum = 0;
     for (int u : use) sum += u;
     return 4 * sum > kShareDies * per_die;
+  }
+  static bool fills(const int (&use)[kShareDies], int per_die) {
+    return *std::min_element(use, use + kShareDies) >= per_die;
+  }
+  // Whether another context is in a call of short kernels, or was lately.
+  bool calls_lately(const Claim* mine, double now_s) {
+    bool any = false;
+    for (Claim* c : claims) {
+      if (c == mine) continue;
+      if (c->calls.load(std::memory_order_relaxed) > 0) c->calls_s = now_s;
+      any |= now_s - c->calls_s < kShareLatelyS;
+    }
+    return any;
   }
   // Whether another context queues groups, or did lately.
   bool groups_lately(const Claim* mine, double now_s) const {

@@ -46,6 +46,12 @@ int main() {
   CHECK(s.turn_ms(&a, 20.0) == 0.0 && s.turn_ms(&b, 20.0) == 0.0);
   // groups of the two-kernel form: seen while they are queued and for a while after
   CHECK(!Share::large(all(8).u, 32) && Share::large(all(9).u, 32) && !Share::large(one(0, 32).u, 32));
+  // calls of short kernels: likewise
+  CHECK(Share::fills(all(32).u, 32) && !Share::fills(one(0, 32).u, 32) && !s.calls_lately(&a, 20.0));
+  b.calls = 1;
+  CHECK(s.calls_lately(&a, 20.0) && !s.calls_lately(&b, 20.0));
+  b.calls = 0;
+  CHECK(s.calls_lately(&a, 20.01) && !s.calls_lately(&a, 21.0));
   int event = 0;
   CHECK(!s.groups_lately(&a, 20.0));
   b.groups.push_back(&event);
