@@ -1439,18 +1439,19 @@ int tick_impl(hobak_sched* S) {
     Share& share = share_of(ctx->device);
     const int per_die = std::max(1, ctx->cus / kResDies);
     const std::lock_guard<std::mutex> lock(share.mu);
-    int use[kResDies] = {}, first_die = 0;
+    int use[kResDies] = {}, sum[kResDies], first_die = 0;
+    const bool others = share.held(&ctx->claim, sum);
     auto over_all = [&](int total) {
       for (auto& u : use) u = std::max(u, std::min(per_die, (total + kResDies - 1) / kResDies));
     };
-    if (die_wgs) {
-      first_die = share.first_die(&ctx->claim, each.data(), (int)each.size(), per_die);
+    if (die_wgs && others) {
+      first_die = Share::first_die(sum, each.data(), (int)each.size(), per_die);
       if (first_die < 0) {
         Batch over{};
         std::vector<int> each_over;
         TRY(resident_tables(ctx, rest, 0, over, each_over));
         over_all(over.total);
-        if (share.fits(&ctx->claim, use, per_die)) {
+        if (Share::fits(sum, use, per_die)) {
           rb = over;
           die_wgs = 0;
         } else {
@@ -1472,7 +1473,7 @@ int tick_impl(hobak_sched* S) {
     const double iter_us = rbig.n ? kBigIterUs : die_wgs ? kDieIterUs : kDeviceIterUs * (1 + rb.total / ctx->cus);
     int sweep_iters = 0;
     for (auto* I : resident) sweep_iters = std::max(sweep_iters, I->sweep_iters);
-    const bool alone = share.fits(&ctx->claim, use, per_die);
+    const bool alone = !others || Share::fits(sum, use, per_die);
     if (!alone) share.meets(&ctx->claim, now_s);
     double turn_ms = share.turn_ms(&ctx->claim, now_s);
     if (Share::fills(use, per_die) && share.calls_lately(&ctx->claim, now_s)) turn_ms = kGroupsTurnMs;

@@ -48,14 +48,21 @@ struct Share {
   std::mutex mu;               // held while a claim is made and its launches are queued
   std::vector<Claim*> claims;  // of every context on the device
 
-  // Whether `use` fits beside the live claims of others (on `per_die` compute units a die).
-  bool fits(const Claim* mine, const int (&use)[kShareDies], int per_die) const {
-    for (int d = 0; d < kShareDies; d++) {
-      int sum = use[d];
-      for (const Claim* c : claims)
-        if (c != mine && c->live) sum += c->use[d];
-      if (sum > per_die) return false;
-    }
+  // The compute units that live claims of others hold on each die; false if there are none.
+  bool held(const Claim* mine, int (&sum)[kShareDies]) const {
+    bool any = false;
+    for (int& u : sum) u = 0;
+    for (const Claim* c : claims)
+      if (c != mine && c->live) {
+        any = true;
+        for (int d = 0; d < kShareDies; d++) sum[d] += c->use[d];
+      }
+    return any;
+  }
+  // Whether `use` fits beside `sum` (on `per_die` compute units a die).
+  static bool fits(const int (&sum)[kShareDies], const int (&use)[kShareDies], int per_die) {
+    for (int d = 0; d < kShareDies; d++)
+      if (sum[d] + use[d] > per_die) return false;
     return true;
   }
   // `mine` does not fit beside the live claims of others.
@@ -98,17 +105,13 @@ struct Share {
   }
   // The die on which to put the first of `n` instances that take wgs[i] compute units of successive dies: where
   // the fullest die is emptiest; -1 if they fit on none.
-  int first_die(const Claim* mine, const int* wgs, int n, int per_die) const {
+  static int first_die(const int (&sum)[kShareDies], const int* wgs, int n, int per_die) {
     int best = -1, least = per_die + 1;
     for (int first = 0; first < kShareDies; first++) {
-      int use[kShareDies] = {};
+      int full = 0, use[kShareDies];
+      std::copy(sum, sum + kShareDies, use);
       for (int i = 0; i < n; i++) use[(first + i) % kShareDies] += wgs[i];
-      int full = 0;
-      for (int d = 0; d < kShareDies; d++) {
-        for (const Claim* c : claims)
-          if (c != mine && c->live) use[d] += c->use[d];
-        full = std::max(full, use[d]);
-      }
+      for (int u : use) full = std::max(full, u);
       if (full < least) {
         least = full;
         best = first;

@@ -14,21 +14,24 @@ struct Use { int u[kShareDies]; };
 Use all(int n) { Use x; for (int& v : x.u) v = n; return x; }
 Use one(int d, int n) { Use x = all(0); x.u[d] = n; return x; }
 void hold(Claim& c, Use x, double ms) { std::copy(x.u, x.u + kShareDies, c.use); c.ms = ms; c.live = true; }
+Use held(const Share& s, const Claim* mine) { Use x; s.held(mine, x.u); return x; }
+bool fits(const Share& s, const Claim* mine, Use use) { return Share::fits(held(s, mine).u, use.u, 32); }
+int first_die(const Share& s, const Claim* mine, const int* w, int n) { return Share::first_die(held(s, mine).u, w, n, 32); }
 int main() {
   Share s;
   Claim a, b, c;
   s.claims = {&a, &b, &c};
   // nobody here: room for everything, no turns
-  CHECK(s.fits(&a, all(32).u, 32) && !s.fits(&a, all(33).u, 32));
+  CHECK(fits(s, &a, all(32)) && !fits(s, &a, all(33)));
   CHECK(s.turn_ms(&a, 10.0) == 0.0);
   int w[2] = {28, 8};
-  CHECK(s.first_die(&a, w, 2, 32) == 0);
+  CHECK(first_die(s, &a, w, 2) == 0);
   // b holds 26 compute units of each die: 6 are left
   hold(b, all(26), 4.7);
-  CHECK(s.fits(&a, all(6).u, 32) && !s.fits(&a, one(3, 7).u, 32));
-  CHECK(s.first_die(&a, w, 2, 32) == -1);
+  CHECK(fits(s, &a, all(6)) && !fits(s, &a, one(3, 7)));
+  CHECK(first_die(s, &a, w, 2) == -1);
   // its own claim is not in a context's way
-  CHECK(s.fits(&b, all(32).u, 32));
+  CHECK(fits(s, &b, all(32)));
   // contexts that met take turns of the other's length, for a while
   CHECK(s.turn_ms(&a, 10.0) == 0.0);
   a.ms = 14.0;
@@ -41,7 +44,7 @@ int main() {
   CHECK(s.turn_ms(&a, 12.0) == kShareTurnMs && s.turn_ms(&b, 12.0) == kShareTurnMs && s.turn_ms(&c, 12.0) == 4.7);
   // a claim given back leaves room at once; contexts used in turn do not meet
   b.live = c.live = false;
-  CHECK(s.fits(&a, all(32).u, 32));
+  CHECK(fits(s, &a, all(32)));
   s.meets(&a, 20.0);
   CHECK(s.turn_ms(&a, 20.0) == 0.0 && s.turn_ms(&b, 20.0) == 0.0);
   // groups of the two-kernel form: seen while they are queued and for a while after
@@ -61,11 +64,11 @@ int main() {
   CHECK(s.groups_lately(&a, 20.01) && !s.groups_lately(&a, 21.0));
   // the emptiest dies
   hold(b, one(0, 28), 1.0);
-  CHECK(s.first_die(&a, w, 1, 32) == 1);
+  CHECK(first_die(s, &a, w, 1) == 1);
   hold(c, one(1, 28), 1.0);
-  CHECK(s.first_die(&a, w, 2, 32) == 2);
+  CHECK(first_die(s, &a, w, 2) == 2);
   int v[8] = {4, 4, 4, 4, 4, 4, 4, 4}, x[8] = {5, 5, 5, 5, 5, 5, 5, 5};
-  CHECK(s.first_die(&a, v, 8, 32) == 0 && s.first_die(&a, x, 8, 32) == -1);
+  CHECK(first_die(s, &a, v, 8) == 0 && first_die(s, &a, x, 8) == -1);
   return 0;
 }
 """
