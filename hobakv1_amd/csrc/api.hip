@@ -178,7 +178,6 @@ struct ClaimGuard {
     if (!ctx->claim.live && ctx->claim.groups.empty()) return;
     std::lock_guard<std::mutex> lock(share_of(ctx->device).mu);
     ctx->claim.live = false;
-    if (!ctx->claim.groups.empty()) ctx->claim.groups_s = now_seconds();
     ctx->claim.groups.clear();
     ctx->claim.passed = 0;
   }

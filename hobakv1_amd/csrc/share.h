@@ -34,7 +34,7 @@ struct Claim {
   bool live = false;         // its launches are queued or running
   std::vector<void*> groups; // the events behind its groups of the two-kernel form in this tick ...
   size_t passed = 0;         // ... of which this many are known to have run
-  double groups_s = -1e9;    // when it last had any
+  double groups_s = -1e9;    // when another's launch last found any
   std::atomic<int> calls{0}; // calls in progress that only launch short kernels (forces, stiffness)
   double calls_s = -1e9;     // when a launch that filled the device last found any
 };
@@ -97,11 +97,15 @@ struct Share {
     }
     return any;
   }
-  // Whether another context queues groups, or did lately.
-  bool groups_lately(const Claim* mine, double now_s) const {
-    for (const Claim* c : claims)
-      if (c != mine && (!c->groups.empty() || now_s - c->groups_s < kShareLatelyS)) return true;
-    return false;
+  // Whether another context has groups queued, or had when a launch lately looked.
+  bool groups_lately(const Claim* mine, double now_s) {
+    bool any = false;
+    for (Claim* c : claims) {
+      if (c == mine) continue;
+      if (!c->groups.empty()) c->groups_s = now_s;
+      any |= now_s - c->groups_s < kShareLatelyS;
+    }
+    return any;
   }
   // The die on which to put the first of `n` instances that take wgs[i] compute units of successive dies: where
   // the fullest die is emptiest; -1 if they fit on none.

@@ -60,8 +60,10 @@ int main() {
   b.groups.push_back(&event);
   CHECK(s.groups_lately(&a, 20.0) && !s.groups_lately(&b, 20.0));
   b.groups.clear();
-  b.groups_s = 20.0;
   CHECK(s.groups_lately(&a, 20.01) && !s.groups_lately(&a, 21.0));
+  b.groups.push_back(&event);  // (groups that came and went between launches: contexts used in turn)
+  b.groups.clear();
+  CHECK(!s.groups_lately(&a, 21.0));
   // the emptiest dies
   hold(b, one(0, 28), 1.0);
   CHECK(first_die(s, &a, w, 1) == 1);
