@@ -605,10 +605,11 @@ __device__ __forceinline__ void resident_solve(const HOBAK_GLOBAL InstDev* __res
       int tid_ = tid;
       T* const zown = (T*)(lds + ZS * own0);
       int it = 0;
-      // where the loop's instructions lie against 32 bytes changes its time by 1% to 3% (the same for all code before
-      // it, which otherwise shifts it with every change): on one die, 24 bytes past was the best of the eight (10^3 FP32 709
-      // us, 707 to 728; 17x9x23 FP64 1.983 ms, 1.99 to 2.01)
-      if constexpr (ONE) asm volatile(".p2align 8\n .rept 6\n s_nop 0\n .endr");
+      // Where the loop's instructions lie against 32 bytes changes its time by 1% to 3%, and without this line every
+      // change to the code before it moves them.  The best of the eight places, on one die: 24 bytes past a boundary (10^3
+      // FP32 709 us, of 707 to 728; 17x9x23 FP64 1.983 ms, of 1.98 to 2.01); over the device: 4 in FP64 and 28 in
+      // FP32 (40^3 step 4.83 ms, of 4.83 to 4.96, and 3.42, of 3.42 to 3.48).
+      asm volatile(".p2align 8\n .rept %0\n s_nop 0\n .endr" ::"n"(ONE ? 6 : kF32 ? 7 : 1));
       for (; it < iters; it++) {
         const unsigned tag = epoch + 1u + (unsigned)it;  // this iteration's words
         const unsigned wprev = wup + ((tag - 1u) & 1u) * wstride;
