@@ -69,9 +69,9 @@
 // time (another program holds the compute units) or one of them cannot hold its columns, the
 // instance is left untouched and counted in Ctl::res_abort, and in Ctl::res_late where only time ran out: the
 // host then takes another form for good, or for a while.  Workgroups that have met run until the launch ends, so the
-// waits of its iterations are short; but where several processes share the device, it takes queues off its compute
-// units and puts them back, and two launches that each got only part of theirs back wait in vain (four
-// processes on one device: once in some 10,000 launches).  A workgroup that waits too long marks the instance
+// waits of its iterations are short; but where several processes share the device, their queues take turns, and two
+// launches that each got only part of their compute units back wait in vain (the likely cause; with four processes
+// waits were in vain once in some 10,000 launches).  A workgroup that waits too long marks the instance
 // (Ctl::res_lost) and leaves, as all others then do; the host starts that solve again from its right-hand side.
 #include "kernels.h"
 #include "pcg_device.h"
